@@ -48,30 +48,55 @@ KERNEL_SAMPLE = 8
 #   backward:   z r/w, invdiag, 3 upper factor entries, and
 #               r for the fused z.r                         -> 7 x 8
 #   update_s:   z, s r/w                                    -> 3 x 8
-# Mixed path: FP32 vectors and factor, FP64 x and matrix entries:
+# A MIC(0) iteration with FP32 vectors and factor, FP64 x and matrix entries,
+# is the yardstick of the mixed path (its kernels are those of KERNEL_BYTES):
 #   spmv_dot:   z, old s, matrix, new s, q (= A s)          -> 4 + 4 + 20 + 4 + 4
 #   forward with the axpy folded in: r r/w, q, invdiag, 3 lower factor
 #               entries, z, and x r/w (FP64), s             -> 8 + 4 + 4 + 12 + 4 + 16 + 4
 #   backward:   7 x 4
 #   the direction update is folded into spmv_dot.
-# A true residual (mixed path only) reads x and b (FP64) and the matrix and
+# A true residual in that iteration reads x and b (FP64) and the matrix and
 # writes r (FP32): 8 + 8 + 20 + 4 = 40 bytes; the forward sweep over it
-# (the same launch) adds r, invdiag, 3 lower factor entries, z: 6 x 4.
+# adds r, invdiag, 3 lower factor entries, z: 6 x 4.
 PCG_BYTES = {
     "fp64": {"k_spmv_dot": 36, "k_axpy_norm": 48, "k_forward": 48, "k_backward": 56, "k_update_s": 24},
     "mixed": {"k_spmv_dot": 36, "k_axpy_norm": 0, "k_forward": 52, "k_backward": 28, "k_update_s": 0},
 }
 TRUE_RESIDUAL_BYTES = 40 + 24
 
+# What the measured path's kernels move at least, per row.  The mixed path is
+# conjugate gradients with a multigrid V-cycle; FP64 x, r, q and diagonal,
+# FP32 couplings (12), inverse diagonal and cycle vectors:
+#   spmv_dot:   z, old s, matrix, new s, q                   -> 4 + 4 + 20 + 4 + 8
+#   axpy_norm:  r, q, x r/w, s, r', inverse diagonal,
+#               couplings, FP32 r, z (first smoothing)       -> 8 + 8 + 16 + 4 + 8 + 4 + 12 + 4 + 4
+#   forward:    restriction: r, z, inverse diagonal,
+#               couplings, an eighth of a coarse r           -> 4 + 4 + 4 + 12 + 0.5
+#   update_s:   correction: r, z, coarse z, inverse
+#               diagonal, couplings, y                       -> 4 + 4 + 0.5 + 4 + 12 + 4
+#   backward:   last smoothing: r, y, inverse diagonal,
+#               couplings, z, FP64 r for z.r                 -> 4 + 4 + 4 + 12 + 4 + 8
+# The coarser levels repeat restriction, correction and the smoothings (24
+# before, 28 after) on an eighth of the rows each time.  The true residual
+# reads x, b and the matrix and writes r: 8 + 8 + 20 + 8.
+KERNEL_BYTES = {
+    "fp64": PCG_BYTES["fp64"],
+    "mixed": {"k_spmv_dot": 40, "k_axpy_norm": 68, "k_forward": 24.5, "k_backward": 36, "k_update_s": 28.5},
+}
+COARSE_LEVEL_BYTES = {"fp64": 0.0, "mixed": (24 + 24.5 + 28.5 + 28) / 7}
+MIXED_TRUE_RESIDUAL_BYTES = 44
+KERNEL_NAMES = {
+    "fp64": {"k_forward": "k_sweep<forward>", "k_backward": "k_sweep<backward>"},
+    "mixed": {"k_spmv_dot": "k_mg_spmv", "k_axpy_norm": "k_mg_axpy_smooth", "k_forward": "k_mg_restrict",
+              "k_update_s": "k_mg_correct", "k_backward": "k_mg_smooth_up"},
+}
+
 # HBM bytes moved per launch, measured with rocprofv3 FETCH_SIZE and WRITE_SIZE
 # passes scaled by a plain 256 MiB copy (x2.0 and x1.0), on the default
 # workload; the commands and counter readings are in
 # profiles/traffic_pcg_kernels_double_dam_256x128x128_mixed.md.  Keyed by
 # (precision, grid); other workloads report null.
-MEASURED_TRAFFIC = {
-    ("mixed", (256, 128, 128)): {"k_backward": 59.63e6, "k_forward": 99.55e6, "k_spmv_dot": 69.48e6,
-                                 "k_true_residual": 116.03e6},
-}
+MEASURED_TRAFFIC = {}
 
 def parse_args(argv=None):
     p = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
@@ -232,7 +257,7 @@ def run_gpu(fa, scene, args, precision, steps, warmup, profiling):
         # dominant one, on every KERNEL_SAMPLE-th iteration (each timed launch
         # costs an event pair, which delays the launches around it).
         wt = sim.stage_times()
-        kern = max(PCG_BYTES[precision], key=lambda k: wt[k][0])
+        kern = max(KERNEL_BYTES[precision], key=lambda k: wt[k][0])
         sim.set_kernel_timing([kern], every=KERNEL_SAMPLE)
     sim.stage_times(reset=True)
 
@@ -259,11 +284,12 @@ def run_gpu(fa, scene, args, precision, steps, warmup, profiling):
     times = sim.stage_times()
     sim.close()
 
-    per_row = PCG_BYTES[precision]
+    per_row = KERNEL_BYTES[precision]
     rows_per_launch = rows_iters / max(iters, 1)
-    # PCG bandwidth: algorithmic bytes of every iteration (PCG_BYTES per
-    # row) plus those of each true residual, over the PCG stage time.
-    pcg_bytes = rows_iters * sum(per_row.values()) + refinements * rows_per_launch * TRUE_RESIDUAL_BYTES
+    # PCG bandwidth: algorithmic bytes of every iteration plus those of each
+    # true residual, over the PCG stage time.
+    pcg_bytes = (rows_iters * (sum(per_row.values()) + COARSE_LEVEL_BYTES[precision])
+                 + refinements * rows_per_launch * MIXED_TRUE_RESIDUAL_BYTES)
     pcg_ms = times["pcg"][0]
     roof = {"kernel": None, "bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": None, "traffic": None}
@@ -278,8 +304,7 @@ def run_gpu(fa, scene, args, precision, steps, warmup, profiling):
         achieved = bytes_per_launch / launch_s / 1e9 if launch_s > 0 else 0.0
         traffic = MEASURED_TRAFFIC.get((precision, tuple(args.size)), {}).get(kern)
         roof.update({
-            "kernel": f"k_sweep<{'forward' if kern == 'k_forward' else 'backward'}>"
-            if kern in ("k_forward", "k_backward") else kern,
+            "kernel": KERNEL_NAMES[precision].get(kern, kern),
             "achieved": achieved,
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": traffic,
@@ -405,7 +430,7 @@ def run_workload(args):
         "p50_ms": lat[len(lat) // 2],
         "p99_ms": lat[min(len(lat) - 1, int(round(0.99 * (len(lat) - 1))))],
         "dtype": "f32 particles/grids, f64 PCG" if precision == "fp64" else
-                 "f32 particles/grids and PCG, f64 dots/x/true residual",
+                 "f32 particles/grids and preconditioner, f64 dots/x/residuals",
         "data": "synthetic",
         "config": {"workload": args.workload, "grid": [I, J, K], "dx": dx, "particles": scene.num_particles,
                    "precision": precision, "tolerance": tol, "updates": updates, "substeps": nsub, "dt": dt,
@@ -546,7 +571,7 @@ def run_serving(args):
         "higher_is_better": True,
         "p50_ms": st["step_ms_p50"],
         "p99_ms": st["step_ms_p99"],
-        "dtype": "f32 particles/grids and PCG, f64 dots/x/true residual",
+        "dtype": "f32 particles/grids and preconditioner, f64 dots/x/residuals",
         "data": "synthetic",
         "config": {
             "workload": (f"{len(reqs)} dam-break requests, grids {SERVING_GRIDS}, fill U(0.2,0.6) in x and height, "
@@ -618,7 +643,7 @@ def main(argv=None):
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32 particles/grids, f64 PCG" if args.precision == "fp64" else
-                 "f32 particles/grids and PCG, f64 dots/x/true residual",
+                 "f32 particles/grids and preconditioner, f64 dots/x/residuals",
         "data": "synthetic",
         "config": {
             "workload": f"double dam break {I}x{J}x{K}, dx=1/{round(1 / dx)}, seed {args.seed}, "

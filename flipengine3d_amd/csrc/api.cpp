@@ -99,8 +99,9 @@ int flipmi_ctx_create(int device, flipmi_ctx **out) {
         delete c;
         return FLIPMI_ERR_HIP;
     }
-    // Device address of this device's flipmi_extrapolate_noalloc scratch.
-    if (noalloc_scratch_init(device) != hipSuccess) {
+    // Device address of this device's flipmi_extrapolate_noalloc scratch, and
+    // the multigrid kernel's LDS.
+    if (noalloc_scratch_init(device) != hipSuccess || mg_allow_lds(device) != hipSuccess) {
         (void)hipStreamDestroy(c->c.stream);
         delete c;
         return FLIPMI_ERR_HIP;
@@ -706,30 +707,40 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
         // _conditionSolidVelocityField (pressuresolver.cpp:124-268) precedes the
         // assembly; with all solid velocities zero it changes nothing.
         const bool solid_given = a->solid_u || a->solid_v || a->solid_w;
-        if (solid_given) {
-            DBuf<int> parent;
+        if (a->precision != FLIPMI_PCG_FP64 && a->precision != FLIPMI_PCG_MIXED)
+            throw StatusError{FLIPMI_ERR_INVALID_ARG, "unknown pcg precision"};
+        bool mixed = a->precision == FLIPMI_PCG_MIXED;
+        if (solid_given || mixed) {
+            DBuf<int> parent, found;
             DBuf<unsigned> flags;
             alloc_dev(parent, nc);
             alloc_dev(flags, nc);
-            hipck(launch_condition_solid(g, liq.p, wu.p, wv.p, ww.p, su.p, sv.p, sw.p, parent.p, flags.p, s),
-                  "solid velocity conditioning");
+            alloc_dev(found, 1);
+            int pocket = 0;
+            hipck(launch_pocket_regions(g, liq.p, wu.p, wv.p, ww.p, parent.p, flags.p, found.p, s), "fluid regions");
+            if (solid_given)
+                hipck(launch_condition_solid(g, parent.p, flags.p, su.p, sv.p, sw.p, s), "solid velocity conditioning");
+            hipck(hipMemcpyAsync(&pocket, found.p, sizeof(int), hipMemcpyDeviceToHost, s), "pockets");
             hipck(hipStreamSynchronize(s), "sync");
+            // The pressure of a pocket that borders no air is fixed up to a
+            // constant only, which follows from the preconditioner.  Callers
+            // of this entry point see the pressures, so such a system keeps
+            // the reference's (a scene uses their differences alone).
+            if (pocket) mixed = false;
         }
-        if (a->precision != FLIPMI_PCG_FP64 && a->precision != FLIPMI_PCG_MIXED)
-            throw StatusError{FLIPMI_ERR_INVALID_ARG, "unknown pcg precision"};
         PressureStore ps;
-        ps.alloc(g, s, a->precision == FLIPMI_PCG_MIXED);
+        ps.alloc(g, s, mixed);
         PressureWork pw;
         pw.g = g; pw.dt = a->dt; pw.tol = a->tolerance; pw.acceptable = a->acceptable_tolerance;
         pw.maxiter = a->max_iterations; pw.precision = a->precision;
         pw.liquid = liq.p; pw.wU = wu.p; pw.wV = wv.p; pw.wW = ww.p; pw.wC = wc.p;
         pw.sU = su.p; pw.sV = sv.p; pw.sW = sw.p;
         pw.u = u.p; pw.v = v.p; pw.w = w.p; pw.vu = vu.p; pw.vv = vv.p; pw.vw = vw.p;
-        PcgScalars *hs = nullptr;
-        hipck(hipHostMalloc((void **)&hs, sizeof(PcgScalars), hipHostMallocDefault), "pinned");
+        void *hs = nullptr;
+        hipck(hipHostMalloc(&hs, kPressureStaging, hipHostMallocDefault), "pinned");
         PressureOutcome o;
         try {
-            o = run_pressure(pw, ps.pb, hs, s, nullptr);
+            o = run_pressure(pw, ps, hs, s, nullptr);
         } catch (...) {
             (void)hipHostFree(hs);
             throw;
@@ -744,11 +755,9 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
         std::vector<float> hl(nc);
         int rows = 0;
         std::vector<double> x;
-        const SlotMap &sm = ps.pb.sm;
-        if (a->pressure_rows) {
-            x.resize(sm.count());
-            hipck(hipMemcpyAsync(x.data(), ps.pb.x, sm.count() * sizeof(double), hipMemcpyDeviceToHost, s),
-                  "download");
+        if (a->pressure_rows && o.solved) {
+            x.resize(o.index.count);
+            hipck(hipMemcpyAsync(x.data(), o.x, x.size() * sizeof(double), hipMemcpyDeviceToHost, s), "download");
         }
         download(hl.data(), liq, nc, s);
         hipck(hipStreamSynchronize(s), "sync");
@@ -758,7 +767,7 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
                 for (int i = 1; i < I - 1; i++) {
                     size_t c = (size_t)i + (size_t)I * ((size_t)j + (size_t)J * k);
                     if (hl[c] < 0) {
-                        if (a->pressure_rows) a->pressure_rows[rows] = o.solved ? x[sm.slot(i, j, k)] : 0.0;
+                        if (a->pressure_rows) a->pressure_rows[rows] = o.solved ? x[o.index(i, j, k)] : 0.0;
                         rows++;
                     }
                 }
@@ -791,7 +800,7 @@ int flipmi_mic0_apply(flipmi_ctx *ctx, int I, int J, int K, double dx, double dt
         hipck(launch_fill_f32(zero_v.p, nV, 0.0f, s), "fill");
         hipck(launch_fill_f32(zero_w.p, nW, 0.0f, s), "fill");
         PressureStore ps;
-        ps.alloc(g, s, false);
+        ps.alloc_slots(g, s);
         hipck(launch_pressure_reset(ps.pb, s), "reset");
         hipck(launch_pressure_assemble(g, dt, liq.p, wu.p, wv.p, ww.p, wc.p, zero_u.p, zero_v.p, zero_w.p,
                                        zero_u.p, zero_v.p, zero_w.p, ps.pb, s),

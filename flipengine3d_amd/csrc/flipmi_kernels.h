@@ -132,11 +132,6 @@ struct PcgScalars {
     unsigned int rows;                  // rows of the system (fluid interior cells)
     unsigned long long absmax_bits;
     double mf;                          // dt / dx^2 of the assembled system (coupling scale)
-    // mixed precision: true-residual replacement ("reliable update")
-    double rmax;                        // |r| at the last true residual
-    double delta;                       // replace when |r32| < delta * rmax
-    int refresh;                        // a true residual is due
-    int refinements;                    // true residuals computed
     // Epoch of the next sweep launch: read by every workgroup of a sweep,
     // advanced by its last tile, so launches replayed from a captured graph
     // still tag their records afresh.  Starts at 1 (records start at 0).
@@ -197,17 +192,6 @@ struct PressureBuffers {
     double *x, *r, *z, *s;              // PCG vectors (FP64)
     double *invdiag, *Lx, *Ly, *Lz;     // MIC(0) factor: column entries (rows +x/+y/+z)
     double *Lxm, *Lym, *Lzm;            // the same entries read from the row: columns -x/-y/-z
-    // Mixed precision (null unless allocated): FP32 copies of the factor and
-    // the FP32 PCG vectors; x and the matrix stay FP64.
-    float *invdiag32, *Lx32, *Ly32, *Lz32, *Lxm32, *Lym32, *Lzm32;
-    float *r32, *z32, *s32;
-    // Mixed precision: the SpMV forms the new direction s = z + beta s from
-    // the old one, so s lives in two buffers: s32 is read, s32b written, and
-    // the host swaps them after each SpMV launch.  s_plain: the next SpMV
-    // reads s32 as it is (right after initialisation).
-    float *s32b;
-    int s_plain;
-    float *q32;  // mixed precision: q = A s, read by the axpy
     double *partials;                   // per-block partial sums
     int npartials;
     unsigned long long *edge;           // tagged values a tile hands to its j / k neighbours
@@ -233,45 +217,49 @@ hipError_t launch_pressure_assemble(const GridGeom &g, double dt, const float *l
                                     const float *w, const float *sU, const float *sV,
                                     const float *sW, PressureBuffers &pb, hipStream_t s);
 hipError_t launch_pressure_reset(PressureBuffers &pb, hipStream_t s);
-// PressureSolver::_conditionSolidVelocityField: zeroes the solid face
-// velocities (sU, sV, sW, in place) around isolated fluid pockets.  Scratch:
-// parent and flags, one element per cell each.
-hipError_t launch_condition_solid(const GridGeom &g, const float *liquid, const float *wU, const float *wV,
-                                  const float *wW, float *sU, float *sV, float *sW, int *parent,
-                                  unsigned *flags, hipStream_t s);
+// Fluid regions (parent and flags, one element per cell each) and whether any
+// of them is an isolated pocket: *found = 0 / 1.
+hipError_t launch_pocket_regions(const GridGeom &g, const float *liquid, const float *wU, const float *wV,
+                                 const float *wW, int *parent, unsigned *flags, int *found, hipStream_t s);
+// PressureSolver::_conditionSolidVelocityField over those regions: zeroes the
+// solid face velocities (sU, sV, sW, in place) around isolated pockets.
+hipError_t launch_condition_solid(const GridGeom &g, int *parent, const unsigned *flags, float *sU, float *sV,
+                                  float *sW, hipStream_t s);
 // Marks the slot groups that hold a row (after assembly).
 hipError_t launch_group_mask(PressureBuffers &pb, hipStream_t s);
 // Zeroes the factor, finds each column tile's row extent and factorises.
 hipError_t launch_mic0_factor(const GridGeom &g, const float *liquid, PressureBuffers &pb,
                               hipStream_t s);
-// mixed: FP32 inner iteration with FP64 dots, FP64 x and true-residual
-// replacement (requires the FP32 arrays of pb).
-hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, bool mixed,
-                           PressureBuffers &pb, hipStream_t s);
-hipError_t launch_pcg_iteration(const GridGeom &g, bool mixed, PressureBuffers &pb, hipStream_t s);
-// The kernels of one PCG iteration.  The FP64 path runs spmv, axpy,
-// forward, backward, update.  The mixed path folds the axpy into the forward
-// sweep and the direction update into the SpMV, and runs kPcgResidual (a
-// true residual and a forward sweep over it) between the forward and the
-// backward sweep; it exits at once unless the forward sweep's residual norm
-// called for a true residual.
+hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, PressureBuffers &pb, hipStream_t s);
+// The timed kernels of one PCG iteration.  FP64 path: SpMV, axpy, forward and
+// backward sweep, direction update.  Mixed precision (k_multigrid.hip): SpMV
+// with the direction update, axpy with the first smoothing, and of the
+// V-cycle on the finest level the restriction (kPcgForward), the coarse
+// correction (kPcgUpdate) and the last smoothing (kPcgBackward).
 enum {
     kPcgSpmv = 0, kPcgAxpy = 1, kPcgForward = 2, kPcgBackward = 3, kPcgUpdate = 4,
     kPcgResidual = 5, kPcgPieces = 6
 };
-bool pcg_piece_used(int piece, bool mixed);
-// Sweep launches per iteration (each takes a record epoch).
-inline unsigned pcg_sweeps_per_iteration(bool mixed) { return mixed ? 3u : 2u; }
-int pcg_piece_at(int q);  // piece executed q-th within an iteration
+constexpr unsigned kPcgSweeps = 2;  // sweep launches per iteration (each takes a record epoch)
 // With kt.start set, the kernel's dispatch records its start and end in the
 // two events.
 struct KernelTiming {
     hipEvent_t start = nullptr, stop = nullptr;
 };
-hipError_t launch_pcg_piece(int piece, const GridGeom &g, bool mixed, PressureBuffers &pb,
-                            hipStream_t s, const KernelTiming &kt);
-// p is in slot order (pb.sm).
-hipError_t launch_pressure_apply(const GridGeom &g, const SlotMap &sm, double dt, const float *liquid,
+hipError_t launch_pcg_iteration(const GridGeom &g, PressureBuffers &pb, hipStream_t s,
+                                const KernelTiming (&kt)[kPcgPieces]);
+// Where a solver keeps the pressure of interior cell (i, j, k): in slot order
+// or, dense, in the rows of the interior cells.
+struct PressureIndex {
+    SlotMap sm;
+    unsigned px = 0, pxy = 0;  // pitches of the dense layout; 0: slots
+    size_t count = 0;          // elements from the first cell to the last
+    __host__ __device__ unsigned operator()(int i, int j, int k) const {
+        if (px == 0) return sm.slot32(i, j, k);
+        return (unsigned)(i - 1) + px * (unsigned)(j - 1) + pxy * (unsigned)(k - 1);
+    }
+};
+hipError_t launch_pressure_apply(const GridGeom &g, const PressureIndex &at, double dt, const float *liquid,
                                  const float *wU, const float *wV, const float *wW,
                                  const double *p, float *u, float *v, float *w, uint8_t *vu,
                                  uint8_t *vv, uint8_t *vw, hipStream_t s);

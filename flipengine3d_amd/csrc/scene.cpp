@@ -114,11 +114,58 @@ size_t PressureStore::device_bytes() const {
                alist.bytes();
     for (int q = 0; q <= kSlotArrays; q++) b += arr[q].bytes();
     for (int q = 0; q < kWeightArrays; q++) b += wgt[q].bytes();
-    for (int q = 0; q < kSlotArrays32; q++) b += arr32[q].bytes();
+    for (int q = 0; q < 6; q++) b += mg_f64[q].bytes();
+    b += mg_part.bytes() + mg_f32.bytes() + mg_ints.bytes() + mg_bricks.bytes() + mg_scal.bytes() +
+         mg_coarse.bytes();
     return b;
 }
 
 void PressureStore::alloc(const GridGeom &g, hipStream_t s, bool mixed) {
+    const MgPlan plan = mixed ? make_mg_plan(g.I, g.J, g.K) : MgPlan{};
+    // Grids without interior cells (no rows) and past 32-bit indices have no
+    // levels; the FP64 path takes them, or refuses them, by itself.
+    if (!plan.usable()) {
+        alloc_slots(g, s);
+        return;
+    }
+    graphs.clear();
+    auto need = [&](hipError_t e) {
+        if (e != hipSuccess) throw StatusError{FLIPMI_ERR_OOM, "mixed-precision arrays: out of device memory"};
+    };
+    size_t nf = 2 * plan.cells[0], nb = 0;
+    for (int l = 0; l < plan.nlevels; l++) nf += 8 * plan.cells[l];
+    for (int l = 0; l < plan.nglobal; l++) nb += plan.bricks[l];
+    double *d[6];
+    for (int q = 0; q < 6; q++) {
+        need(mg_f64[q].alloc(plan.cells[0]));
+        d[q] = mg_f64[q].p;
+    }
+    need(mg_f32.alloc(nf));
+    need(mg_part.alloc(kMgPartials));
+    need(mg_ints.alloc(2 * nb + 2 * kMgMaxLevels + scan_scratch_elems((int)nb)));
+    need(mg_bricks.alloc(nb));
+    need(mg_scal.alloc(1));
+    need(mg_coarse.alloc(1));
+    mg.bind(plan, d, mg_f32.p, nf, mg_part.p, mg_ints.p, mg_bricks.p, mg_scal.p, mg_coarse.p);
+    if (hipMemcpyAsync(mg_coarse.p, &mg.coarse_host, sizeof(MgCoarse), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        throw StatusError{FLIPMI_ERR_HIP, "pressure arrays: upload failed"};
+    // Padding and guards are read and never written: they stay zero.
+    if (mg.clear(s) != hipSuccess)
+        throw StatusError{FLIPMI_ERR_HIP, "pressure arrays: clearing failed"};
+    mg_on = true;
+    mg_dirty = false;
+}
+
+void PressureStore::release_multigrid() {
+    graphs.clear();
+    for (int q = 0; q < 6; q++) mg_f64[q].release();
+    mg_part.release(); mg_f32.release(); mg_ints.release(); mg_bricks.release(); mg_scal.release();
+    mg_coarse.release();
+    mg_on = false;
+}
+
+void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s) {
     graphs.clear();  // captured launches point into the buffers replaced here
     SlotMap sm = make_slot_map(g.I, g.J, g.K);
     // Slot arrays carry the zero and sink groups after the last tile.
@@ -155,16 +202,6 @@ void PressureStore::alloc(const GridGeom &g, hipStream_t s, bool mixed) {
     pb.Lxm = arr[10].p; pb.Lym = arr[11].p; pb.Lzm = arr[12].p;
     pb.wx = wgt[0].p; pb.wy = wgt[1].p; pb.wz = wgt[2].p;
     pb.partials = arr[kSlotArrays].p;
-    if (mixed) {
-        for (int q = 0; q < kSlotArrays32; q++) {
-            if (arr32[q].alloc(ns) != hipSuccess)
-                throw StatusError{FLIPMI_ERR_OOM, "mixed-precision arrays: out of device memory"};
-            (void)launch_fill_f32(arr32[q].p, ns, 0.0f, s);
-        }
-        float **dst[kSlotArrays32] = {&pb.invdiag32, &pb.Lx32, &pb.Ly32, &pb.Lz32, &pb.Lxm32, &pb.Lym32,
-                                      &pb.Lzm32, &pb.r32, &pb.z32, &pb.s32, &pb.s32b, &pb.q32};
-        for (int q = 0; q < kSlotArrays32; q++) *dst[q] = arr32[q].p;
-    }
     pb.npartials = npart;
     pb.edge = edge.p;
     const int groups_per_tile = sm.S / 4;
@@ -194,20 +231,20 @@ static void hip_check(hipError_t e, const char *what) {
         throw StatusError{FLIPMI_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e)};
 }
 
-// One batch of PCG iterations as a graph: captured the first time this
-// (batch size, starting s buffer) occurs, replayed afterwards.  The kernels
-// read their scalars (alpha, beta, the sweep epoch, done) from device memory,
-// so a replay computes exactly what launching the kernels would; only the
-// host's bookkeeping of the launches (the s buffer swap of each SpMV, the
-// count of sweep launches) is advanced by hand on a replay.
-static void launch_pcg_batch_graph(PcgGraphs &G, const GridGeom &g, bool mixed, PressureBuffers &pb, int batch,
-                                   hipStream_t s) {
-    const auto key = std::make_pair(batch, (const void *)pb.s32);
+// One batch of PCG iterations as a graph: captured the first time this batch
+// size occurs with the iteration's swapped buffers in this state, replayed
+// afterwards.  The kernels read their scalars (alpha, beta, the sweep epoch,
+// done) from device memory, so a replay computes exactly what launching the
+// kernels would; only the host's bookkeeping of the launches is advanced by
+// hand on a replay (replayed).
+template <class Launch, class Replayed>
+static void launch_pcg_batch_graph(PcgGraphs &G, int batch, int state, hipStream_t s, Launch &&launch,
+                                   Replayed &&replayed) {
+    const auto key = std::make_pair(batch, state);
     auto it = G.exec.find(key);
     if (it == G.exec.end()) {
         hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "pcg graph capture");
-        hipError_t le = hipSuccess;
-        for (int q = 0; q < batch && le == hipSuccess; q++) le = launch_pcg_iteration(g, mixed, pb, s);
+        hipError_t le = launch();
         hipGraph_t graph = nullptr;
         hipError_t ce = hipStreamEndCapture(s, &graph);
         hip_check(le, "pcg iteration (capture)");
@@ -218,15 +255,141 @@ static void launch_pcg_batch_graph(PcgGraphs &G, const GridGeom &g, bool mixed, 
         hip_check(ie, "pcg graph instantiate");
         it = G.exec.emplace(key, exec).first;
     } else {
-        if (mixed && (batch & 1)) std::swap(pb.s32, pb.s32b);
-        pb.epoch += pcg_sweeps_per_iteration(mixed) * (unsigned)batch;
+        replayed();
     }
     hip_check(hipGraphLaunch(it->second, s), "pcg graph launch");
 }
 
-PressureOutcome run_pressure(const PressureWork &w, PressureBuffers &pb, PcgScalars *hs,
-                             hipStream_t s, Scene *prof) {
+// Iterations the observed convergence rate still needs from residual `now` to
+// `target`, or -1 when it gives none.
+static int iterations_needed(double before, double now, int iterations, double target) {
+    if (iterations <= 0 || !(now > 0) || !(now < before) || !(target > 0)) return -1;
+    const double rate = std::log(now / before) / iterations;  // < 0
+    const double need = std::log(target / now) / rate;
+    return need > 0 && need < 1e6 ? (int)std::ceil(need) : -1;
+}
+
+// Pressure events of an iteration at profiling level 2.
+static bool take_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces]) {
+    if (!prof || prof->profiling < 2 || prof->kernel_mask == 0 ||
+        prof->pcg_iteration_count++ % prof->kernel_every != 0)
+        return false;
+    for (int piece = 0; piece < kPcgPieces; piece++) {
+        if (piece == kPcgResidual || !((prof->kernel_mask >> piece) & 1u)) continue;
+        kt[piece].start = prof->take_event();
+        kt[piece].stop = prof->take_event();
+    }
+    return true;
+}
+static void book_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces]) {
+    for (int piece = 0; piece < kPcgPieces; piece++)
+        if (kt[piece].start) prof->add_timed(FLIPMI_STAGE_K_SPMV + piece, kt[piece].start, kt[piece].stop);
+}
+
+static void apply_pressure(const PressureWork &w, PressureOutcome &out, hipStream_t s, Scene *prof) {
+    hipEvent_t ev = nullptr;
+    if (prof) prof->begin_stage(FLIPMI_STAGE_APPLY, &ev);
+    hip_check(launch_pressure_apply(w.g, out.index, w.dt, w.liquid, w.wU, w.wV, w.wW, out.x, w.u, w.v, w.w, w.vu,
+                                    w.vv, w.vw, s),
+              "pressure apply");
+    if (prof) prof->end_stage(FLIPMI_STAGE_APPLY, ev);
+    out.solved = true;
+}
+
+// The mixed-precision solve.  Returns false when it has not converged: the
+// caller then solves the system on the FP64 path (nothing has been applied).
+constexpr int kMgMaxIterations = 200;  // over ten times what it takes
+static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *hs, hipStream_t s, Scene *prof,
+                          PressureOutcome &out) {
+    MgSolver &mg = ps.mg;
+    hipEvent_t ev = nullptr;
+    // Values that are not finite would survive in cells that are no rows now
+    // and may be rows later.
+    if (ps.mg_dirty) hip_check(mg.clear(s), "multigrid clear");
+    ps.mg_dirty = true;
+    if (prof) prof->begin_stage(FLIPMI_STAGE_ASSEMBLE, &ev);
+    const PressureFields fields{w.liquid, w.wU, w.wV, w.wW, w.wC, w.u, w.v, w.w, w.sU, w.sV, w.sW};
+    hip_check(mg.setup(w.g, w.dt, fields, w.tol, std::min(w.maxiter, kMgMaxIterations), s), "pressure assemble");
+    if (prof) prof->end_stage(FLIPMI_STAGE_ASSEMBLE, ev);
+    if (prof) prof->begin_stage(FLIPMI_STAGE_PCG, &ev);
+    hip_check(mg.start(false, s), "pcg start");
+    // Iterations are enqueued in batches between host checks of the device
+    // scalars; kernels past convergence return at once.  The count hardly
+    // depends on the system (13 to 16 for 1e-9, 8 to 10 for 1e-6), so the
+    // first batch stops short of that and the rate gives the rest.
+    int batch = 8, launched = 0, prev_iters = 0;
+    double prev_resid = 0.0;
+    for (;;) {
+        const bool use_graph = w.graphs && !(prof && prof->profiling >= 2);
+        const int state = mg.turn + 2 * (mg.first ? 1 : 0);
+        auto all = [&]() -> hipError_t {
+            hipError_t e = hipSuccess;
+            for (int q = 0; q < batch && e == hipSuccess; q++) {
+                KernelTiming kt[kPcgPieces];
+                const bool timed = take_kernel_timings(prof, kt);
+                e = mg.iterate(s, timed ? kt : nullptr);
+                if (timed) book_kernel_timings(prof, kt);
+            }
+            return e == hipSuccess ? mg.verify(s) : e;
+        };
+        if (use_graph) {
+            launch_pcg_batch_graph(*w.graphs, batch, state, s, all, [&] {
+                mg.turn ^= batch & 1;
+                mg.first = false;
+            });
+        } else {
+            hip_check(all(), "pcg iteration");
+        }
+        launched += batch;
+        hip_check(hipMemcpyAsync(hs, mg.sc, sizeof(MgScalars), hipMemcpyDeviceToHost, s), "scalars");
+        hip_check(hipStreamSynchronize(s), "pcg sync");
+        if (hs->done) break;
+        if (launched > 2 * kMgMaxIterations) break;
+        if (hs->restart) hip_check(mg.start(true, s), "pcg restart");
+        const int need = iterations_needed(prev_resid > 0 ? prev_resid : hs->bnorm, hs->resid,
+                                           hs->iters - prev_iters, hs->tol);
+        prev_iters = hs->iters;
+        prev_resid = hs->resid;
+        batch = std::max(1, std::min(need > 0 ? need : 8, 16));
+    }
+    if (prof) prof->end_stage(FLIPMI_STAGE_PCG, ev);
+    out.rows = hs->rows;
+    if (hs->bnorm < w.tol) {
+        // Early exit of PressureSolver::solve when max|rhs| < tolerance
+        // (pressuresolver.cpp:52-62): nothing is solved or applied.
+        ps.mg_dirty = false;
+        out.iterations = 0;
+        out.residual = 0.0;
+        out.success = true;
+        return true;
+    }
+    if (prof) prof->stage_calls[FLIPMI_STAGE_PCG_ITERS] += hs->iters;
+    if (!hs->converged) return false;
+    ps.mg_dirty = false;
+    out.iterations = hs->iters;
+    out.residual = hs->resid;
+    out.refinements = hs->refinements;
+    out.success = true;
+    out.x = mg.fine.x;
+    out.index.px = mg.lv[0].px;
+    out.index.pxy = mg.lv[0].pxy;
+    out.index.count = (size_t)mg.lv[0].pxy * mg.lv[0].nz;
+    apply_pressure(w, out, s, prof);
+    return true;
+}
+
+PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *host_sc, hipStream_t s, Scene *prof) {
     PressureOutcome out;
+    if (ps.mg_on) {
+        if (run_multigrid(w, ps, static_cast<MgScalars *>(host_sc), s, prof, out)) return out;
+        // Not positive definite, not finite, or capped: the reference's
+        // solver decides, here and for the rest of this store's life.
+        hip_check(hipStreamSynchronize(s), "pcg sync");
+        ps.release_multigrid();
+        ps.alloc_slots(w.g, s);
+    }
+    PressureBuffers &pb = ps.pb;
+    PcgScalars *hs = static_cast<PcgScalars *>(host_sc);
     hipEvent_t ev = nullptr;
     if (prof) prof->begin_stage(FLIPMI_STAGE_ASSEMBLE, &ev);
     hip_check(launch_pressure_reset(pb, s), "pressure reset");
@@ -248,11 +411,9 @@ PressureOutcome run_pressure(const PressureWork &w, PressureBuffers &pb, PcgScal
         return out;
     }
     if (prof) prof->begin_stage(FLIPMI_STAGE_MIC0, &ev);
-    const bool mixed = w.precision == FLIPMI_PCG_MIXED;
-    if (mixed && !pb.r32) throw StatusError{FLIPMI_ERR_INVALID_ARG, "mixed precision arrays not allocated"};
     hip_check(launch_group_mask(pb, s), "group mask");
     hip_check(launch_mic0_factor(w.g, w.liquid, pb, s), "mic0 factor");
-    hip_check(launch_pcg_init(w.g, w.tol, w.maxiter, mixed, pb, s), "pcg init");
+    hip_check(launch_pcg_init(w.g, w.tol, w.maxiter, pb, s), "pcg init");
     if (prof) prof->end_stage(FLIPMI_STAGE_MIC0, ev);
     if (prof) prof->begin_stage(FLIPMI_STAGE_PCG, &ev);
     // Iterations are enqueued in batches between host checks of the device
@@ -265,37 +426,25 @@ PressureOutcome run_pressure(const PressureWork &w, PressureBuffers &pb, PcgScal
     double prev_resid = bnorm;
     const double target = w.tol * bnorm;
     for (;;) {
-        // A batch runs from a captured graph once the first SpMV (which reads
-        // s as initialised) is behind, unless kernels are being timed or the
-        // sweep tag is near its wrap-around (which clears the records).
-        const bool use_graph = w.graphs && pb.s_plain == 0 && !(prof && prof->profiling >= 2) &&
-                               pb.epoch + pcg_sweeps_per_iteration(mixed) * (unsigned)batch + 8u < 0xfffffff0u;
-        for (int q = 0; q < batch; q++) {
-            const bool timed = prof && prof->profiling >= 2 && prof->kernel_mask != 0 &&
-                               prof->pcg_iteration_count++ % prof->kernel_every == 0;
-            if (timed) {
-                // Time the selected kernels of the iteration on the launch stream.
-                for (int q = 0; q < kPcgPieces; q++) {
-                    int piece = pcg_piece_at(q);
-                    if (!pcg_piece_used(piece, mixed)) continue;
-                    int stage = piece == kPcgResidual ? FLIPMI_STAGE_K_RESIDUAL : FLIPMI_STAGE_K_SPMV + piece;
-                    KernelTiming kt;
-                    if ((prof->kernel_mask >> piece) & 1u) {
-                        kt.start = prof->take_event();
-                        kt.stop = prof->take_event();
-                    }
-                    hip_check(launch_pcg_piece(piece, w.g, mixed, pb, s, kt), "pcg kernel");
-                    if (kt.start) prof->add_timed(stage, kt.start, kt.stop);
-                }
-            } else if (use_graph) {
-                // (Never at profiling level 2: there every iteration runs on
-                // its own, timed or not.)
-                launch_pcg_batch_graph(*w.graphs, w.g, mixed, pb, batch, s);
-                break;  // the graph holds the whole batch
-            } else {
-                hip_check(launch_pcg_iteration(w.g, mixed, pb, s), "pcg iteration");
+        // A batch runs from a captured graph unless kernels are being timed
+        // or the sweep tag is near its wrap-around (which clears the records).
+        const bool use_graph = w.graphs && !(prof && prof->profiling >= 2) &&
+                               pb.epoch + kPcgSweeps * (unsigned)batch + 8u < 0xfffffff0u;
+        auto all = [&]() -> hipError_t {
+            hipError_t e = hipSuccess;
+            for (int q = 0; q < batch && e == hipSuccess; q++) {
+                KernelTiming kt[kPcgPieces];
+                const bool timed = take_kernel_timings(prof, kt);
+                e = launch_pcg_iteration(w.g, pb, s, kt);
+                if (timed) book_kernel_timings(prof, kt);
             }
-        }
+            return e;
+        };
+        if (use_graph)
+            launch_pcg_batch_graph(*w.graphs, batch, 0, s, all,
+                                   [&] { pb.epoch += kPcgSweeps * (unsigned)batch; });
+        else
+            hip_check(all(), "pcg iteration");
         launched += batch;
         hip_check(hipMemcpyAsync(hs, pb.sc, sizeof(PcgScalars), hipMemcpyDeviceToHost, s), "scalars");
         hip_check(hipStreamSynchronize(s), "pcg sync");
@@ -303,13 +452,8 @@ PressureOutcome run_pressure(const PressureWork &w, PressureBuffers &pb, PcgScal
         if (hs->done) break;
         if (launched > w.maxiter + 16)
             throw StatusError{FLIPMI_ERR_HIP, "pcg did not terminate within its iteration cap"};
-        int next = std::min(batch * 2, 32);
-        const int done_iters = hs->iters - prev_iters;
-        if (done_iters > 0 && hs->resid > 0 && hs->resid < prev_resid && target > 0) {
-            const double rate = std::log(hs->resid / prev_resid) / done_iters;  // < 0
-            const double need = std::log(target / hs->resid) / rate;
-            if (need > 0 && need < 1e6) next = (int)std::ceil(need) + 2;
-        }
+        const int need = iterations_needed(prev_resid, hs->resid, hs->iters - prev_iters, target);
+        const int next = need > 0 ? need + 2 : std::min(batch * 2, 32);
         prev_iters = hs->iters;
         prev_resid = hs->resid;
         batch = std::max(2, std::min(next, 64));
@@ -318,18 +462,13 @@ PressureOutcome run_pressure(const PressureWork &w, PressureBuffers &pb, PcgScal
     if (prof) prof->stage_calls[FLIPMI_STAGE_PCG_ITERS] += hs->iters;
     out.iterations = hs->failed ? 0 : hs->iters;
     out.residual = hs->resid;
-    out.refinements = mixed ? hs->refinements : 0;
     bool converged = hs->converged != 0;
     // PressureSolver::_solveLinearSystem (pressuresolver.cpp:810-840).
     out.success = converged || (!hs->failed && out.iterations == w.maxiter && out.residual < w.acceptable);
-    if (out.success) {
-        if (prof) prof->begin_stage(FLIPMI_STAGE_APPLY, &ev);
-        hip_check(launch_pressure_apply(w.g, pb.sm, w.dt, w.liquid, w.wU, w.wV, w.wW, pb.x, w.u, w.v, w.w,
-                                        w.vu, w.vv, w.vw, s),
-                  "pressure apply");
-        if (prof) prof->end_stage(FLIPMI_STAGE_APPLY, ev);
-        out.solved = true;
-    }
+    out.x = pb.x;
+    out.index.sm = pb.sm;
+    out.index.count = pb.sm.count();
+    if (out.success) apply_pressure(w, out, s, prof);
     return out;
 }
 
@@ -442,8 +581,7 @@ void Scene::alloc_all() {
     need(status.alloc(nf));
     press = new PressureStore();
     press->alloc(g, stream, desc.pcg_precision == FLIPMI_PCG_MIXED);
-    static_assert(sizeof(PcgScalars) <= 4096, "the PCG scalars are read back through the staging buffer");
-    check(hipHostMalloc(&host_stage, 4096, hipHostMallocDefault), "pinned staging");
+    check(hipHostMalloc(&host_stage, kPressureStaging, hipHostMallocDefault), "pinned staging");
     // Fresh MeshLevelSet: phi = distance upper bound everywhere
     // (meshlevelset.cpp:35-42, 760-762); zero solid face velocities.
     float upper = (float)((double)((I + 1) + (J + 1) + (K + 1)) * g.dx);
@@ -600,14 +738,17 @@ size_t estimate_scene_bytes(const flipmi_scene_desc &d, int64_t cap) {
     b += sizeof(float) * nc + sizeof(float) * 2 * (nU + nV + nW) + (nU + nV + nW) + nf;
     SlotMap sm = make_slot_map(d.isize, d.jsize, d.ksize);
     const size_t ns = sm.alloc_count(), ntiles = (size_t)sm.ntj * sm.ntk;
-    b += sizeof(double) * (PressureStore::kSlotArrays * ns + 2 * 2048 + ntiles);
-    b += sizeof(float) * PressureStore::kWeightArrays * ns;
-    if (d.pcg_precision == FLIPMI_PCG_MIXED) b += sizeof(float) * PressureStore::kSlotArrays32 * ns;
-    b += sizeof(unsigned long long) * edge_record_count(sm);
-    b += sizeof(unsigned long long) * ntiles * (size_t)((sm.S / 4 + 63) / 64);
-    b += sizeof(unsigned) * (ntiles + 1) + sizeof(int) * 2 * ntiles + sizeof(PcgScalars);
-    b += sizeof(int) * ((sm.count() >> 8) + 1);
-    return b;
+    size_t slots = sizeof(double) * (PressureStore::kSlotArrays * ns + 2 * 2048 + ntiles);
+    slots += sizeof(float) * PressureStore::kWeightArrays * ns;
+    slots += sizeof(unsigned long long) * edge_record_count(sm);
+    slots += sizeof(unsigned long long) * ntiles * (size_t)((sm.S / 4 + 63) / 64);
+    slots += sizeof(unsigned) * (ntiles + 1) + sizeof(int) * 2 * ntiles + sizeof(PcgScalars);
+    slots += sizeof(int) * ((sm.count() >> 8) + 1);
+    // A mixed scene holds the multigrid levels, or the slots of the FP64 path
+    // once a system has gone there.
+    if (d.pcg_precision == FLIPMI_PCG_MIXED)
+        slots = std::max(slots, make_mg_plan(d.isize, d.jsize, d.ksize).device_bytes());
+    return b + slots;
 }
 
 GridGeom make_geom(int I, int J, int K, double dx) {
@@ -706,7 +847,7 @@ void Scene::pressure_solve(double dt) {
     pw.u = u.p; pw.v = v.p; pw.w = w.p; pw.vu = vu.p; pw.vv = vv.p; pw.vw = vw.p;
     pw.graphs = launch_graphs ? &press->graphs : nullptr;
     PressureOutcome o =
-        run_pressure(pw, press->pb, (PcgScalars *)host_stage, stream, profiling ? this : nullptr);
+        run_pressure(pw, *press, host_stage, stream, profiling ? this : nullptr);
     last_iters = o.iterations;
     last_resid = o.residual;
     last_ok = o.success ? 1 : 0;

@@ -11,6 +11,7 @@
 
 #include "../../include/flipmi.h"
 #include "flipmi_kernels.h"
+#include "multigrid.h"
 
 namespace flipmi {
 
@@ -241,10 +242,11 @@ struct Scene {
 
 // Pressure solve over caller grids already on the device (used by the
 // PressureSolver drop-in and by Scene::pressure_solve).
-// PCG iteration batches captured as HIP graphs, one per (batch size, s32
-// buffer the batch starts from); replayed instead of launching each kernel.
+// PCG iteration batches captured as HIP graphs, one per (batch size, state of
+// the buffers that the iterations swap); replayed instead of launching each
+// kernel.
 struct PcgGraphs {
-    std::map<std::pair<int, const void *>, hipGraphExec_t> exec;
+    std::map<std::pair<int, int>, hipGraphExec_t> exec;
     PcgGraphs() {}
     PcgGraphs(const PcgGraphs &) = delete;
     PcgGraphs &operator=(const PcgGraphs &) = delete;
@@ -271,21 +273,27 @@ struct PressureOutcome {
     bool solved = false;  // the pressure update was applied
     int refinements = 0;
     int64_t rows = 0;
+    // The solution, where solved: on the device, until the next solve.
+    const double *x = nullptr;
+    PressureIndex index;
 };
-PressureOutcome run_pressure(const PressureWork &w, PressureBuffers &pb, PcgScalars *host_sc,
-                             hipStream_t s, Scene *prof);
+struct PressureStore;
+// host_sc: pinned host memory of at least kPressureStaging bytes.
+constexpr size_t kPressureStaging = 4096;
+static_assert(sizeof(PcgScalars) <= kPressureStaging && sizeof(MgScalars) <= kPressureStaging,
+              "the solvers' scalars are read back through the staging buffer");
+PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *host_sc, hipStream_t s, Scene *prof);
 
-// Device storage of one pressure system in slot order: arr[0..12] are the
-// FP64 slot arrays (diag, rhs, x, r, z, s, invdiag, Lx, Ly, Lz, Lxm, Lym,
+// Device storage of one pressure system.  FP64 path: in slot order,
+// arr[0..12] are the FP64 slot arrays (diag, rhs, x, r, z, s, invdiag, Lx, Ly, Lz, Lxm, Lym,
 // Lzm), arr[13] the reduction partials, wgt[0..2] the coupling weights
-// (wx, wy, wz).
+// (wx, wy, wz).  Mixed precision: the multigrid solver's levels; a system it
+// does not solve goes to the FP64 path, whose storage then replaces them.
 struct PressureStore {
     static constexpr int kSlotArrays = 13;
     static constexpr int kWeightArrays = 3;
-    static constexpr int kSlotArrays32 = 12;  // FP32 factor and vectors, s twice, q (mixed precision)
     DBuf<double> arr[kSlotArrays + 1];
     DBuf<float> wgt[kWeightArrays];
-    DBuf<float> arr32[kSlotArrays32];
     DBuf<unsigned long long> edge, mask;
     DBuf<unsigned> progress, ticket;
     DBuf<int> irange;
@@ -293,7 +301,18 @@ struct PressureStore {
     DBuf<PcgScalars> scal;
     PressureBuffers pb{};
     PcgGraphs graphs;             // captured iteration batches (pointers into these buffers)
+    MgSolver mg;                  // bound while its buffers are allocated
+    bool mg_on = false;
+    bool mg_dirty = false;        // the last solve may have left values that are not finite
+    DBuf<double> mg_f64[6], mg_part;
+    DBuf<float> mg_f32;
+    DBuf<int> mg_ints;
+    DBuf<int4> mg_bricks;
+    DBuf<MgScalars> mg_scal;
+    DBuf<MgCoarse> mg_coarse;
     void alloc(const GridGeom &g, hipStream_t s, bool mixed);
+    void alloc_slots(const GridGeom &g, hipStream_t s);
+    void release_multigrid();
     size_t device_bytes() const;
 };
 

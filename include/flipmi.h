@@ -43,7 +43,8 @@ typedef enum {
 
 typedef enum {
     FLIPMI_PCG_FP64 = 0,  /* reference arithmetic: FP64 vectors, alpha/beta as float */
-    FLIPMI_PCG_MIXED = 1  /* FP32 PCG, FP64 dots + iterative refinement */
+    FLIPMI_PCG_MIXED = 1  /* FP64 x, residuals and dots, FP32 directions and multigrid
+                             preconditioner; converged on the FP64 true residual */
 } flipmi_pcg_precision;
 
 typedef struct flipmi_ctx flipmi_ctx;
@@ -78,7 +79,8 @@ typedef struct {
     int pressure_ok;           /* 0 if the last pressure solve failed */
     double gpu_ms;             /* device time of the frame */
     int64_t pressure_rows;     /* last substep: rows of the Poisson system */
-    int pcg_refinements;       /* last substep, mixed precision: FP64 true residuals */
+    int pcg_refinements;       /* last substep, mixed precision: FP64 true residuals (0: the FP64
+                                  path solved it) */
 } flipmi_frame_stats;
 
 /* Per-stage device time accumulated since the last reset (hipEvents). */
@@ -106,7 +108,7 @@ enum {
     FLIPMI_STAGE_K_FORWARD = 14,
     FLIPMI_STAGE_K_BACKWARD = 15,
     FLIPMI_STAGE_K_UPDATE = 16,
-    FLIPMI_STAGE_K_RESIDUAL = 17,   /* mixed precision: FP64 true residual + forward sweep over it */
+    FLIPMI_STAGE_K_RESIDUAL = 17,   /* not timed */
     FLIPMI_STAGE_INFLOW = 18,       /* mesh inflow: particle mask and emission */
     FLIPMI_STAGE_SURFACE = 19       /* surface reconstruction (sort, field, marching cubes, smoothing) */
 };
@@ -299,9 +301,10 @@ int flipmi_scene_stage_times(flipmi_scene *scene, flipmi_stage_times *out, int r
  * stage, 2 additionally one pair around every PCG kernel launch. */
 int flipmi_scene_set_profiling(flipmi_scene *scene, int level);
 /* PCG kernels timed at profiling level 2, one bit per FLIPMI_STAGE_K_*
- * stage minus FLIPMI_STAGE_K_SPMV (bit 5: the true residual and, on the
- * mixed path, the forward sweep over it; the mixed path's forward sweep also
- * does its axpy, so its FLIPMI_STAGE_K_AXPY stays empty); default all.
+ * stage minus FLIPMI_STAGE_K_SPMV; default all.  On the mixed path AXPY is
+ * the axpy with the first smoothing, FORWARD the restriction, UPDATE the
+ * coarse correction and BACKWARD the last smoothing, each on the finest
+ * level; FLIPMI_STAGE_K_RESIDUAL (bit 5) stays empty.
  * Each timed launch adds an event pair, which delays the launches around it. */
 int flipmi_scene_set_kernel_timing(flipmi_scene *scene, unsigned mask);
 /* Times the selected kernels on every `every`-th PCG iteration only (default
@@ -310,7 +313,7 @@ int flipmi_scene_set_kernel_timing(flipmi_scene *scene, unsigned mask);
 int flipmi_scene_set_kernel_sampling(flipmi_scene *scene, int every);
 /* Not in the reference: run the PCG's iteration batches as HIP graphs,
  * each (batch size, starting buffer) captured on first use and replayed
- * afterwards, so a batch of k iterations is one launch instead of 5 k.
+ * afterwards, so a batch of iterations is one launch.
  * Results are bit-identical either way.  Off by default; graphs are not
  * used while PCG kernels are timed (profiling level 2). */
 int flipmi_scene_set_launch_graphs(flipmi_scene *scene, int enabled);
@@ -397,7 +400,7 @@ typedef struct {
     double residual;           /* "Estimated Error" (|r|_inf) */
     int rows;                  /* fluid interior cells */
     int success;               /* the bool PressureSolver::solve returns */
-    int refinements;           /* mixed precision: outer refinement passes */
+    int refinements;           /* mixed precision: FP64 true residuals (0: the FP64 path solved it) */
 } flipmi_pressure_report;
 
 /* bool PressureSolver::solve(PressureSolverParameters) + getSolverStatus()

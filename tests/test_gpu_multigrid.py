@@ -1,0 +1,108 @@
+"""The mixed-precision solve's multigrid preconditioner where it can go wrong.
+
+Level sizes: bricks are 64 x 2 x 2 cells, levels halve with an odd cell left
+over, levels of up to 2048 cells are done by one workgroup; the grids below
+leave remainders on every axis, have one to three levels above that workgroup
+and, the smallest, a single cell per level.  Both paths stop on the same FP64
+true residual, 1e-9 of |b|_inf, so the pressures agree to the bound the mixed
+path states (1e-6 of the largest) and the velocities to 1e-5 of the fastest.
+
+What the preconditioner does not solve goes to the FP64 path, with that
+path's results bit for bit: an iteration cap below its need, values that are
+not finite, and a pocket that borders no air (its pressure is fixed up to a
+constant only).
+"""
+
+import numpy as np
+import pytest
+
+from tests.helpers import bits_equal, dam, pocket_inputs
+from tests.test_gpu_mixed import _projection_inputs
+
+pytestmark = pytest.mark.gpu
+
+FP64, MIXED = 0, 1
+
+
+def _both(gpu, inputs, dims, **kw):
+    dx, _, weights, liquid, mac, valid = inputs
+    return [gpu.pressure_solve(*dims, dx, 1 / 60, liquid, weights, mac, valid, precision=p, **kw)
+            for p in (FP64, MIXED)]
+
+
+@pytest.mark.parametrize("dims", [(8, 5, 6), (66, 9, 7), (67, 35, 34), (131, 20, 18), (30, 67, 26), (90, 70, 74)])
+@pytest.mark.parametrize("box", [(0.0, 0.0, 0.0, 0.45, 0.6, 1.0), (0.3, 0.0, 0.1, 1.0, 0.55, 0.9)])
+def test_level_sizes(gpu, oracle, dims, box):
+    inputs = _projection_inputs(oracle, *dims, seed=5, box=box)
+    a, b = _both(gpu, inputs, dims)
+    assert a["ok"] == b["ok"] == 1 and a["rows"] == b["rows"] > 0
+    # One true residual confirms the solve; 0: the FP64 path did it, which only
+    # the smallest grid calls for (cells of its single layer touch no air).
+    assert b["refinements"] == 1 or dims == (8, 5, 6)
+    assert np.abs(a["soln"] - b["soln"]).max() <= 1e-6 * np.abs(a["soln"]).max()
+    vmax = max(float(np.abs(g).max()) for g in a["mac"])
+    for x, y in zip(a["mac"], b["mac"]):
+        assert np.abs(x.astype(np.float64) - y).max() <= 1e-5 * vmax
+    for x, y in zip(a["valid"], b["valid"]):
+        assert bits_equal(x, y)
+
+
+def test_no_rows(gpu, oracle):
+    for dims in ((2, 5, 5), (3, 3, 3)):
+        z = [np.zeros(s, np.float32) for s in ((dims[2], dims[1], dims[0] + 1), (dims[2], dims[1] + 1, dims[0]),
+                                               (dims[2] + 1, dims[1], dims[0]))]
+        phi = np.ones(dims[::-1], np.float32)
+        valid = [np.zeros(g.shape, np.uint8) for g in z]
+        for p in (FP64, MIXED):
+            r = gpu.pressure_solve(*dims, 0.1, 0.01, phi, (*z, np.zeros_like(phi)), z, valid, precision=p)
+            assert r["ok"] == 1 and r["rows"] == 0 and r["iters"] == 0
+
+
+@pytest.mark.parametrize("cap", [1, 4])
+def test_capped_solve_is_the_fp64_paths(gpu, oracle, cap):
+    dims = (24, 28, 21)
+    a, b = _both(gpu, _projection_inputs(oracle, *dims), dims, maxiter=cap)
+    assert a["iters"] == b["iters"] == cap and a["ok"] == b["ok"] and a["err"] == b["err"]
+    assert bits_equal(a["soln"], b["soln"])
+    for x, y in zip(a["mac"], b["mac"]):
+        assert bits_equal(x, y)
+
+
+def test_not_finite(gpu, oracle):
+    dims = (24, 28, 21)
+    inputs = list(_projection_inputs(oracle, *dims))
+    bad = [g.copy() for g in inputs[4]]
+    bad[0][10, 8, 5] = np.nan
+    a, b = _both(gpu, [*inputs[:4], bad, inputs[5]], dims)
+    assert a["ok"] == b["ok"] == 0
+    for x, y in zip(a["mac"], b["mac"]):
+        assert bits_equal(x, y)
+    a, b = _both(gpu, inputs, dims)
+    assert a["ok"] == b["ok"] == 1
+
+
+def test_pocket_keeps_its_constant(gpu, oracle):
+    dims = (20, 18, 17)
+    dx, solid, weights, liquid, mac, valid, *_ = pocket_inputs(oracle, *dims)
+    a, b = _both(gpu, (dx, solid, weights, liquid, mac, valid), dims)
+    assert a["ok"] == b["ok"] == 1 and bits_equal(a["soln"], b["soln"])
+
+
+def test_scene_goes_on_after_the_fp64_path_took_over(gpu):
+    import flipengine3d_amd as fa
+    n = 24
+    s = dam(n, n, n, seed=2)
+    sims = []
+    for prec in (fa.PCG_FP64, fa.PCG_MIXED):
+        sim = fa.FluidSimulation(n, n, n, s.dx, ctx=gpu, precision=prec)
+        sim.addBodyForce(0.0, -9.81, 0.0)
+        sim.setPressureSolverTolerance(1e-9, 5)
+        sim.loadMarkerParticleData(s.positions, s.velocities)
+        sim.initialize()
+        sim.set_launch_graphs(True)
+        sims.append(sim)
+    for f in range(3):
+        st = [sim.update(1 / 60) for sim in sims]
+        assert st[0].pressure_ok == st[1].pressure_ok and st[0].pcg_iterations == st[1].pcg_iterations
+        for x, y in zip(sims[0].particles(), sims[1].particles()):
+            assert bits_equal(x, y)
