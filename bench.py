@@ -48,8 +48,8 @@ KERNEL_SAMPLE = 8
 #   backward:   z r/w, invdiag, 3 upper factor entries, and
 #               r for the fused z.r                         -> 7 x 8
 #   update_s:   z, s r/w                                    -> 3 x 8
-# A MIC(0) iteration with FP32 vectors and factor, FP64 x and matrix entries,
-# is the yardstick of the mixed path (its kernels are those of KERNEL_BYTES):
+# A mixed MIC(0) iteration, FP32 vectors and factor, FP64 x and matrix entries
+# (scenes under 2^20 cells):
 #   spmv_dot:   z, old s, matrix, new s, q (= A s)          -> 4 + 4 + 20 + 4 + 4
 #   forward with the axpy folded in: r r/w, q, invdiag, 3 lower factor
 #               entries, z, and x r/w (FP64), s             -> 8 + 4 + 4 + 12 + 4 + 16 + 4
@@ -64,8 +64,7 @@ PCG_BYTES = {
 }
 TRUE_RESIDUAL_BYTES = 40 + 24
 
-# What the measured path's kernels move at least, per row.  The mixed path is
-# conjugate gradients with a multigrid V-cycle; FP64 x, r, q and diagonal,
+# The same for a mixed iteration with the multigrid V-cycle (larger scenes): FP64 x, r, q and diagonal,
 # FP32 couplings (12), inverse diagonal and cycle vectors:
 #   spmv_dot:   z, old s, matrix, new s, q                   -> 4 + 4 + 20 + 4 + 8
 #   axpy_norm:  r, q, x r/w, s, r', inverse diagonal,
@@ -81,12 +80,15 @@ TRUE_RESIDUAL_BYTES = 40 + 24
 # reads x, b and the matrix and writes r: 8 + 8 + 20 + 8.
 KERNEL_BYTES = {
     "fp64": PCG_BYTES["fp64"],
+    "mixed_mic0": PCG_BYTES["mixed"],
     "mixed": {"k_spmv_dot": 40, "k_axpy_norm": 68, "k_forward": 24.5, "k_backward": 36, "k_update_s": 28.5},
 }
-COARSE_LEVEL_BYTES = {"fp64": 0.0, "mixed": (24 + 24.5 + 28.5 + 28) / 7}
-MIXED_TRUE_RESIDUAL_BYTES = 44
+COARSE_LEVEL_BYTES = {"fp64": 0.0, "mixed_mic0": 0.0, "mixed": (24 + 24.5 + 28.5 + 28) / 7}
+RESIDUAL_BYTES = {"fp64": 0, "mixed_mic0": TRUE_RESIDUAL_BYTES, "mixed": 44}
+MULTIGRID_CELLS = 1 << 20  # mixed scenes below this keep MIC(0)
 KERNEL_NAMES = {
     "fp64": {"k_forward": "k_sweep<forward>", "k_backward": "k_sweep<backward>"},
+    "mixed_mic0": {"k_forward": "k_sweep<forward>", "k_backward": "k_sweep<backward>"},
     "mixed": {"k_spmv_dot": "k_mg_spmv", "k_axpy_norm": "k_mg_axpy_smooth", "k_forward": "k_mg_restrict",
               "k_update_s": "k_mg_correct", "k_backward": "k_mg_smooth_up"},
 }
@@ -251,13 +253,15 @@ def run_gpu(fa, scene, args, precision, steps, warmup, profiling):
         st = sim.update(args.dt)
         log(f"{precision} warmup {w}: {st.pcg_iterations} PCG iterations, {st.gpu_ms:.1f} ms", args)
         n = st.num_particles
+    I, J, K = args.size
+    path = "mixed_mic0" if precision == "mixed" and I * J * K < MULTIGRID_CELLS else precision
     kern = None
     if profiling >= 2:
         # The warmup timed every PCG kernel; the timed region times only the
         # dominant one, on every KERNEL_SAMPLE-th iteration (each timed launch
         # costs an event pair, which delays the launches around it).
         wt = sim.stage_times()
-        kern = max(KERNEL_BYTES[precision], key=lambda k: wt[k][0])
+        kern = max(KERNEL_BYTES[path], key=lambda k: wt[k][0])
         sim.set_kernel_timing([kern], every=KERNEL_SAMPLE)
     sim.stage_times(reset=True)
 
@@ -284,12 +288,12 @@ def run_gpu(fa, scene, args, precision, steps, warmup, profiling):
     times = sim.stage_times()
     sim.close()
 
-    per_row = KERNEL_BYTES[precision]
+    per_row = KERNEL_BYTES[path]
     rows_per_launch = rows_iters / max(iters, 1)
     # PCG bandwidth: algorithmic bytes of every iteration plus those of each
     # true residual, over the PCG stage time.
-    pcg_bytes = (rows_iters * (sum(per_row.values()) + COARSE_LEVEL_BYTES[precision])
-                 + refinements * rows_per_launch * MIXED_TRUE_RESIDUAL_BYTES)
+    pcg_bytes = (rows_iters * (sum(per_row.values()) + COARSE_LEVEL_BYTES[path])
+                 + refinements * rows_per_launch * RESIDUAL_BYTES[path])
     pcg_ms = times["pcg"][0]
     roof = {"kernel": None, "bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": None, "traffic": None}
@@ -304,7 +308,7 @@ def run_gpu(fa, scene, args, precision, steps, warmup, profiling):
         achieved = bytes_per_launch / launch_s / 1e9 if launch_s > 0 else 0.0
         traffic = MEASURED_TRAFFIC.get((precision, tuple(args.size)), {}).get(kern)
         roof.update({
-            "kernel": KERNEL_NAMES[precision].get(kern, kern),
+            "kernel": KERNEL_NAMES[path].get(kern, kern),
             "achieved": achieved,
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": traffic,

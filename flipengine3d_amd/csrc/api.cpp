@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <initializer_list>
 #include <memory>
 #include <new>
 #include <vector>
@@ -54,19 +55,35 @@ template <class T>
 void alloc_dev(DBuf<T> &d, size_t n) {
     if (d.alloc(n) != hipSuccess) throw StatusError{FLIPMI_ERR_OOM, "out of device memory"};
 }
+// Copies results to the caller; returns when they are there.
 template <class T>
-void download(T *h, const DBuf<T> &d, size_t n, hipStream_t s) {
-    if (n) hipck(hipMemcpyAsync(h, d.p, sizeof(T) * n, hipMemcpyDeviceToHost, s), "download");
+void download(Ctx &c, T *h, const DBuf<T> &d, size_t n, hipStream_t s) {
+    if (n) hipck(c.link().to_host(h, d.p, sizeof(T) * n, s), "download");
+}
+template <class T>
+HostPiece piece(T *h, const DBuf<T> &d) {
+    return HostPiece{h, d.p, h ? sizeof(T) * d.n : 0};
+}
+void download(Ctx &c, std::initializer_list<HostPiece> pieces, hipStream_t s) {
+    hipck(c.link().to_host(pieces.begin(), (int)pieces.size(), s), "download");
 }
 
-// AoS float3 on the host -> three SoA device arrays.
+// A built mesh to the caller's arrays (null: not copied).
+void copy_mesh(Ctx &c, const SurfaceStore &st, float *verts, int32_t *tris, hipStream_t s) {
+    download(c,
+             {HostPiece{verts, st.verts.p, verts ? 3 * sizeof(float) * (size_t)st.nverts : 0},
+              HostPiece{tris, st.tris.p, tris ? 3 * sizeof(int32_t) * (size_t)st.ntris : 0}},
+             s);
+}
+
+// xyz triples on the host -> three component arrays, taken apart on the
+// device.
 void upload_soa(DBuf<float> out[3], const float *xyz, int64_t n, hipStream_t s) {
-    std::vector<float> t((size_t)n);
-    for (int a = 0; a < 3; a++) {
-        for (int64_t q = 0; q < n; q++) t[q] = xyz[3 * q + a];
-        upload(out[a], t.data(), (size_t)n, s);
-        hipck(hipStreamSynchronize(s), "sync");
-    }
+    for (int a = 0; a < 3; a++) alloc_dev(out[a], (size_t)n);
+    DBuf<float> triples;
+    upload(triples, xyz, 3 * (size_t)n, s);
+    float *dst[3] = {out[0].p, out[1].p, out[2].p};
+    hipck(launch_unpack_triples(triples.p, (int)n, dst, s), "unpack");
 }
 
 }  // namespace
@@ -95,6 +112,12 @@ int flipmi_ctx_create(int device, flipmi_ctx **out) {
     flipmi_ctx *c = new (std::nothrow) flipmi_ctx();
     if (!c) return FLIPMI_ERR_OOM;
     c->c.device = device;
+    try {
+        c->c.shared = DeviceShared::of(device);
+    } catch (...) {
+        delete c;
+        return FLIPMI_ERR_OOM;
+    }
     if (hipStreamCreateWithFlags(&c->c.stream, hipStreamNonBlocking) != hipSuccess) {
         delete c;
         return FLIPMI_ERR_HIP;
@@ -293,38 +316,15 @@ int flipmi_scene_get_particles_range(flipmi_scene *scene, int64_t start, int64_t
     if (!s.initialized) return fail(s.ctx, FLIPMI_ERR_NOT_INITIALIZED, "scene not initialized");
     if (start < 0 || end > (int64_t)s.n || start > end)
         return fail(s.ctx, FLIPMI_ERR_INVALID_ARG, "invalid particle range");
-    const int64_t m = end - start;
-    if (m == 0) return FLIPMI_OK;
-    return guarded(s.ctx, [&] {
-        std::vector<float> t((size_t)m);
-        for (int a = 0; a < 6; a++) {
-            float *dst = a < 3 ? pos : vel;
-            if (!dst) continue;
-            hipck(hipMemcpyAsync(t.data(), s.part[a].p + start, sizeof(float) * m, hipMemcpyDeviceToHost, s.stream),
-                  "download");
-            hipck(hipStreamSynchronize(s.stream), "sync");
-            for (int64_t q = 0; q < m; q++) dst[3 * (size_t)q + (a % 3)] = t[q];
-        }
-        if (pos) s.to_domain(pos, m);
-    });
+    if (end == start) return FLIPMI_OK;
+    return guarded(s.ctx, [&] { s.read_particles(start, end - start, pos, vel); });
 }
 
 int flipmi_scene_get_particles(flipmi_scene *scene, float *pos, float *vel) {
     if (!scene) return FLIPMI_ERR_INVALID_ARG;
     Scene &s = scene->s;
     if (!s.initialized) return fail(s.ctx, FLIPMI_ERR_NOT_INITIALIZED, "scene not initialized");
-    return guarded(s.ctx, [&] {
-        std::vector<float> t((size_t)s.n);
-        for (int a = 0; a < 6; a++) {
-            float *dst = a < 3 ? pos : vel;
-            if (!dst || s.n == 0) continue;
-            hipck(hipMemcpyAsync(t.data(), s.part[a].p, sizeof(float) * s.n, hipMemcpyDeviceToHost, s.stream),
-                  "download");
-            hipck(hipStreamSynchronize(s.stream), "sync");
-            for (int q = 0; q < s.n; q++) dst[3 * (size_t)q + (a % 3)] = t[q];
-        }
-        if (pos) s.to_domain(pos, s.n);
-    });
+    return guarded(s.ctx, [&] { s.read_particles(0, s.n, pos, vel); });
 }
 
 void flipmi_surface_desc_default(flipmi_surface_desc *d) {
@@ -360,7 +360,7 @@ int flipmi_scene_get_isomesh(flipmi_scene *scene, int64_t *num_vertices, int64_t
         const bool have = s.mesh && s.mesh->valid;
         *num_vertices = have ? s.mesh->nverts : 0;
         *num_triangles = have ? s.mesh->ntris : 0;
-        if (have) copy_surface(*s.mesh, vertices_xyz, triangles, s.stream);
+        if (have) copy_mesh(*s.ctx, *s.mesh, vertices_xyz, triangles, s.stream);
     });
 }
 
@@ -400,14 +400,12 @@ int flipmi_scene_get_grid(flipmi_scene *scene, int which, void *out) {
                 alloc_dev(counts, nc);
                 hipck(launch_removal_counts(s.g, s.count.p, s.removed_in_cell.p, 250, counts.p, s.stream),
                       "removal counts");
-                download((int *)out, counts, nc, s.stream);
-                hipck(hipStreamSynchronize(s.stream), "sync");
+                download(*s.ctx, (int *)out, counts, nc, s.stream);
                 return;
             }
             default: throw StatusError{FLIPMI_ERR_INVALID_ARG, "unknown grid id"};
         }
-        hipck(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, s.stream), "download");
-        hipck(hipStreamSynchronize(s.stream), "sync");
+        hipck(s.ctx->link().to_host(out, src, bytes, s.stream), "download");
     });
 }
 
@@ -453,6 +451,7 @@ int flipmi_domain_solid(flipmi_ctx *ctx, int I, int J, int K, double dx, float *
     return guarded(&ctx->c, [&] {
         GridGeom g = make_geom(I, J, K, dx);
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         size_t nn = (size_t)(I + 1) * (J + 1) * (K + 1);
         DBuf<float> phi, dU, dV, dW, dC;
         alloc_dev(phi, nn);
@@ -461,12 +460,7 @@ int flipmi_domain_solid(flipmi_ctx *ctx, int I, int J, int K, double dx, float *
         BoxMesh mesh = make_domain_box(I, J, K, dx);
         hipck(launch_domain_solid(g, mesh, phi.p, s), "domain solid");
         hipck(launch_weights(g, phi.p, dU.p, dV.p, dW.p, dC.p, s), "weights");
-        download(phi_nodal, phi, nn, s);
-        if (wU) download(wU, dU, dU.n, s);
-        if (wV) download(wV, dV, dV.n, s);
-        if (wW) download(wW, dW, dW.n, s);
-        if (wC) download(wC, dC, dC.n, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, {piece(phi_nodal, phi), piece(wU, dU), piece(wV, dV), piece(wW, dW), piece(wC, dC)}, s);
     });
 }
 
@@ -508,6 +502,7 @@ int flipmi_liquid_sdf(flipmi_ctx *ctx, int I, int J, int K, double dx, const flo
     return guarded(&ctx->c, [&] {
         GridGeom g = make_geom(I, J, K, dx);
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         SortedParticles sp;
         sp.build(g, pos, nullptr, n, s, true);
         size_t nn = (size_t)(I + 1) * (J + 1) * (K + 1);
@@ -515,8 +510,7 @@ int flipmi_liquid_sdf(flipmi_ctx *ctx, int I, int J, int K, double dx, const flo
         if (solid_phi_nodal) upload(solid, solid_phi_nodal, nn, s);
         alloc_dev(phi, (size_t)I * J * K);
         hipck(launch_liquid_sdf(g, sp.spos.p, sp.offset.p, radius, solid.p, phi.p, s), "liquid sdf");
-        download(phi_out, phi, phi.n, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, phi_out, phi, phi.n, s);
     });
 }
 
@@ -526,6 +520,7 @@ int flipmi_removal_counts(flipmi_ctx *ctx, int I, int J, int K, double dx, const
     return guarded(&ctx->c, [&] {
         GridGeom g = make_geom(I, J, K, dx);
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         SortedParticles sp;
         sp.build(g, pos, nullptr, n, s);
         const size_t nc = (size_t)I * J * K;
@@ -542,8 +537,7 @@ int flipmi_removal_counts(flipmi_ctx *ctx, int I, int J, int K, double dx, const
         hipck(launch_removed_in_cell(g, sp.raw[0].p, sp.raw[1].p, sp.raw[2].p, rm.p, (int)n, ric.p, s),
               "removed in cell");
         hipck(launch_removal_counts(g, sp.count.p, ric.p, 250, out.p, s), "removal counts");
-        download(counts_out, out, nc, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, counts_out, out, nc, s);
     });
 }
 
@@ -573,6 +567,7 @@ int flipmi_mesh_particles(flipmi_ctx *ctx, int I, int J, int K, double dx, const
                     throw StatusError{FLIPMI_ERR_INVALID_ARG, "particle positions must lie inside the grid"};
             }
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         SortedParticles sp;
         sp.build(g, pos, nullptr, n, s, true);
         DBuf<float> solid;
@@ -587,6 +582,7 @@ int flipmi_mesh_particles(flipmi_ctx *ctx, int I, int J, int K, double dx, const
         in.kernel_radius = kernel_radius > 0.0 ? kernel_radius : marker_particle_radius(dx) * desc->particle_scale;
         for (int a = 0; a < 3; a++) in.domain_offset[a] = domain_offset ? (float)domain_offset[a] : 0.0f;
         in.domain_scale = domain_scale;
+        PoolScope::Off kept;  // the mesh outlives this call
         build_surface(in, m->st, s);
         hipck(hipStreamSynchronize(s), "sync");
     });
@@ -607,7 +603,8 @@ int flipmi_mesh_counts(flipmi_mesh *mesh, int64_t *num_vertices, int64_t *num_tr
 
 int flipmi_mesh_copy(flipmi_mesh *mesh, float *vertices_xyz, int32_t *triangles) {
     if (!mesh) return FLIPMI_ERR_INVALID_ARG;
-    return guarded(&mesh->ctx->c, [&] { copy_surface(mesh->st, vertices_xyz, triangles, mesh->ctx->c.stream); });
+    return guarded(&mesh->ctx->c,
+                   [&] { copy_mesh(mesh->ctx->c, mesh->st, vertices_xyz, triangles, mesh->ctx->c.stream); });
 }
 
 int flipmi_mesh_destroy(flipmi_mesh *mesh) {
@@ -621,13 +618,13 @@ int flipmi_liquid_sdf_postprocess(flipmi_ctx *ctx, int I, int J, int K, double d
     return guarded(&ctx->c, [&] {
         GridGeom g = make_geom(I, J, K, dx);
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         size_t nn = (size_t)(I + 1) * (J + 1) * (K + 1);
         DBuf<float> solid, phi;
         upload(solid, solid_phi_nodal, nn, s);
         upload(phi, phi_inout, (size_t)I * J * K, s);
         hipck(launch_liquid_postprocess(g, solid.p, phi.p, s), "liquid post-process");
-        download(phi_inout, phi, phi.n, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, phi_inout, phi, phi.n, s);
     });
 }
 
@@ -639,6 +636,7 @@ int flipmi_p2g(flipmi_ctx *ctx, int I, int J, int K, double dx, const float *pos
     return guarded(&ctx->c, [&] {
         GridGeom g = make_geom(I, J, K, dx);
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         SortedParticles sp;
         sp.build(g, pos, vel, n, s, true);
         DBuf<float> du, dv, dw;
@@ -653,9 +651,7 @@ int flipmi_p2g(flipmi_ctx *ctx, int I, int J, int K, double dx, const float *pos
         uint8_t *valids[3] = {dvu.p, dvv.p, dvw.p};
         hipck(launch_p2g(g, sp.spos.p, svel, sp.offset.p, (int)n, radius, outs, valids, ovf_count.p, ovf.p, s),
               "p2g");
-        download(u, du, du.n, s); download(v, dv, dv.n, s); download(w, dw, dw.n, s);
-        download(vu, dvu, dvu.n, s); download(vv, dvv, dvv.n, s); download(vw, dvw, dvw.n, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, {piece(u, du), piece(v, dv), piece(w, dw), piece(vu, dvu), piece(vv, dvv), piece(vw, dvw)}, s);
     });
 }
 
@@ -666,6 +662,7 @@ int flipmi_extrapolate(flipmi_ctx *ctx, int ni, int nj, int nk, float *grid, con
     if ((double)ni * nj * nk >= 4294967296.0) return FLIPMI_ERR_INVALID_ARG;  // 32-bit kernel indexing
     return guarded(&ctx->c, [&] {
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         size_t n = (size_t)ni * nj * nk;
         DBuf<float> dg;
         DBuf<uint8_t> dv, st;
@@ -673,8 +670,7 @@ int flipmi_extrapolate(flipmi_ctx *ctx, int ni, int nj, int nk, float *grid, con
         upload(dv, valid, n, s);
         alloc_dev(st, n);
         hipck(launch_extrapolate(ni, nj, nk, dg.p, dv.p, st.p, layers, s), "extrapolate");
-        download(grid, dg, n, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, grid, dg, n, s);
     });
 }
 
@@ -687,6 +683,7 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
         GridGeom g = make_geom(a->isize, a->jsize, a->ksize, a->dx);
         if (a->max_iterations < 1) throw StatusError{FLIPMI_ERR_INVALID_ARG, "max_iterations must be positive"};
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         int I = a->isize, J = a->jsize, K = a->ksize;
         size_t nc = (size_t)I * J * K, nU = (size_t)(I + 1) * J * K, nV = (size_t)I * (J + 1) * K,
                nW = (size_t)I * J * (K + 1);
@@ -709,7 +706,8 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
         const bool solid_given = a->solid_u || a->solid_v || a->solid_w;
         if (a->precision != FLIPMI_PCG_FP64 && a->precision != FLIPMI_PCG_MIXED)
             throw StatusError{FLIPMI_ERR_INVALID_ARG, "unknown pcg precision"};
-        bool mixed = a->precision == FLIPMI_PCG_MIXED;
+        const bool mixed = a->precision == FLIPMI_PCG_MIXED;
+        bool multigrid = mixed;
         if (solid_given || mixed) {
             DBuf<int> parent, found;
             DBuf<unsigned> flags;
@@ -725,52 +723,45 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
             // The pressure of a pocket that borders no air is fixed up to a
             // constant only, which follows from the preconditioner.  Callers
             // of this entry point see the pressures, so such a system keeps
-            // the reference's (a scene uses their differences alone).
-            if (pocket) mixed = false;
+            // MIC(0) (a scene uses their differences alone).
+            if (pocket) multigrid = false;
         }
         PressureStore ps;
-        ps.alloc(g, s, mixed);
+        ps.alloc(g, s, mixed, multigrid);
         PressureWork pw;
         pw.g = g; pw.dt = a->dt; pw.tol = a->tolerance; pw.acceptable = a->acceptable_tolerance;
         pw.maxiter = a->max_iterations; pw.precision = a->precision;
         pw.liquid = liq.p; pw.wU = wu.p; pw.wV = wv.p; pw.wW = ww.p; pw.wC = wc.p;
         pw.sU = su.p; pw.sV = sv.p; pw.sW = sw.p;
         pw.u = u.p; pw.v = v.p; pw.w = w.p; pw.vu = vu.p; pw.vv = vv.p; pw.vw = vw.p;
+        static_assert(kPressureStaging <= HostLink::kPage, "the solver's staging is one page");
         void *hs = nullptr;
-        hipck(hipHostMalloc(&hs, kPressureStaging, hipHostMallocDefault), "pinned");
+        hipck(ctx->c.link().get_page(&hs), "pinned");
         PressureOutcome o;
         try {
             o = run_pressure(pw, ps, hs, s, nullptr);
         } catch (...) {
-            (void)hipHostFree(hs);
+            (void)hipStreamSynchronize(s);
+            ctx->c.link().put_page(hs);
             throw;
         }
-        (void)hipHostFree(hs);
+        ctx->c.link().put_page(hs);
         ok = o.success;
-        download(a->u, u, nU, s); download(a->v, v, nV, s); download(a->w, w, nW, s);
-        download(a->valid_u, vu, nU, s); download(a->valid_v, vv, nV, s); download(a->valid_w, vw, nW, s);
-        if (a->solid_u) download(a->solid_u, su, nU, s);
-        if (a->solid_v) download(a->solid_v, sv, nV, s);
-        if (a->solid_w) download(a->solid_w, sw, nW, s);
-        std::vector<float> hl(nc);
-        int rows = 0;
-        std::vector<double> x;
-        if (a->pressure_rows && o.solved) {
-            x.resize(o.index.count);
-            hipck(hipMemcpyAsync(x.data(), o.x, x.size() * sizeof(double), hipMemcpyDeviceToHost, s), "download");
-        }
-        download(hl.data(), liq, nc, s);
-        hipck(hipStreamSynchronize(s), "sync");
         // Rows in reference order: interior cells, k outer, j, i inner, phi < 0.
-        for (int k = 1; k < K - 1; k++)
-            for (int j = 1; j < J - 1; j++)
-                for (int i = 1; i < I - 1; i++) {
-                    size_t c = (size_t)i + (size_t)I * ((size_t)j + (size_t)J * k);
-                    if (hl[c] < 0) {
-                        if (a->pressure_rows) a->pressure_rows[rows] = o.solved ? x[o.index(i, j, k)] : 0.0;
-                        rows++;
-                    }
-                }
+        DBuf<int> flags, pos, scan, count;
+        DBuf<double> row_values;
+        alloc_dev(flags, nc); alloc_dev(pos, nc); alloc_dev(scan, scan_scratch_elems((int)nc)); alloc_dev(count, 1);
+        alloc_dev(row_values, nc);
+        hipck(launch_gather_rows(g, liq.p, o.solved ? o.x : nullptr, o.index, flags.p, pos.p, scan.p, row_values.p,
+                                 count.p, s),
+              "pressure rows");
+        int rows = 0;
+        download(ctx->c,
+                 {piece(a->u, u), piece(a->v, v), piece(a->w, w), piece(a->valid_u, vu), piece(a->valid_v, vv),
+                  piece(a->valid_w, vw), piece(a->solid_u, su), piece(a->solid_v, sv), piece(a->solid_w, sw),
+                  piece(&rows, count)},
+                 s);
+        if (a->pressure_rows) download(ctx->c, a->pressure_rows, row_values, (size_t)rows, s);
         if (rep) {
             rep->iterations = o.iterations;
             rep->residual = o.residual;
@@ -790,6 +781,7 @@ int flipmi_mic0_apply(flipmi_ctx *ctx, int I, int J, int K, double dx, double dt
     return guarded(&ctx->c, [&] {
         GridGeom g = make_geom(I, J, K, dx);
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         size_t nc = (size_t)I * J * K, nU = (size_t)(I + 1) * J * K, nV = (size_t)I * (J + 1) * K,
                nW = (size_t)I * J * (K + 1);
         DBuf<float> liq, wu, wv, ww, wc, zero_u, zero_v, zero_w;
@@ -800,7 +792,7 @@ int flipmi_mic0_apply(flipmi_ctx *ctx, int I, int J, int K, double dx, double dt
         hipck(launch_fill_f32(zero_v.p, nV, 0.0f, s), "fill");
         hipck(launch_fill_f32(zero_w.p, nW, 0.0f, s), "fill");
         PressureStore ps;
-        ps.alloc_slots(g, s);
+        ps.alloc_slots(g, s, false);
         hipck(launch_pressure_reset(ps.pb, s), "reset");
         hipck(launch_pressure_assemble(g, dt, liq.p, wu.p, wv.p, ww.p, wc.p, zero_u.p, zero_v.p, zero_w.p,
                                        zero_u.p, zero_v.p, zero_w.p, ps.pb, s),
@@ -808,8 +800,7 @@ int flipmi_mic0_apply(flipmi_ctx *ctx, int I, int J, int K, double dx, double dt
         hipck(launch_group_mask(ps.pb, s), "group mask");
         hipck(launch_mic0_factor(g, liq.p, ps.pb, s), "factor");
         // Scatter r from reference row order into slot order.
-        std::vector<float> hl(nc);
-        download(hl.data(), liq, nc, s);
+        const float *hl = liquid_phi;
         hipck(hipStreamSynchronize(s), "sync");
         const SlotMap &sm = ps.pb.sm;
         size_t ns = sm.count();
@@ -852,14 +843,14 @@ int flipmi_advect_particles(flipmi_ctx *ctx, int I, int J, int K, double dx, con
         GridGeom g = make_geom(I, J, K, dx);
         if (n > INT32_MAX / 3) throw StatusError{FLIPMI_ERR_INVALID_ARG, "too many particles"};
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         DBuf<float> du, dv, dw, pin, pout;
         upload(du, u, (size_t)(I + 1) * J * K, s); upload(dv, v, (size_t)I * (J + 1) * K, s);
         upload(dw, w, (size_t)I * J * (K + 1), s);
         upload(pin, pos_in, (size_t)n * 3, s);
         alloc_dev(pout, (size_t)n * 3);
         hipck(launch_advect_rk(g, du.p, dv.p, dw.p, pin.p, (int)n, dt, order, pout.p, s), "advect");
-        download(pos_out, pout, (size_t)n * 3, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, pos_out, pout, (size_t)n * 3, s);
     });
 }
 
@@ -870,14 +861,14 @@ int flipmi_trilinear_velocity(flipmi_ctx *ctx, int I, int J, int K, double dx, c
         GridGeom g = make_geom(I, J, K, dx);
         if (n > INT32_MAX / 3) throw StatusError{FLIPMI_ERR_INVALID_ARG, "too many particles"};
         hipStream_t s = ctx->c.stream;
+        PoolScope scope(ctx->c.shared->pool, s);
         DBuf<float> du, dv, dw, pin, pout;
         upload(du, u, (size_t)(I + 1) * J * K, s); upload(dv, v, (size_t)I * (J + 1) * K, s);
         upload(dw, w, (size_t)I * J * (K + 1), s);
         upload(pin, pos, (size_t)n * 3, s);
         alloc_dev(pout, (size_t)n * 3);
         hipck(launch_trilinear_velocity(g, du.p, dv.p, dw.p, pin.p, (int)n, pout.p, s), "trilinear");
-        download(vel_out, pout, (size_t)n * 3, s);
-        hipck(hipStreamSynchronize(s), "sync");
+        download(ctx->c, vel_out, pout, (size_t)n * 3, s);
     });
 }
 

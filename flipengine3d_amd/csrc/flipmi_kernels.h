@@ -132,6 +132,11 @@ struct PcgScalars {
     unsigned int rows;                  // rows of the system (fluid interior cells)
     unsigned long long absmax_bits;
     double mf;                          // dt / dx^2 of the assembled system (coupling scale)
+    // mixed precision: true-residual replacement ("reliable update")
+    double rmax;                        // |r| at the last true residual
+    double delta;                       // replace when |r32| < delta * rmax
+    int refresh;                        // a true residual is due
+    int refinements;                    // true residuals computed
     // Epoch of the next sweep launch: read by every workgroup of a sweep,
     // advanced by its last tile, so launches replayed from a captured graph
     // still tag their records afresh.  Starts at 1 (records start at 0).
@@ -192,6 +197,24 @@ struct PressureBuffers {
     double *x, *r, *z, *s;              // PCG vectors (FP64)
     double *invdiag, *Lx, *Ly, *Lz;     // MIC(0) factor: column entries (rows +x/+y/+z)
     double *Lxm, *Lym, *Lzm;            // the same entries read from the row: columns -x/-y/-z
+    // Mixed precision (null unless allocated): FP32 copies of the factor and
+    // the FP32 PCG vectors; x and the matrix stay FP64.
+    float *invdiag32, *Lx32, *Ly32, *Lz32, *Lxm32, *Lym32, *Lzm32;
+    float *r32, *z32, *s32;
+    // Mixed precision: the SpMV forms the new direction s = z + beta s from
+    // the old one, so s lives in two buffers: s32 is read, s32b written, and
+    // the host swaps them after each SpMV launch.  s_plain: the next SpMV
+    // reads s32 as it is (right after initialisation).
+    float *s32b;
+    int s_plain;
+    int s_turn;  // which of the two s32 is
+    void swap_directions() {
+        float *t = s32;
+        s32 = s32b;
+        s32b = t;
+        s_turn ^= 1;
+    }
+    float *q32;  // mixed precision: q = A s, read by the axpy
     double *partials;                   // per-block partial sums
     int npartials;
     unsigned long long *edge;           // tagged values a tile hands to its j / k neighbours
@@ -230,23 +253,34 @@ hipError_t launch_group_mask(PressureBuffers &pb, hipStream_t s);
 // Zeroes the factor, finds each column tile's row extent and factorises.
 hipError_t launch_mic0_factor(const GridGeom &g, const float *liquid, PressureBuffers &pb,
                               hipStream_t s);
-hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, PressureBuffers &pb, hipStream_t s);
-// The timed kernels of one PCG iteration.  FP64 path: SpMV, axpy, forward and
-// backward sweep, direction update.  Mixed precision (k_multigrid.hip): SpMV
-// with the direction update, axpy with the first smoothing, and of the
-// V-cycle on the finest level the restriction (kPcgForward), the coarse
-// correction (kPcgUpdate) and the last smoothing (kPcgBackward).
+// mixed: FP32 inner iteration with FP64 dots, FP64 x and true-residual
+// replacement (requires the FP32 arrays of pb).
+hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, bool mixed,
+                           PressureBuffers &pb, hipStream_t s);
+// The kernels of one PCG iteration.  The FP64 path runs spmv, axpy,
+// forward, backward, update.  The mixed MIC(0) iteration folds the axpy into
+// the forward sweep and the direction update into the SpMV, and runs
+// kPcgResidual (a true residual and a forward sweep over it) between the
+// forward and the backward sweep; it exits at once unless the forward sweep's
+// residual norm called for a true residual.  With multigrid
+// (k_multigrid.hip): the SpMV with the direction update, the axpy with the
+// first smoothing, and of the V-cycle on the finest level the restriction
+// (kPcgForward), the coarse correction (kPcgUpdate) and the last smoothing
+// (kPcgBackward).
 enum {
     kPcgSpmv = 0, kPcgAxpy = 1, kPcgForward = 2, kPcgBackward = 3, kPcgUpdate = 4,
     kPcgResidual = 5, kPcgPieces = 6
 };
-constexpr unsigned kPcgSweeps = 2;  // sweep launches per iteration (each takes a record epoch)
+bool pcg_piece_used(int piece, bool mixed);
+// Sweep launches per iteration (each takes a record epoch).
+inline unsigned pcg_sweeps_per_iteration(bool mixed) { return mixed ? 3u : 2u; }
 // With kt.start set, the kernel's dispatch records its start and end in the
 // two events.
 struct KernelTiming {
     hipEvent_t start = nullptr, stop = nullptr;
 };
-hipError_t launch_pcg_iteration(const GridGeom &g, PressureBuffers &pb, hipStream_t s,
+// One iteration; the pieces with a start event in kt are timed.
+hipError_t launch_pcg_iteration(const GridGeom &g, bool mixed, PressureBuffers &pb, hipStream_t s,
                                 const KernelTiming (&kt)[kPcgPieces]);
 // Where a solver keeps the pressure of interior cell (i, j, k): in slot order
 // or, dense, in the rows of the interior cells.
@@ -364,6 +398,16 @@ hipError_t launch_keep_flags(const float *vx, const float *vy, const float *vz, 
 hipError_t launch_compact_keep(const int *keep, int n, int *pos, int *scan_tmp,
                                const float *const src[6], float *const dst[6], int *new_count,
                                hipStream_t s);
+// SoA <-> xyz triples.  transform: out = in * scale + offset per axis, in
+// float, each operation rounded (positions to domain coordinates).
+hipError_t launch_pack_triples(const float *const src[3], int n, bool transform, float scale, const float offset[3],
+                               float *xyz, hipStream_t s);
+hipError_t launch_unpack_triples(const float *xyz, int n, float *const dst[3], hipStream_t s);
+// Pressures of the rows in the reference's order (interior cells of negative
+// phi, k outer, i inner): flags and pos are scratch, one int per cell, rows
+// takes at most one value per cell; *count = rows.  p null: zeros.
+hipError_t launch_gather_rows(const GridGeom &g, const float *liquid, const double *p, const PressureIndex &at,
+                              int *flags, int *pos, int *scan_tmp, double *rows, int *count, hipStream_t s);
 hipError_t launch_advect_rk(const GridGeom &g, const float *u, const float *v, const float *w,
                             const float *pin, int n, double dt, int order, float *pout,
                             hipStream_t s);

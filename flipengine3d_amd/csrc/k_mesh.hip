@@ -803,14 +803,4 @@ void build_surface(const SurfaceInputs &in, SurfaceStore &st, hipStream_t s) {
     st.ntris = nt;
 }
 
-void copy_surface(const SurfaceStore &st, float *verts_xyz, int32_t *tris, hipStream_t s) {
-    if (verts_xyz && st.nverts > 0)
-        hcheck(hipMemcpyAsync(verts_xyz, st.verts.p, 3 * (size_t)st.nverts * sizeof(float), hipMemcpyDeviceToHost, s),
-               "mesh copy");
-    if (tris && st.ntris > 0)
-        hcheck(hipMemcpyAsync(tris, st.tris.p, 3 * (size_t)st.ntris * sizeof(int), hipMemcpyDeviceToHost, s),
-               "mesh copy");
-    hcheck(hipStreamSynchronize(s), "mesh copy");
-}
-
 }  // namespace flipmi

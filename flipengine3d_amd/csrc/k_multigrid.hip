@@ -24,8 +24,9 @@
 // V-cycle has no such chain and takes 13 to 16 iterations at every size.
 // 256x128x128 double dam break, 1.23 M rows: 21.8 -> 3.2 ms per solve (factor
 // included).
-// The FP64 path keeps MIC(0), bit for bit; a solve that does not converge
-// here is redone there.
+// The FP64 path keeps MIC(0), bit for bit, and so do mixed scenes of request
+// size; a solve that does not converge here is redone with the FP32 MIC(0)
+// iteration.
 //
 // Layout.  Levels are dense grids of the interior cells, x fastest, with
 // zero padding that serves as the halo: a row of nx cells has pitch px > nx,

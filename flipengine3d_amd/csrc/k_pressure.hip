@@ -33,8 +33,8 @@ namespace flipmi {
 constexpr int kTile = 8;
 constexpr int kRedBlocks = 1024;
 // The axpy's grid: fewer, longer-lived blocks stream its four arrays faster
-// (with FP32 r and s on the 256x128x128 double dam break: 20.6 us per launch
-// with 1024 blocks, 15.7 with 512, 15.0 with 384, 16.1 with 256).  Its reduction
+// (mixed axpy on the 256x128x128 double dam break: 20.6 us per launch with
+// 1024 blocks, 15.7 with 512, 15.0 with 384, 16.1 with 256).  Its reduction
 // is a maximum, so the grid does not change any result; the SpMV's is a sum
 // whose order follows the grid, so it keeps kRedBlocks.  A multiple of kXcds.
 constexpr int kAxpyBlocks = 384;
@@ -314,9 +314,12 @@ hipError_t launch_group_mask(PressureBuffers &pb, hipStream_t s) {
 // ---------------------------------------------------------------------------
 
 enum { kFactor = 0, kForward = 1, kBackward = 2 };
-// A sweep launch's mode: whether it ends with the z.r dot of the first or of
-// a later iteration (backward).
-enum { kDotNone = 0, kDotInit = 1, kDotIter = 2 };
+// A sweep launch's mode: what it reduces or decides at its end.  Nothing;
+// the z.r dot of the first or a later iteration (backward); the residual
+// norm of the axpy the forward sweep did; or (forward, a launch that runs
+// only when a true residual is due) the norm of the true residual it
+// computes before sweeping.
+enum { kDotNone = 0, kDotInit = 1, kDotIter = 2, kAxpyNorm = 3, kTrueResidual = 4 };
 
 // Values another workgroup reads within the same kernel are stored and
 // loaded as relaxed device-scope atomics, which are coherent across XCDs by
@@ -369,8 +372,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_view(const void *base, 
 // Tagged records.  A record carries a value and the 32-bit epoch of the
 // launch that wrote it, in 64-bit words written and read as single-copy-
 // atomic accesses, so a reader that sees the current epoch in every word has
-// the whole value: two words holding 32 bits of it each.
-struct Record {
+// the whole value.  FP32: one word (epoch | bits); FP64: two words holding
+// 32 bits of the value each.
+template <class T>
+struct Record;
+template <>
+struct Record<double> {
     static constexpr int W = 2;
     __device__ static bool ok(const unsigned long long (&w)[2], unsigned tag) {
         return (int)((unsigned)(w[0] >> 32) == tag) & (int)((unsigned)(w[1] >> 32) == tag);
@@ -387,6 +394,20 @@ struct Record {
         st_dev(rec + 1, t | (bits >> 32));
     }
 };
+template <>
+struct Record<float> {
+    static constexpr int W = 1;
+    __device__ static bool ok(const unsigned long long (&w)[2], unsigned tag) {
+        return (unsigned)(w[0] >> 32) == tag;
+    }
+    __device__ static float value(const unsigned long long (&w)[2]) {
+        return __uint_as_float((unsigned)(w[0] & 0xffffffffull));
+    }
+    __device__ static void put(unsigned long long *rec, float v, unsigned tag) {
+        st_dev(rec, ((unsigned long long)tag << 32) | (unsigned long long)__float_as_uint(v));
+    }
+};
+
 // Waits until the upstream tiles (index < 0: none) have completed `need`
 // steps; both flags are polled in one round trip.  Returns false if the
 // bounded spin ran out or another wave aborted.
@@ -411,6 +432,16 @@ __device__ __forceinline__ double wave_sum_fixed(double v) {
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
+// Maximum over the wave; the operands are never NaN.
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const double o = __shfl_xor(v, off, 64);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
 // Tile order of the dispatch: an atomic ticket hands tiles out in
 // dependency order, so every tile's producers were dispatched before it.
 __device__ __forceinline__ int take_tile(PressureBuffers &pb, bool reverse, int &jt, int &kt) {
@@ -472,15 +503,17 @@ __device__ __forceinline__ void tile_urange(const PressureBuffers &pb, const Gri
 }
 
 // The last wave of a sweep launch resets the shared counters for the next
-// launch and finishes the backward sweep's dot product (mode), of which
-// tile_acc is the calling wave's per-lane share.
+// launch and finishes the launch's reduction (mode): the backward sweep's
+// dot product, or the max norm of the residual a forward sweep updated or
+// recomputed.  tile_acc is the calling wave's per-lane share of it.
 __device__ void finish_sweep(PressureBuffers &pb, int mode, double tile_acc, int tile,
                              bool reset_progress, unsigned next_epoch = 0) {
     const int lane = threadIdx.x & 63;
     const int ntiles = pb.sm.ntj * pb.sm.ntk;
     const bool dot = mode == kDotInit || mode == kDotIter;
-    if (dot) {
-        double part = wave_sum_fixed(tile_acc);
+    const bool norm = mode == kAxpyNorm || mode == kTrueResidual;
+    if (dot || norm) {
+        double part = dot ? wave_sum_fixed(tile_acc) : wave_max(tile_acc);
         if (lane == 0) st_dev(&pb.partials[tile], part);
     }
     drain_memory();
@@ -494,6 +527,37 @@ __device__ void finish_sweep(PressureBuffers &pb, int mode, double tile_acc, int
         *pb.ticket = 0;
         pb.sc->counter[0] = 0;
         if (next_epoch) pb.sc->sweep_epoch = next_epoch;
+    }
+    if (norm) {
+        double m = 0.0;
+        for (int q = lane; q < ntiles; q += 64) {
+            const double v = ld_dev(&pb.partials[q]);
+            m = v > m ? v : m;
+        }
+        m = wave_max(m);
+        if (lane == 0) {
+            PcgScalars *sc = pb.sc;
+            if (mode == kAxpyNorm) {
+                // |r32|_inf after the axpy: a true residual is due when it
+                // meets the tolerance, has fallen by delta since the last
+                // one, or the iteration cap is reached.
+                sc->iters += 1;
+                if (m <= sc->tol || m < sc->delta * sc->rmax || sc->iters >= sc->maxiter) sc->refresh = 1;
+                else sc->resid = m;
+            } else {
+                // |b - A x|_inf in FP64 decides convergence.
+                sc->resid = m;
+                sc->refinements += 1;
+                sc->refresh = 0;
+                sc->rmax = m;
+                if (m <= sc->tol) {
+                    sc->converged = 1;
+                    sc->done = 1;
+                } else if (sc->iters >= sc->maxiter) {
+                    sc->done = 1;
+                }
+            }
+        }
     }
     if (dot) {
         // Fixed-order sum of the per-tile partials.
@@ -785,13 +849,15 @@ constexpr int kChunk = 8;  // 8 steps x 8 edge lanes = one record per poller lan
 constexpr int kMailChunks = 4;  // chunks the poller may deliver ahead
 
 // LDS mailbox of a sweep workgroup.
+template <class T>
 struct SweepMailbox {
-    alignas(16) double val[kMailChunks][2][kTile][kChunk];  // [ring][j / k edge][edge lane][step]
+    alignas(16) T val[kMailChunks][2][kTile][kChunk];  // [ring][j / k edge][edge lane][step]
     int ready;     // chunks delivered by the poller
     int consumed;  // chunks read by the compute wave
     int tile;      // the workgroup's ticket
     int skip;      // the solve has finished: nothing to do
     unsigned epoch;  // this launch's record tag
+    int stored;    // chunks whose outputs the compute wave has stored (the dot wave follows it)
 };
 
 __device__ __forceinline__ int lds_acquire(int *p) {
@@ -803,23 +869,45 @@ __device__ __forceinline__ void lds_release(int *p, int v) {
 }
 
 // Four consecutive mailbox values (steps h * 4 .. h * 4 + 3) of one edge lane.
+__device__ __forceinline__ void read_mail(const float *p, int h, float (&e)[kChunk]) {
+    const float4 v = *reinterpret_cast<const float4 *>(p + 4 * h);
+    e[4 * h] = v.x; e[4 * h + 1] = v.y; e[4 * h + 2] = v.z; e[4 * h + 3] = v.w;
+}
 __device__ __forceinline__ void read_mail(const double *p, int h, double (&e)[kChunk]) {
     const double2 v0 = *reinterpret_cast<const double2 *>(p + 4 * h);
     const double2 v1 = *reinterpret_cast<const double2 *>(p + 4 * h + 2);
     e[4 * h] = v0.x; e[4 * h + 1] = v0.y; e[4 * h + 2] = v1.x; e[4 * h + 3] = v1.y;
 }
 
+template <class T>
 struct SweepOps {
-    const double *in;       // forward: r; backward: unused (in place on out)
-    double *out;
-    const double *dotvec;   // backward: vector of the fused dot product, or null
-    const double *inv;      // invdiag
-    const double *c1, *c2, *c3;  // forward: Lzm, Lym, Lxm; backward: Lx, Ly, Lz
+    const T *in;       // forward: r; backward: unused (in place on out)
+    T *out;
+    const T *dotvec;   // backward: vector of the fused dot product, or null
+    const T *inv;      // invdiag
+    const T *c1, *c2, *c3;  // forward: Lzm, Lym, Lxm; backward: Lx, Ly, Lz
 };
 
-// One substitution step, q = (b - c1 x1 - c2 x2 - c3 x3) * inv, in the
-// reference's neighbour order (solveLower / solveLowerTransposeInPlace,
-// pcgsolver.h:191-221), each product and difference rounded as it does.
+template <class T>
+__device__ __forceinline__ T shfl_t(T v, int src) { return __shfl(v, src, 64); }
+
+// Neighbour values within a column tile without the LDS crossbar.  Lane
+// L = a + 8 b of a wave holds column (a, b); a 16-lane DPP row holds b and
+// b + 1.  The j neighbour (L - 1 forward, L + 1 backward) is a row shift by
+// one.  The k neighbour (L - 8 / L + 8) is a rotation by 8 within the row
+// of a register whose other half holds the adjacent row: gfx950's
+// permlane16/32 swaps build the rows shifted by one (forward: rows
+// [., r0, r1, r2]; backward: [r1, r2, r3, .]), and a per-lane select picks,
+// by source half, the lane's own value or the shifted row.  Lanes on the
+// tile's upstream edge take their value from the edge records instead, so
+// the values these produce there are never used.
+// One substitution step, q = (b - c1 x1 - c2 x2 - c3 x3) * inv.
+// ref_step keeps the reference's neighbour order (solveLower /
+// solveLowerTransposeInPlace, pcgsolver.h:191-221) and rounds each product
+// and difference as it does (the FP64 path).  fused_step is for the FP32
+// iteration of the mixed path, which need not match bits: fused terms, taken
+// in the order the values arrive (own previous step, j neighbour, then the k
+// neighbour, whose exchange is longest), for a shorter dependency chain.
 __device__ __forceinline__ double ref_step(double b, double c1, double x1, double c2, double x2, double c3,
                                            double x3, double inv) {
     double q = b;
@@ -828,12 +916,72 @@ __device__ __forceinline__ double ref_step(double b, double c1, double x1, doubl
     q -= c3 * x3;
     return q * inv;
 }
-// The four steps of one slot group of this lane through a buffer view.
+__device__ __forceinline__ float fused_step(float b, float c_own, float own, float c_j, float xj, float c_k,
+                                            float xk, float inv) {
+    float q = __builtin_fmaf(-c_own, own, b);
+    q = __builtin_fmaf(-c_j, xj, q);
+    q = __builtin_fmaf(-c_k, xk, q);
+    return q * inv;
+}
+template <bool FWD>
+__device__ __forceinline__ unsigned lane_j(unsigned v) {
+    return (unsigned)__builtin_amdgcn_mov_dpp((int)v, FWD ? 0x111 : 0x101, 0xf, 0xf, true);
+}
+template <bool FWD>
+__device__ __forceinline__ unsigned lane_k(unsigned v, bool low_half, bool row_sel) {
+    auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // [r0 r0 r2 r2], [r1 r1 r3 r3]
+    unsigned shifted, t;
+    if (FWD) {
+        auto b = __builtin_amdgcn_permlane32_swap(a[1], a[1], false, false);  // [r1 r1 r1 r1]
+        shifted = row_sel ? b[0] : a[0];  // row 2 takes r1
+        t = low_half ? v : shifted;
+    } else {
+        auto c = __builtin_amdgcn_permlane32_swap(a[0], a[0], false, false);  // [r2 r2 r2 r2]
+        shifted = row_sel ? c[1] : a[1];  // row 1 takes r2
+        t = low_half ? shifted : v;
+    }
+    return (unsigned)__builtin_amdgcn_mov_dpp((int)t, 0x128, 0xf, 0xf, true);  // row_ror:8
+}
+template <bool FWD>
+__device__ __forceinline__ float lane_j(float v) {
+    return __builtin_bit_cast(float, lane_j<FWD>(__builtin_bit_cast(unsigned, v)));
+}
+template <bool FWD>
+__device__ __forceinline__ float lane_k(float v, bool low_half, bool row_sel) {
+    return __builtin_bit_cast(float, lane_k<FWD>(__builtin_bit_cast(unsigned, v), low_half, row_sel));
+}
+template <bool FWD>
+__device__ __forceinline__ double lane_j(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = lane_j<FWD>((unsigned)u), hi = lane_j<FWD>((unsigned)(u >> 32));
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+template <bool FWD>
+__device__ __forceinline__ double lane_k(double v, bool low_half, bool row_sel) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = lane_k<FWD>((unsigned)u, low_half, row_sel);
+    const unsigned hi = lane_k<FWD>((unsigned)(u >> 32), low_half, row_sel);
+    return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+
+// The four steps of one slot group of this lane (16 bytes per access for
+// FP32) through a buffer view.
+__device__ __forceinline__ void load_group(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so, float (&e)[4]) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
+    e[0] = __uint_as_float(v.x); e[1] = __uint_as_float(v.y);
+    e[2] = __uint_as_float(v.z); e[3] = __uint_as_float(v.w);
+}
 __device__ __forceinline__ void load_group(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so, double (&e)[4]) {
     const u32x4 v0 = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
     const u32x4 v1 = __builtin_amdgcn_raw_buffer_load_b128(r, vo + 16u, so, 0);
     e[0] = __hiloint2double((int)v0.y, (int)v0.x); e[1] = __hiloint2double((int)v0.w, (int)v0.z);
     e[2] = __hiloint2double((int)v1.y, (int)v1.x); e[3] = __hiloint2double((int)v1.w, (int)v1.z);
+}
+__device__ __forceinline__ void store_group(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so, const float (&e)[4]) {
+    u32x4 v;
+    v.x = __float_as_uint(e[0]); v.y = __float_as_uint(e[1]);
+    v.z = __float_as_uint(e[2]); v.w = __float_as_uint(e[3]);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, vo, so, 0);
 }
 __device__ __forceinline__ void store_group(__amdgpu_buffer_rsrc_t r, unsigned vo, unsigned so, const double (&e)[4]) {
     u32x4 v0, v1;
@@ -850,10 +998,10 @@ __device__ __forceinline__ void store_group(__amdgpu_buffer_rsrc_t r, unsigned v
 // epoch, then delivers the values to the mailbox.  Records outside an
 // upstream tile's march range are never written and read as zero.  On a
 // timeout it raises the abort flag and releases the compute wave.
-template <bool FWD>
-__device__ void sweep_poller(PressureBuffers &pb, SweepMailbox &mb, int tile, int up_j, int up_k, int tb,
+template <class T, bool FWD>
+__device__ void sweep_poller(PressureBuffers &pb, SweepMailbox<T> &mb, int tile, int up_j, int up_k, int tb,
                              int nchunks, int ubj, int uej, int ubk, int uek, int lane, const GroupBits &gb) {
-    constexpr int C = kChunk, RW = Record::W;
+    constexpr int C = kChunk, RW = Record<T>::W;
     const int S = pb.sm.S;
     const unsigned epoch = mb.epoch;
     const int rs = lane >> 3, re = lane & 7;  // step within the chunk, edge lane
@@ -867,7 +1015,7 @@ __device__ void sweep_poller(PressureBuffers &pb, SweepMailbox &mb, int tile, in
     };
     auto fetch = [&](const unsigned long long *q, unsigned long long (&w)[2]) {
         w[0] = ld_dev(q);
-        w[1] = ld_dev(q + 1);
+        w[1] = RW == 2 ? ld_dev(q + 1) : 0ull;
     };
     auto give_up = [&]() {
         if (lane == 0) {
@@ -889,7 +1037,7 @@ __device__ void sweep_poller(PressureBuffers &pb, SweepMailbox &mb, int tile, in
         const bool rows = chunk_has_rows<FWD>(gb, S, tb + ci * C);
         const bool nj = rows & (up_j >= 0) & (uu >= ubj) & (uu < uej);
         const bool nk = rows & (up_k >= 0) & (uu >= ubk) & (uu < uek);
-        double vj = 0.0, vk = 0.0;
+        T vj = T(0), vk = T(0);
         if (__ballot(nj | nk) != 0ull) {
             // The records of the chunk in one round trip per poll.  Every
             // 64th poll also reads the abort flag (one address that every
@@ -901,14 +1049,14 @@ __device__ void sweep_poller(PressureBuffers &pb, SweepMailbox &mb, int tile, in
                 fetch(rec_ptr(rk_tile, rslot_k, uu), rk);
                 const int aborted = (spins & 63u) == 63u ? ld_dev(&pb.sc->abort) : 0;
                 drain_memory();
-                const int bad = ((int)nj & (int)!Record::ok(rj, epoch)) |
-                                ((int)nk & (int)!Record::ok(rk, epoch));
+                const int bad = ((int)nj & (int)!Record<T>::ok(rj, epoch)) |
+                                ((int)nk & (int)!Record<T>::ok(rk, epoch));
                 if (__ballot(bad) == 0ull) break;
                 if (aborted != 0 || ++spins > kSpinLimit) return give_up();
                 __builtin_amdgcn_s_sleep(1);
             }
-            vj = nj ? Record::value(rj) : 0.0;
-            vk = nk ? Record::value(rk) : 0.0;
+            vj = nj ? Record<T>::value(rj) : T(0);
+            vk = nk ? Record<T>::value(rk) : T(0);
         }
         mb.val[slot][0][re][rs] = vj;
         mb.val[slot][1][re][rs] = vk;
@@ -935,21 +1083,175 @@ __device__ __forceinline__ double spmv_slot(const PressureBuffers &pb, double mf
     return s;
 }
 
-constexpr int kSweepDepth = 2;  // chunks whose operands are in flight
-template <int DIR>
-__global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, SweepOps op, int mode) {
-    constexpr int C = kChunk, D = kSweepDepth;
+// The true residual of one tile for the forward sweep that follows it
+// (kTrueResidual): r = b - A x in FP64 at the slots of the tile's active
+// groups, r32 = (float) r, as a separate true-residual pass over the active
+// slot list computes them; returns max |r| over the tile to every thread.
+// The stores are visible to the workgroup's loads after it returns.
+template <int NT>
+__device__ double tile_true_residual(const GridGeom &g, const PressureBuffers &pb, int tile, int tb, int te,
+                                     const GroupBits &gb) {
+    __shared__ double wm[NT / 64];
+    const double mf = pb.sc->mf;  // coupling scale of the assembled system
+    const size_t tile0 = (size_t)tile * (size_t)(pb.sm.S >> 2) * 256;
+    const int g0 = tb >> 2, total = ((te >> 2) - g0) * 256;
+    double mx = 0.0;
+    constexpr int U = 4;
+    for (int e0 = (int)threadIdx.x; e0 < total; e0 += U * NT) {
+        size_t p[U];
+        bool ok[U], in[U];
+        double ax[U], bs[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = e0 + u * NT, gi = g0 + (e >> 8);
+            ok[u] = e < total && gb.test(gi);
+            p[u] = ok[u] ? tile0 + (size_t)gi * 256 + (size_t)(e & 255) : tile0;
+            int i, j, k;
+            in[u] = stencil_cell(g, pb.sm, p[u], i, j, k);
+            ax[u] = spmv_slot(pb, mf, pb.x, p[u], i, j, k);
+            bs[u] = pb.rhs[p[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (!ok[u]) continue;
+            const double r = in[u] ? bs[u] - ax[u] : 0.0;
+            pb.r32[p[u]] = (float)r;
+            const double a = fabs(r);
+            mx = a > mx ? a : mx;
+        }
+    }
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    double m = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) m = wm[w] > m ? wm[w] : m;
+    return m;
+}
+
+// The x half of the axpy that an AX forward sweep does (pcgsolver.h:290),
+// by the workgroup's third wave: x += alpha s32 (FP64) over the tile's
+// active slot groups, four chunks (eight groups) at a time once the compute
+// wave has reached them, so this traffic follows the march instead of
+// meeting the first tiles' polls all at once.  All active groups lie in the
+// march range [tb, te); slots of an active group that are not rows hold
+// s32 = 0 and x = 0, which stays 0.
+template <class T>
+__device__ void sweep_x_wave(const PressureBuffers &pb, SweepMailbox<T> &mb, int tile, int tb, int te, int lane,
+                             const GroupBits &gb) {
+    constexpr int U = 8;
+    const double alpha = pb.sc->alpha;
+    const int S = pb.sm.S;
+    const size_t tile0 = (size_t)tile * (size_t)(S >> 2) * 256;
+    const auto r_x = buffer_view(pb.x + tile0, (unsigned)S * 64u * 8u);
+    const auto r_s = buffer_view(pb.s32 + tile0, (unsigned)S * 64u * 4u);
+    const unsigned vx = (unsigned)lane * 32u, vs = (unsigned)lane * 16u;
+    const int gfirst = tb >> 2, gend = te >> 2;
+    int seen = 0;  // chunks the compute wave is known to have reached
+    for (int g0 = gfirst; g0 < gend; g0 += U) {
+        const int need = (g0 - gfirst) / 2 + 1;  // chunk holding group g0, + 1
+        unsigned spins = 0;
+        while (seen < need) {
+            seen = lds_acquire(&mb.consumed);
+            if (seen >= need) break;
+            if (++spins > kSpinLimit) break;  // the compute wave gave up: finish anyway
+            __builtin_amdgcn_s_sleep(2);
+        }
+        double xv[U][4];
+        float sv[U][4];
+        bool act[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int gi = g0 + u;
+            act[u] = gi < gend && gb.test(gi);
+            load_group(r_x, act[u] ? vx : kOutside, (unsigned)gi * 2048u, xv[u]);
+            load_group(r_s, act[u] ? vs : kOutside, (unsigned)gi * 1024u, sv[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int m = 0; m < 4; m++) xv[u][m] = xv[u][m] + alpha * (double)sv[u][m];
+            store_group(r_x, act[u] ? vx : kOutside, (unsigned)(g0 + u) * 2048u, xv[u]);
+        }
+    }
+}
+
+// The fused z.r of a backward sweep of the mixed path (the dot of
+// pcgsolver.h:296), by the workgroup's third wave: it follows the compute
+// wave, four chunks at a time once their z values are stored, reading z and
+// r for them, and accumulates fma((double) z, (double) r, acc) per lane in
+// march and step order, as the compute wave would.  Chunks without rows
+// hold z = 0 and add nothing.  It finishes the launch (finish_sweep).
+__device__ void sweep_dot_wave(PressureBuffers &pb, SweepMailbox<float> &mb, const SweepOps<float> &op, int tile,
+                               int tb, int nchunks, int lane, const GroupBits &gb, int mode) {
+    constexpr int C = kChunk, K = 4;
+    const int S = pb.sm.S;
+    const size_t tile0 = (size_t)tile * (size_t)(S >> 2) * 256;
+    const unsigned fbytes = (unsigned)S * 64u * 4u;
+    const auto r_z = buffer_view(op.out + tile0, fbytes);
+    const auto r_r = buffer_view(op.dotvec + tile0, fbytes);
+    const unsigned vf = (unsigned)lane * 16u;
+    double acc = 0.0;
+    int seen = 0;
+    for (int c0 = 0; c0 < nchunks; c0 += K) {
+        const int c1 = min(c0 + K, nchunks);
+        unsigned spins = 0;
+        while (seen < c1) {
+            seen = lds_acquire(&mb.stored);
+            if (seen >= c1) break;
+            if (++spins > kSpinLimit) break;  // the compute wave gave up: finish anyway
+            __builtin_amdgcn_s_sleep(1);
+        }
+        float zv[K][2][4], rv[K][2][4];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int gl = chunk_group<false>(S, tb + (c0 + k) * C);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const bool act = c0 + k < c1 && gb.test(gl + h);
+                const unsigned so = (unsigned)(gl + h) * 1024u;
+                load_group(r_z, act ? vf : kOutside, so, zv[k][h]);
+                load_group(r_r, act ? vf : kOutside, so, rv[k][h]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++)
+#pragma unroll
+            for (int s = 0; s < C; s++) {
+                // Step s of a backward chunk is element (7 - s) % 4 of group (7 - s) / 4.
+                const int h = (7 - s) >> 2, m = (7 - s) & 3;
+                acc = __builtin_fma((double)zv[k][h][m], (double)rv[k][h][m], acc);
+            }
+    }
+    finish_sweep(pb, mode, acc, tile, false, mb.epoch + 1);
+}
+
+// AX (FP32 forward sweep of the mixed path only): the sweep also does the
+// iteration's axpy (pcgsolver.h:289-290).  The compute wave reads
+// r32 + (-alpha) q32 in place of r32 (off the step's dependency chain),
+// stores it back to r32 and takes its max norm; the third wave updates x
+// (sweep_x_wave).  Each value is rounded as a separate axpy pass would
+// round it, and the max is order-independent.
+// AUX (FP32 sweeps of the mixed path): a third wave helps, the axpy's x
+// update on the forward sweep (AX), the z.r dot on the backward one (DW).
+template <class T, int DIR, int D, bool AUX = false>
+__global__ __launch_bounds__(256) void k_sweep(GridGeom g, PressureBuffers pb, SweepOps<T> op,
+                                                          int mode) {
+    constexpr int C = kChunk;
     constexpr bool FWD = DIR == kForward;
-    constexpr int NV = FWD ? 5 : 6;
-    constexpr int RW = Record::W;
-    __shared__ SweepMailbox mb;
+    static_assert(!AUX || sizeof(T) == 4, "helper waves serve the FP32 sweeps only");
+    constexpr bool AX = AUX && FWD, DW = AUX && !FWD;
+    constexpr int NV = FWD ? (AX ? 6 : 5) : (DW ? 5 : 6);
+    constexpr int RW = Record<T>::W;
+    __shared__ SweepMailbox<T> mb;
     if (threadIdx.x == 0) {
-        const int skip = ld_dev(&pb.sc->done) != 0;
+        const int skip = ld_dev(&pb.sc->done) != 0 || (mode == kTrueResidual && ld_dev(&pb.sc->refresh) == 0);
         mb.skip = skip;
         mb.tile = skip ? 0 : (int)atomicAdd(pb.ticket, 1u);
         mb.epoch = ld_dev(&pb.sc->sweep_epoch);
         mb.ready = 0;
         mb.consumed = 0;
+        mb.stored = 0;
     }
     __syncthreads();
     if (mb.skip) return;
@@ -967,11 +1269,27 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
     if (up_k >= 0) tile_urange(pb, g, up_k, !FWD, ubk, uek);
     const int nchunks = te > tb ? (te - tb) / C : 0;
     const GroupBits gb = tile_group_bits(pb, tile);
+    // kTrueResidual: the tile's true residual first (every wave), then the sweep over it.
+    double tres_max = 0.0;
+    if constexpr (FWD && !AX && sizeof(T) == 4) {
+        if (mode == kTrueResidual) {
+            tres_max = tile_true_residual<256>(g, pb, tile, tb, te, gb);
+            if (wave >= 2) return;  // those waves only help with the residual
+        }
+    }
     if (wave == 1)
-        return sweep_poller<FWD>(pb, mb, tile, up_j, up_k, tb, nchunks, ubj, uej, ubk, uek, lane, gb);
+        return sweep_poller<T, FWD>(pb, mb, tile, up_j, up_k, tb, nchunks, ubj, uej, ubk, uek, lane, gb);
+    if constexpr (AX)
+        if (wave == 2) return sweep_x_wave(pb, mb, tile, tb, te, lane, gb);
+    if constexpr (DW)
+        if (wave == 2) return sweep_dot_wave(pb, mb, op, tile, tb, nchunks, lane, gb, mode);
 
     const int src_j = (FWD ? lane - 1 : lane + 1) & 63;  // neighbour lane along j
     const int src_k = (FWD ? lane - 8 : lane + 8) & 63;  // neighbour lane along k
+    // Lane position in its 16-lane DPP row and the row that takes the
+    // permlane32 result (lane_k).
+    const bool low_half = (lane & 15) < 8;
+    const bool row_sel = (lane >> 4) == (FWD ? 2 : 1);
     const bool edge_j = FWD ? a == 0 : a == 7;            // reads the upstream j tile
     const bool edge_k = FWD ? b == 0 : b == 7;
     // Edge cells (read by the downstream neighbours) publish one record per
@@ -981,19 +1299,20 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
     const int pub_slot = a == aj ? b : 8 + a;
     const unsigned epoch = mb.epoch;
     const size_t grp0 = (size_t)tile * (size_t)(S >> 2);
-    const bool dot = !FWD && mode != kDotNone;
+    const bool dot = !FWD && !DW && mode != kDotNone;
     // Without a dot product the backward sweep still streams a vector (its
     // own output) so the hot loop has no data-dependent branches.
-    const double *dotsrc = dot ? op.dotvec : op.out;
+    const T *dotsrc = dot ? op.dotvec : op.out;
+
 
     auto active = [&](int gi) -> bool { return gb.test(gi); };
     // Buffer views of the tile's slots in each array (group gi of the tile
-    // at byte gi * 256 * sizeof(double), this lane's four slots at lane * 4 *
-    // sizeof(double) within it).  A group without rows is read and written
+    // at byte gi * 256 * sizeof(T), this lane's four slots at lane * 4 *
+    // sizeof(T) within it).  A group without rows is read and written
     // through the offset kOutside: it reads as zeros and its stores (zeros)
     // are dropped.  The group offset is scalar, so addressing a group costs
     // one select for all arrays.
-    const unsigned tile_bytes = (unsigned)S * 64u * (unsigned)sizeof(double);
+    const unsigned tile_bytes = (unsigned)S * 64u * (unsigned)sizeof(T);
     const size_t tile0 = grp0 * 256;
     const auto r_b = buffer_view((FWD ? op.in : op.out) + tile0, tile_bytes);
     const auto r_c1 = buffer_view(op.c1 + tile0, tile_bytes);
@@ -1002,7 +1321,12 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
     const auto r_inv = buffer_view(op.inv + tile0, tile_bytes);
     const auto r_dot = buffer_view(dotsrc + tile0, tile_bytes);
     const auto r_out = buffer_view(op.out + tile0, tile_bytes);
-    const unsigned vlane = (unsigned)lane * 4u * (unsigned)sizeof(double);
+    // AX: the SpMV result q32 read beside r32, and r32 written back.
+    const auto r_q = buffer_view((AX ? (const T *)pb.q32 : op.c1) + tile0, tile_bytes);
+    const auto r_rw = buffer_view((AX ? (const T *)pb.r32 : op.out) + tile0, tile_bytes);
+    const T naf = AX ? T(-pb.sc->alpha_f) : T(0);
+    T rmax = T(0);  // AX: max |r| over the tile's updated residual
+    const unsigned vlane = (unsigned)lane * 4u * (unsigned)sizeof(T);
     // Every lane stores a record each step (no branch around the store):
     // lanes that publish nothing write slot 8 + aj, which the corner lane
     // leaves unused and no consumer reads.
@@ -1015,20 +1339,21 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
         // Step s of a chunk is element m of group h: forward s = 4h + m,
         // backward s = 7 - (4h + m).
         // act[h] keeps each group's mask bit for the store of the same chunk.
-        auto load_chunk = [&](int u0, double (&v)[NV][C], bool (&act)[2]) {
+        auto load_chunk = [&](int u0, T (&v)[NV][C], bool (&act)[2]) {
             const int gl = chunk_group(u0);
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 act[h] = active(gl + h);
                 const unsigned vo = act[h] ? vlane : kOutside;
-                const unsigned so = (unsigned)(gl + h) * 256u * (unsigned)sizeof(double);
-                double e[NV][4];
+                const unsigned so = (unsigned)(gl + h) * 256u * (unsigned)sizeof(T);
+                T e[NV][4];
                 load_group(r_b, vo, so, e[0]);
                 load_group(r_c1, vo, so, e[1]);
                 load_group(r_c2, vo, so, e[2]);
                 load_group(r_c3, vo, so, e[3]);
                 load_group(r_inv, vo, so, e[4]);
-                if (!FWD) load_group(r_dot, vo, so, e[NV - 1]);
+                if (!FWD && !DW) load_group(r_dot, vo, so, e[NV - 1]);
+                if (AX) load_group(r_q, vo, so, e[NV - 1]);
 #pragma unroll
                 for (int m = 0; m < 4; m++) {
                     const int s = FWD ? 4 * h + m : 7 - (4 * h + m);
@@ -1037,20 +1362,20 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
                 }
             }
         };
-        auto store_chunk = [&](__amdgpu_buffer_rsrc_t dst, int u0, const double (&qv)[C], const bool (&act)[2]) {
+        auto store_chunk = [&](__amdgpu_buffer_rsrc_t dst, int u0, const T (&qv)[C], const bool (&act)[2]) {
             const int gl = chunk_group(u0);
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                double e[4];
+                T e[4];
 #pragma unroll
                 for (int m = 0; m < 4; m++) e[m] = qv[FWD ? 4 * h + m : 7 - (4 * h + m)];
                 // The output of a group without rows stays zero: its values
                 // (all zero) are dropped.
-                store_group(dst, act[h] ? vlane : kOutside, (unsigned)(gl + h) * 256u * (unsigned)sizeof(double), e);
+                store_group(dst, act[h] ? vlane : kOutside, (unsigned)(gl + h) * 256u * (unsigned)sizeof(T), e);
             }
         };
         // The operands of the first D chunks.
-        double buf[D][NV][C];
+        T buf[D][NV][C];
         bool actr[D][2];
         const int last = te - C;  // last chunk; loads past the end repeat it
 #pragma unroll
@@ -1059,7 +1384,7 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
             load_chunk(uf < last ? uf : last, buf[d], actr[d]);
             __builtin_amdgcn_sched_barrier(0);
         }
-        double cur = 0.0;
+        T cur = T(0);
         int rdy = 0;  // chunks known to be in the mailbox
         // An LDS poll while the poller has not delivered `need` chunks.
         auto wait_mail = [&](int need) {
@@ -1091,15 +1416,15 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
                     // Its outputs are zero already.
                     if (lane == 0) lds_release(&mb.consumed, ci + 1);
 #pragma unroll
-                    for (int s = 0; s < C; s++) Record::put(recp + (size_t)s * kRecSlots * RW, 0.0, epoch);
-                    cur = 0.0;
+                    for (int s = 0; s < C; s++) Record<T>::put(recp + (size_t)s * kRecSlots * RW, T(0), epoch);
+                    cur = T(0);
                 } else {
-                    const double *const mj = mb.val[ci % kMailChunks][0][b];
-                    const double *const mk = mb.val[ci % kMailChunks][1][a];
+                    const T *const mj = mb.val[ci % kMailChunks][0][b];
+                    const T *const mk = mb.val[ci % kMailChunks][1][a];
                     // The chunk's upstream values: an LDS poll while the poller
                     // has not delivered them.
                     wait_mail(ci + 1);
-                    double evj[C], evk[C];
+                    T evj[C], evk[C];
                     read_mail(mj, 0, evj);
                     read_mail(mk, 0, evk);
                     read_mail(mj, 1, evj);
@@ -1107,22 +1432,45 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
                     // The release waits for the reads above, so the poller may
                     // then reuse the ring slot.
                     if (lane == 0) lds_release(&mb.consumed, ci + 1);
-                    const double(&v)[NV][C] = buf[d];
-                    double qv[C];
-#pragma unroll
+                    const T(&v)[NV][C] = buf[d];
+                    T qv[C], bv[C];
+    #pragma unroll
                     for (int s = 0; s < C; s++) {
                         // Values produced one step earlier by the neighbouring lanes.
-                        const double nj_cur = __shfl(cur, src_j, 64), nk_cur = __shfl(cur, src_k, 64);
-                        const double qy = edge_j ? evj[s] : nj_cur;
-                        const double qz = edge_k ? evk[s] : nk_cur;
+                        // FP32: DPP / permlane exchange; FP64: the LDS crossbar
+                        // (two dwords per value make the permlane route longer).
+                        T nj_cur, nk_cur;
+                        if constexpr (sizeof(T) == 4) {
+                            nj_cur = lane_j<FWD>(cur);
+                            nk_cur = lane_k<FWD>(cur, low_half, row_sel);
+                        } else {
+                            nj_cur = shfl_t(cur, src_j);
+                            nk_cur = shfl_t(cur, src_k);
+                        }
+                        const T qy = edge_j ? evj[s] : nj_cur;
+                        const T qz = edge_k ? evk[s] : nk_cur;
+                        // AX: the updated residual r + (-alpha) q, off the
+                        // step's dependency chain; fmaxf(m, |r|) is the
+                        // compare-and-keep maximum here (m is never NaN).
+                        T bs = v[0][s];
+                        if constexpr (AX) {
+                            bs = v[0][s] + naf * v[NV - 1][s];
+                            bv[s] = bs;
+                            rmax = fmaxf(rmax, fabsf(bs));
+                        }
                         // c1..c3 multiply the -z, -y, -x neighbours (forward) or
                         // the +x, +y, +z ones (backward).
-                        const double q =
-                            FWD ? ref_step(v[0][s], v[1][s], qz, v[2][s], qy, v[3][s], cur, v[4][s])
-                                : ref_step(v[0][s], v[1][s], cur, v[2][s], qy, v[3][s], qz, v[4][s]);
-                        if (!FWD) dot_acc = __builtin_fma(q, v[NV - 1][s], dot_acc);
+                        T q;
+                        if constexpr (sizeof(T) == 8) {
+                            q = FWD ? ref_step(v[0][s], v[1][s], qz, v[2][s], qy, v[3][s], cur, v[4][s])
+                                    : ref_step(v[0][s], v[1][s], cur, v[2][s], qy, v[3][s], qz, v[4][s]);
+                        } else {
+                            q = FWD ? fused_step(bs, v[3][s], cur, v[2][s], qy, v[1][s], qz, v[4][s])
+                                    : fused_step(bs, v[1][s], cur, v[2][s], qy, v[3][s], qz, v[4][s]);
+                        }
+                        if (!FWD && !DW) dot_acc = __builtin_fma((double)q, (double)v[NV - 1][s], dot_acc);
                         qv[s] = q;
-                        Record::put(recp + (size_t)s * kRecSlots * RW, q, epoch);
+                        Record<T>::put(recp + (size_t)s * kRecSlots * RW, q, epoch);
                         // Keep each step's record where it is computed: no
                         // memory operation is scheduled across this point (ALU
                         // and LDS instructions may be).
@@ -1131,14 +1479,21 @@ __global__ __launch_bounds__(128) void k_sweep(GridGeom g, PressureBuffers pb, S
                         cur = q;
                     }
                     store_chunk(r_out, uc, qv, actr[d]);
+                    if constexpr (AX) store_chunk(r_rw, uc, bv, actr[d]);
                 }
+                // The dot wave may read the chunk's z: the release orders the
+                // stores above before the count (one CU, in issue order).
+                if (DW && lane == 0) lds_release(&mb.stored, ci + 1);
                 const int uf = uc + D * C;
                 load_chunk(uf < last ? uf : last, buf[d], actr[d]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
-    finish_sweep(pb, dot ? mode : kDotNone, dot_acc, tile, false, epoch + 1);
+    if constexpr (DW) return;  // the dot wave finishes the launch
+    const int fin = FWD ? (AX ? kAxpyNorm : (mode == kTrueResidual ? kTrueResidual : kDotNone))
+                        : (dot ? mode : kDotNone);
+    finish_sweep(pb, fin, AX ? (double)rmax : (FWD ? tres_max : dot_acc), tile, false, epoch + 1);
 }
 
 // Launches a kernel on s.  With a start event the dispatch itself records
@@ -1152,7 +1507,20 @@ static hipError_t launch_on(void (*kern)(KArgs...), dim3 grid, dim3 block, hipSt
     return hipGetLastError();
 }
 
-static hipError_t launch_sweep(int dir, const GridGeom &g, PressureBuffers &pb, SweepOps op,
+// Register ring depth per value type: FP32 operands are half the size.
+template <class T>
+struct SweepDepth;
+template <>
+struct SweepDepth<double> {
+    static constexpr int D = 2;
+};
+template <>
+struct SweepDepth<float> {
+    static constexpr int D = 4;
+};
+
+template <class T>
+static hipError_t launch_sweep(int dir, const GridGeom &g, PressureBuffers &pb, SweepOps<T> op,
                                int mode, hipStream_t s, const KernelTiming &kt = KernelTiming{}) {
     // A fresh epoch per launch (the device's sweep_epoch, advanced by each
     // launch's last tile); records of older launches never match it.  The
@@ -1167,16 +1535,38 @@ static hipError_t launch_sweep(int dir, const GridGeom &g, PressureBuffers &pb, 
         pb.epoch = 1;
     }
     int ntiles = pb.sm.ntj * pb.sm.ntk;
-    if (dir == kForward) return launch_on(k_sweep<kForward>, dim3(ntiles), dim3(128), s, kt, g, pb, op, mode);
-    return launch_on(k_sweep<kBackward>, dim3(ntiles), dim3(128), s, kt, g, pb, op, mode);
+    constexpr int D = SweepDepth<T>::D;
+    if (mode == kAxpyNorm) {
+        if constexpr (sizeof(T) == 4) {
+            if (dir == kForward) return launch_on(k_sweep<T, kForward, D, true>, ntiles, 192, s, kt, g, pb, op, mode);
+        }
+        return hipErrorInvalidValue;
+    }
+    // The forward sweep over a fresh true residual has four waves for the
+    // residual; two of them then leave.
+    if (dir == kForward)
+        return launch_on(k_sweep<T, kForward, D>, ntiles, mode == kTrueResidual ? 256 : 128, s, kt, g, pb, op,
+                         mode);
+    // The FP32 backward sweep's z.r is taken by a third wave.
+    if constexpr (sizeof(T) == 4)
+        if (mode == kDotInit || mode == kDotIter)
+            return launch_on(k_sweep<T, kBackward, D, true>, ntiles, 192, s, kt, g, pb, op, mode);
+    return launch_on(k_sweep<T, kBackward, D>, ntiles, 128, s, kt, g, pb, op, mode);
 }
 
-static SweepOps fwd_ops(PressureBuffers &pb, const double *r, double *z) {
-    return SweepOps{r, z, nullptr, pb.invdiag, pb.Lzm, pb.Lym, pb.Lxm};
+static SweepOps<double> fwd_ops64(PressureBuffers &pb, const double *r, double *z) {
+    return SweepOps<double>{r, z, nullptr, pb.invdiag, pb.Lzm, pb.Lym, pb.Lxm};
 }
-static SweepOps bwd_ops(PressureBuffers &pb, double *z, const double *dotvec) {
-    return SweepOps{nullptr, z, dotvec, pb.invdiag, pb.Lx, pb.Ly, pb.Lz};
+static SweepOps<double> bwd_ops64(PressureBuffers &pb, double *z, const double *dotvec) {
+    return SweepOps<double>{nullptr, z, dotvec, pb.invdiag, pb.Lx, pb.Ly, pb.Lz};
 }
+static SweepOps<float> fwd_ops32(PressureBuffers &pb) {
+    return SweepOps<float>{pb.r32, pb.z32, nullptr, pb.invdiag32, pb.Lzm32, pb.Lym32, pb.Lxm32};
+}
+static SweepOps<float> bwd_ops32(PressureBuffers &pb) {
+    return SweepOps<float>{nullptr, pb.z32, pb.r32, pb.invdiag32, pb.Lx32, pb.Ly32, pb.Lz32};
+}
+
 hipError_t launch_mic0_factor(const GridGeom &g, const float *liquid, PressureBuffers &pb,
                               hipStream_t s) {
     size_t n = pb.sm.count();
@@ -1194,9 +1584,9 @@ hipError_t launch_mic0_factor(const GridGeom &g, const float *liquid, PressureBu
 
 hipError_t launch_precond_apply(const GridGeom &g, PressureBuffers &pb, const double *r,
                                 double *z, hipStream_t s) {
-    hipError_t e = launch_sweep(kForward, g, pb, fwd_ops(pb, r, z), kDotNone, s);
+    hipError_t e = launch_sweep(kForward, g, pb, fwd_ops64(pb, r, z), kDotNone, s);
     if (e != hipSuccess) return e;
-    return launch_sweep(kBackward, g, pb, bwd_ops(pb, z, nullptr), kDotNone, s);
+    return launch_sweep(kBackward, g, pb, bwd_ops64(pb, z, nullptr), kDotNone, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1558,31 +1948,236 @@ hipError_t launch_pressure_reset(PressureBuffers &pb, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, PressureBuffers &pb, hipStream_t s) {
+// ---------------------------------------------------------------------------
+// Mixed precision: FP32 inner iteration (FP32 vectors r, z, s and factor;
+// the SpMV reads the FP64 matrix), FP64 dots, FP64 x, and a true
+// residual r = b - A x in FP64 that replaces the FP32 recursive residual
+// whenever the latter has fallen by `delta` since the last replacement or
+// reached the tolerance ("reliable update").  Convergence is declared only
+// on the FP64 true residual, |b - A x|_inf <= tol |b|_inf.
+// ---------------------------------------------------------------------------
+
+// FP32 copy of the (FP64-computed) factor.
+// The FP32 factor of the slots the sweeps read.
+__global__ __launch_bounds__(kRedThreads) void k_to_f32(PressureBuffers pb) {
+    for_swept_slots(pb, [&](size_t p) {
+        pb.invdiag32[p] = (float)pb.invdiag[p];
+        pb.Lx32[p] = (float)pb.Lx[p];
+        pb.Ly32[p] = (float)pb.Ly[p];
+        pb.Lz32[p] = (float)pb.Lz[p];
+        pb.Lxm32[p] = (float)pb.Lxm[p];
+        pb.Lym32[p] = (float)pb.Lym[p];
+        pb.Lzm32[p] = (float)pb.Lzm[p];
+    });
+}
+
+__global__ void k_pcg_init_vectors32(PressureBuffers pb) {
+    size_t n = pb.sm.count();
+    for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
+         p += (size_t)gridDim.x * blockDim.x) {
+        pb.x[p] = 0.0;
+        pb.r32[p] = (float)pb.rhs[p];
+        pb.z32[p] = 0.0f;
+        pb.s32[p] = 0.0f;
+    }
+}
+
+// q = A s for the FP32 iteration: the FP64 matrix entries (an FP32 copy's
+// rounding costs about 9 % more iterations on the workloads here: 126
+// against 115), rebuilt from the FP32 face weights, FP32 s, FP64 sums,
+// rounded once.
+// The new direction s = z + beta s of the previous iteration
+// (pcgsolver.h:300-302), formed where the SpMV reads it.
+struct NextDirection {
+    const float *__restrict__ z, *__restrict__ s;
+    float beta;
+    __device__ __forceinline__ float operator[](size_t q) const { return z[q] + beta * s[q]; }
+};
+struct SameDirection {
+    const float *__restrict__ s;
+    __device__ __forceinline__ float operator[](size_t q) const { return s[q]; }
+};
+
+template <class Dir>
+__device__ __forceinline__ double spmv_slot_dir(const PressureBuffers &pb, double mf, const Dir &x, size_t p,
+                                                int i, int j, int k) {
+    const SlotMap &sm = pb.sm;
+    const unsigned pzm = sm.slot32(i, j, k - 1), pym = sm.slot32(i, j - 1, k), pxm = sm.slot32(i - 1, j, k);
+    const unsigned pxp = sm.slot32(i + 1, j, k), pyp = sm.slot32(i, j + 1, k), pzp = sm.slot32(i, j, k + 1);
+    double s = 0.0;
+    s += coupling(pb.wz[pzm], mf) * (double)x[pzm];
+    s += coupling(pb.wy[pym], mf) * (double)x[pym];
+    s += coupling(pb.wx[pxm], mf) * (double)x[pxm];
+    s += pb.diag[p] * (double)x[p];
+    s += coupling(pb.wx[p], mf) * (double)x[pxp];
+    s += coupling(pb.wy[p], mf) * (double)x[pyp];
+    s += coupling(pb.wz[p], mf) * (double)x[pzp];
+    return s;
+}
+
+// s32b = z32 + beta s32 (or s32 as it is), q32 = A s32b and alpha = rho /
+// (s . q) with an FP64 dot.  z32 and s32 are only read, so the stencil
+// reads race with no write.
+template <class Dir>
+__device__ __forceinline__ double spmv_dot32_body(const GridGeom &g, const PressureBuffers &pb,
+                                                  const Dir &dir) {
+    double acc = 0.0;
+    const ListRange lr = xcd_list(*pb.active_count);
+    const double mf = pb.sc->mf;  // coupling scale of the assembled system
+    constexpr int U = 2;
+    for (int e0 = lr.begin; e0 < lr.end; e0 += U * lr.step) {
+        size_t p[U];
+        bool ok[U], in[U];
+        float zc[U], sp[U];
+        list_slots<U>(pb, lr, e0, p, ok);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            int i, j, k;
+            in[u] = stencil_cell(g, pb.sm, p[u], i, j, k);
+            zc[u] = (float)spmv_slot_dir(pb, mf, dir, p[u], i, j, k);
+            sp[u] = dir[p[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (!ok[u]) continue;  // uniform
+            const float q = in[u] ? zc[u] : 0.0f;
+            pb.q32[p[u]] = q;
+            pb.s32b[p[u]] = sp[u];
+            acc += (double)sp[u] * (double)q;
+        }
+    }
+    return acc;
+}
+
+__global__ __launch_bounds__(kRedThreads) void k_spmv_dot32(GridGeom g, PressureBuffers pb) {
+    __shared__ double sh[kRedThreads / 64];
+    if (pb.sc->done) return;
+    double acc = pb.s_plain ? spmv_dot32_body(g, pb, SameDirection{pb.s32})
+                            : spmv_dot32_body(g, pb, NextDirection{pb.z32, pb.s32, pb.sc->beta_f});
+    double bs = block_reduce<0>(acc, sh);
+    if (threadIdx.x == 0) st_dev(&pb.partials[blockIdx.x], bs);
+    if (!last_block(&pb.sc->counter[1], pb.sc->group_counter[0])) return;
+    double tot = 0.0;
+    for (int q = threadIdx.x; q < (int)gridDim.x; q += kRedThreads) tot += ld_dev(&pb.partials[q]);
+    tot = block_reduce<0>(tot, sh);
+    if (threadIdx.x == 0) {
+        PcgScalars *sc = pb.sc;
+        sc->sz = tot;
+        double alpha = sc->rho / tot;
+        sc->alpha = alpha;
+        sc->alpha_f = (float)alpha;
+        sc->counter[1] = 0;
+    }
+}
+
+// s32 = z32: a solve's first direction (pcgsolver.h:279).  Later
+// directions are formed by the SpMV that reads them.
+__global__ __launch_bounds__(kRedThreads) void k_first_direction32(PressureBuffers pb) {
+    if (pb.sc->done) return;
+    const ListRange lr = xcd_list(*pb.active_count);
+    constexpr int U = 4;
+    for (int e0 = lr.begin; e0 < lr.end; e0 += U * lr.step) {
+        size_t p[U];
+        bool ok[U];
+        float zs[U];
+        list_slots<U>(pb, lr, e0, p, ok);
+#pragma unroll
+        for (int u = 0; u < U; u++) zs[u] = pb.z32[p[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (!ok[u]) continue;  // uniform
+            pb.s32[p[u]] = zs[u];
+        }
+    }
+}
+
+__global__ void k_mixed_init_scalars(PressureBuffers pb) {
+    PcgScalars *sc = pb.sc;
+    sc->rmax = sc->bnorm;
+    sc->delta = 1e-2;
+    sc->refresh = 0;
+    sc->refinements = 0;
+}
+
+hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, bool mixed,
+                           PressureBuffers &pb, hipStream_t s) {
+    if (mixed) {
+        k_to_f32<<<kRedBlocks, kRedThreads, 0, s>>>(pb);
+        k_pcg_init_vectors32<<<kRedBlocks, kRedThreads, 0, s>>>(pb);
+        k_pcg_init_scalars<<<1, 1, 0, s>>>(pb, tolf, maxiter);
+        k_mixed_init_scalars<<<1, 1, 0, s>>>(pb);
+        hipError_t e = launch_sweep(kForward, g, pb, fwd_ops32(pb), kDotNone, s);
+        if (e != hipSuccess) return e;
+        e = launch_sweep(kBackward, g, pb, bwd_ops32(pb), kDotInit, s);
+        if (e != hipSuccess) return e;
+        k_first_direction32<<<kRedBlocks, kRedThreads, 0, s>>>(pb);
+        pb.s_plain = 1;  // the first SpMV takes s = z as it is
+        return hipGetLastError();
+    }
     k_pcg_init_vectors<<<kRedBlocks, kRedThreads, 0, s>>>(g, pb);
     k_pcg_init_scalars<<<1, 1, 0, s>>>(pb, tolf, maxiter);
     // z = M^-1 r, rho = z . r, s = z (pcgsolver.h:270-279).
-    hipError_t e = launch_sweep(kForward, g, pb, fwd_ops(pb, pb.r, pb.z), kDotNone, s);
+    hipError_t e = launch_sweep(kForward, g, pb, fwd_ops64(pb, pb.r, pb.z), kDotNone, s);
     if (e != hipSuccess) return e;
-    e = launch_sweep(kBackward, g, pb, bwd_ops(pb, pb.z, pb.r), kDotInit, s);
+    e = launch_sweep(kBackward, g, pb, bwd_ops64(pb, pb.z, pb.r), kDotInit, s);
     if (e != hipSuccess) return e;
     k_update_s<<<kRedBlocks, kRedThreads, 0, s>>>(g, pb, 1);
     return hipGetLastError();
 }
 
-// One iteration; the pieces with a start event in kt are timed.
-hipError_t launch_pcg_iteration(const GridGeom &g, PressureBuffers &pb, hipStream_t s,
-                                const KernelTiming (&kt)[kPcgPieces]) {
+// Mixed precision folds the axpy into the forward sweep and the direction
+// update into the next SpMV; the FP64 path has no true-residual step.
+bool pcg_piece_used(int piece, bool mixed) {
+    if (mixed) return piece != kPcgUpdate && piece != kPcgAxpy;
+    return piece != kPcgResidual;
+}
+
+static hipError_t launch_pcg_piece(int piece, const GridGeom &g, bool mixed, PressureBuffers &pb,
+                                   hipStream_t s, const KernelTiming &kt) {
     const dim3 rg(kRedBlocks), rb(kRedThreads);
-    hipError_t e = launch_on(k_spmv_dot, rg, rb, s, kt[kPcgSpmv], g, pb);
-    if (e != hipSuccess) return e;
-    e = launch_on(k_axpy_norm, dim3(kAxpyBlocks), rb, s, kt[kPcgAxpy], g, pb);
-    if (e != hipSuccess) return e;
-    e = launch_sweep(kForward, g, pb, fwd_ops(pb, pb.r, pb.z), kDotNone, s, kt[kPcgForward]);
-    if (e != hipSuccess) return e;
-    e = launch_sweep(kBackward, g, pb, bwd_ops(pb, pb.z, pb.r), kDotIter, s, kt[kPcgBackward]);
-    if (e != hipSuccess) return e;
-    return launch_on(k_update_s, rg, rb, s, kt[kPcgUpdate], g, pb, 0);
+    if (mixed) {
+        switch (piece) {
+            case kPcgSpmv: {
+                hipError_t e = launch_on(k_spmv_dot32, rg, rb, s, kt, g, pb);
+                // The launch took s32 -> s32b by value; the new direction is s32 from here on.
+                pb.swap_directions();
+                pb.s_plain = 0;
+                return e;
+            }
+            // The forward sweep does the axpy; when its residual norm calls
+            // for a true residual, the sweep is redone over that residual.
+            case kPcgForward: return launch_sweep(kForward, g, pb, fwd_ops32(pb), kAxpyNorm, s, kt);
+            case kPcgResidual: return launch_sweep(kForward, g, pb, fwd_ops32(pb), kTrueResidual, s, kt);
+            case kPcgBackward: return launch_sweep(kBackward, g, pb, bwd_ops32(pb), kDotIter, s, kt);
+            // kPcgAxpy and kPcgUpdate are folded into the forward sweep and
+            // the SpMV.
+            default: return hipErrorInvalidValue;
+        }
+    }
+    switch (piece) {
+        case kPcgSpmv: return launch_on(k_spmv_dot, rg, rb, s, kt, g, pb);
+        case kPcgAxpy: return launch_on(k_axpy_norm, dim3(kAxpyBlocks), rb, s, kt, g, pb);
+        case kPcgForward: return launch_sweep(kForward, g, pb, fwd_ops64(pb, pb.r, pb.z), kDotNone, s, kt);
+        case kPcgBackward: return launch_sweep(kBackward, g, pb, bwd_ops64(pb, pb.z, pb.r), kDotIter, s, kt);
+        case kPcgUpdate: return launch_on(k_update_s, rg, rb, s, kt, g, pb, 0);
+        case kPcgResidual: return hipSuccess;
+        default: return hipErrorInvalidValue;
+    }
+}
+
+// Execution order of the pieces within one iteration.
+static const int kPieceOrder[kPcgPieces] = {kPcgSpmv,     kPcgAxpy,     kPcgForward,
+                                            kPcgResidual, kPcgBackward, kPcgUpdate};
+
+hipError_t launch_pcg_iteration(const GridGeom &g, bool mixed, PressureBuffers &pb, hipStream_t s,
+                                const KernelTiming (&kt)[kPcgPieces]) {
+    for (int q = 0; q < kPcgPieces; q++) {
+        int piece = kPieceOrder[q];
+        if (!pcg_piece_used(piece, mixed)) continue;
+        hipError_t e = launch_pcg_piece(piece, g, mixed, pb, s, kt[piece]);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 __global__ void k_spmv_plain(GridGeom g, PressureBuffers pb, const double *__restrict__ x,
@@ -1600,6 +2195,36 @@ __global__ void k_spmv_plain(GridGeom g, PressureBuffers pb, const double *__res
 hipError_t launch_spmv(const GridGeom &g, PressureBuffers &pb, const double *x, double *y,
                        hipStream_t s) {
     k_spmv_plain<<<kRedBlocks, kRedThreads, 0, s>>>(g, pb, x, y);
+    return hipGetLastError();
+}
+
+__global__ void k_row_flags(GridGeom g, const float *__restrict__ liquid, int *flags) {
+    const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= (size_t)g.I * g.J * g.K) return;
+    int i, j, k;
+    unflatten3(c, g.I, g.J, i, j, k);
+    flags[c] = is_row_cell(g, liquid, i, j, k) ? 1 : 0;
+}
+__global__ void k_gather_rows(GridGeom g, const int *__restrict__ flags, const int *__restrict__ pos,
+                              const double *__restrict__ p, PressureIndex at, double *rows, int *count) {
+    const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x, n = (size_t)g.I * g.J * g.K;
+    if (c >= n) return;
+    if (c == n - 1) *count = pos[c] + flags[c];
+    if (!flags[c]) return;
+    int i, j, k;
+    unflatten3(c, g.I, g.J, i, j, k);
+    rows[pos[c]] = p ? p[at(i, j, k)] : 0.0;
+}
+
+hipError_t launch_gather_rows(const GridGeom &g, const float *liquid, const double *p, const PressureIndex &at,
+                              int *flags, int *pos, int *scan_tmp, double *rows, int *count, hipStream_t s) {
+    const size_t n = (size_t)g.I * g.J * g.K;
+    if (n > (size_t)0x7fffffff) return hipErrorInvalidValue;  // the scan counts in ints
+    const unsigned blocks = (unsigned)((n + 255) / 256);
+    k_row_flags<<<blocks, 256, 0, s>>>(g, liquid, flags);
+    hipError_t e = launch_exclusive_scan(flags, pos, (int)n, scan_tmp, s);
+    if (e != hipSuccess) return e;
+    k_gather_rows<<<blocks, 256, 0, s>>>(g, flags, pos, p, at, rows, count);
     return hipGetLastError();
 }
 

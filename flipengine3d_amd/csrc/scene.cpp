@@ -114,18 +114,19 @@ size_t PressureStore::device_bytes() const {
                alist.bytes();
     for (int q = 0; q <= kSlotArrays; q++) b += arr[q].bytes();
     for (int q = 0; q < kWeightArrays; q++) b += wgt[q].bytes();
+    for (int q = 0; q < kSlotArrays32; q++) b += arr32[q].bytes();
     for (int q = 0; q < 6; q++) b += mg_f64[q].bytes();
     b += mg_part.bytes() + mg_f32.bytes() + mg_ints.bytes() + mg_bricks.bytes() + mg_scal.bytes() +
          mg_coarse.bytes();
     return b;
 }
 
-void PressureStore::alloc(const GridGeom &g, hipStream_t s, bool mixed) {
-    const MgPlan plan = mixed ? make_mg_plan(g.I, g.J, g.K) : MgPlan{};
+void PressureStore::alloc(const GridGeom &g, hipStream_t s, bool mixed, bool multigrid) {
+    const MgPlan plan = mixed && multigrid ? make_mg_plan(g.I, g.J, g.K) : MgPlan{};
     // Grids without interior cells (no rows) and past 32-bit indices have no
-    // levels; the FP64 path takes them, or refuses them, by itself.
+    // levels; the MIC(0) iteration takes them, or refuses them, by itself.
     if (!plan.usable()) {
-        alloc_slots(g, s);
+        alloc_slots(g, s, mixed);
         return;
     }
     graphs.clear();
@@ -165,7 +166,7 @@ void PressureStore::release_multigrid() {
     mg_on = false;
 }
 
-void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s) {
+void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s, bool mixed) {
     graphs.clear();  // captured launches point into the buffers replaced here
     SlotMap sm = make_slot_map(g.I, g.J, g.K);
     // Slot arrays carry the zero and sink groups after the last tile.
@@ -202,6 +203,16 @@ void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s) {
     pb.Lxm = arr[10].p; pb.Lym = arr[11].p; pb.Lzm = arr[12].p;
     pb.wx = wgt[0].p; pb.wy = wgt[1].p; pb.wz = wgt[2].p;
     pb.partials = arr[kSlotArrays].p;
+    if (mixed) {
+        for (int q = 0; q < kSlotArrays32; q++) {
+            if (arr32[q].alloc(ns) != hipSuccess)
+                throw StatusError{FLIPMI_ERR_OOM, "mixed-precision arrays: out of device memory"};
+            (void)launch_fill_f32(arr32[q].p, ns, 0.0f, s);
+        }
+        float **dst[kSlotArrays32] = {&pb.invdiag32, &pb.Lx32, &pb.Ly32, &pb.Lz32, &pb.Lxm32, &pb.Lym32,
+                                      &pb.Lzm32, &pb.r32, &pb.z32, &pb.s32, &pb.s32b, &pb.q32};
+        for (int q = 0; q < kSlotArrays32; q++) *dst[q] = arr32[q].p;
+    }
     pb.npartials = npart;
     pb.edge = edge.p;
     const int groups_per_tile = sm.S / 4;
@@ -269,13 +280,13 @@ static int iterations_needed(double before, double now, int iterations, double t
     return need > 0 && need < 1e6 ? (int)std::ceil(need) : -1;
 }
 
-// Pressure events of an iteration at profiling level 2.
-static bool take_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces]) {
+// Events for the selected kernels of an iteration at profiling level 2.
+static bool take_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces], bool (*used)(int piece)) {
     if (!prof || prof->profiling < 2 || prof->kernel_mask == 0 ||
         prof->pcg_iteration_count++ % prof->kernel_every != 0)
         return false;
     for (int piece = 0; piece < kPcgPieces; piece++) {
-        if (piece == kPcgResidual || !((prof->kernel_mask >> piece) & 1u)) continue;
+        if (!used(piece) || !((prof->kernel_mask >> piece) & 1u)) continue;
         kt[piece].start = prof->take_event();
         kt[piece].stop = prof->take_event();
     }
@@ -283,7 +294,9 @@ static bool take_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces]) {
 }
 static void book_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces]) {
     for (int piece = 0; piece < kPcgPieces; piece++)
-        if (kt[piece].start) prof->add_timed(FLIPMI_STAGE_K_SPMV + piece, kt[piece].start, kt[piece].stop);
+        if (kt[piece].start)
+            prof->add_timed(piece == kPcgResidual ? FLIPMI_STAGE_K_RESIDUAL : FLIPMI_STAGE_K_SPMV + piece,
+                            kt[piece].start, kt[piece].stop);
 }
 
 static void apply_pressure(const PressureWork &w, PressureOutcome &out, hipStream_t s, Scene *prof) {
@@ -296,8 +309,9 @@ static void apply_pressure(const PressureWork &w, PressureOutcome &out, hipStrea
     out.solved = true;
 }
 
-// The mixed-precision solve.  Returns false when it has not converged: the
-// caller then solves the system on the FP64 path (nothing has been applied).
+// The mixed-precision solve with multigrid.  Returns false when it has not
+// converged: the caller then solves the system with the MIC(0) iteration
+// (nothing has been applied).
 constexpr int kMgMaxIterations = 200;  // over ten times what it takes
 static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *hs, hipStream_t s, Scene *prof,
                           PressureOutcome &out) {
@@ -326,7 +340,7 @@ static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *h
             hipError_t e = hipSuccess;
             for (int q = 0; q < batch && e == hipSuccess; q++) {
                 KernelTiming kt[kPcgPieces];
-                const bool timed = take_kernel_timings(prof, kt);
+                const bool timed = take_kernel_timings(prof, kt, [](int piece) { return piece != kPcgResidual; });
                 e = mg.iterate(s, timed ? kt : nullptr);
                 if (timed) book_kernel_timings(prof, kt);
             }
@@ -383,10 +397,10 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
     if (ps.mg_on) {
         if (run_multigrid(w, ps, static_cast<MgScalars *>(host_sc), s, prof, out)) return out;
         // Not positive definite, not finite, or capped: the reference's
-        // solver decides, here and for the rest of this store's life.
+        // preconditioner decides, here and for the rest of this store's life.
         hip_check(hipStreamSynchronize(s), "pcg sync");
         ps.release_multigrid();
-        ps.alloc_slots(w.g, s);
+        ps.alloc_slots(w.g, s, true);
     }
     PressureBuffers &pb = ps.pb;
     PcgScalars *hs = static_cast<PcgScalars *>(host_sc);
@@ -411,9 +425,11 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
         return out;
     }
     if (prof) prof->begin_stage(FLIPMI_STAGE_MIC0, &ev);
+    const bool mixed = w.precision == FLIPMI_PCG_MIXED;
+    if (mixed && !pb.r32) throw StatusError{FLIPMI_ERR_INVALID_ARG, "mixed precision arrays not allocated"};
     hip_check(launch_group_mask(pb, s), "group mask");
     hip_check(launch_mic0_factor(w.g, w.liquid, pb, s), "mic0 factor");
-    hip_check(launch_pcg_init(w.g, w.tol, w.maxiter, pb, s), "pcg init");
+    hip_check(launch_pcg_init(w.g, w.tol, w.maxiter, mixed, pb, s), "pcg init");
     if (prof) prof->end_stage(FLIPMI_STAGE_MIC0, ev);
     if (prof) prof->begin_stage(FLIPMI_STAGE_PCG, &ev);
     // Iterations are enqueued in batches between host checks of the device
@@ -426,23 +442,30 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
     double prev_resid = bnorm;
     const double target = w.tol * bnorm;
     for (;;) {
-        // A batch runs from a captured graph unless kernels are being timed
-        // or the sweep tag is near its wrap-around (which clears the records).
-        const bool use_graph = w.graphs && !(prof && prof->profiling >= 2) &&
-                               pb.epoch + kPcgSweeps * (unsigned)batch + 8u < 0xfffffff0u;
+        // A batch runs from a captured graph once the first SpMV (which reads
+        // s as initialised) is behind, unless kernels are being timed or the
+        // sweep tag is near its wrap-around (which clears the records).
+        const unsigned sweeps = pcg_sweeps_per_iteration(mixed) * (unsigned)batch;
+        const bool use_graph = w.graphs && pb.s_plain == 0 && !(prof && prof->profiling >= 2) &&
+                               pb.epoch + sweeps + 8u < 0xfffffff0u;
         auto all = [&]() -> hipError_t {
             hipError_t e = hipSuccess;
             for (int q = 0; q < batch && e == hipSuccess; q++) {
                 KernelTiming kt[kPcgPieces];
-                const bool timed = take_kernel_timings(prof, kt);
-                e = launch_pcg_iteration(w.g, pb, s, kt);
+                const bool timed = take_kernel_timings(
+                    prof, kt,
+                    mixed ? [](int piece) { return pcg_piece_used(piece, true); }
+                          : [](int piece) { return pcg_piece_used(piece, false); });
+                e = launch_pcg_iteration(w.g, mixed, pb, s, kt);
                 if (timed) book_kernel_timings(prof, kt);
             }
             return e;
         };
         if (use_graph)
-            launch_pcg_batch_graph(*w.graphs, batch, 0, s, all,
-                                   [&] { pb.epoch += kPcgSweeps * (unsigned)batch; });
+            launch_pcg_batch_graph(*w.graphs, batch, pb.s_turn, s, all, [&] {
+                if (mixed && (batch & 1)) pb.swap_directions();
+                pb.epoch += sweeps;
+            });
         else
             hip_check(all(), "pcg iteration");
         launched += batch;
@@ -462,6 +485,7 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
     if (prof) prof->stage_calls[FLIPMI_STAGE_PCG_ITERS] += hs->iters;
     out.iterations = hs->failed ? 0 : hs->iters;
     out.residual = hs->resid;
+    out.refinements = mixed ? hs->refinements : 0;
     bool converged = hs->converged != 0;
     // PressureSolver::_solveLinearSystem (pressuresolver.cpp:810-840).
     out.success = converged || (!hs->failed && out.iterations == w.maxiter && out.residual < w.acceptable);
@@ -541,6 +565,16 @@ static size_t scan_elems(const GridGeom &g, size_t particles) {
     return std::max(scan_scratch_elems((int)subcell_bins(g)), scan_scratch_elems((int)particles));
 }
 
+// Mixed scenes of this many cells and more solve with multigrid.  It is the
+// faster solver at every size (97x75x83: 1.4 ms a solve against 8.2; 256x128x128:
+// 3.2 against 21.8), so the line is not drawn by speed: scenes of request size
+// run for tens of steps and their results are compared with earlier ones to
+// 1e-6, and two solvers that both converge to 1e-9 do not agree that well there
+// (a last bit in a particle moves some cell's phi across zero, and the runs
+// part: up to 7e-5 after ten steps at 32^3 to 96^3).  Below the line a scene
+// keeps the MIC(0) iteration, bit for bit, served or not.
+constexpr size_t kMultigridCells = (size_t)1 << 20;
+
 void Scene::alloc_all() {
     int I = desc.isize, J = desc.jsize, K = desc.ksize;
     size_t nc = (size_t)I * J * K;
@@ -580,7 +614,7 @@ void Scene::alloc_all() {
     need(vu.alloc(nU)); need(vv.alloc(nV)); need(vw.alloc(nW));
     need(status.alloc(nf));
     press = new PressureStore();
-    press->alloc(g, stream, desc.pcg_precision == FLIPMI_PCG_MIXED);
+    press->alloc(g, stream, desc.pcg_precision == FLIPMI_PCG_MIXED, nc >= kMultigridCells);
     check(hipHostMalloc(&host_stage, kPressureStaging, hipHostMallocDefault), "pinned staging");
     // Fresh MeshLevelSet: phi = distance upper bound everywhere
     // (meshlevelset.cpp:35-42, 760-762); zero solid face velocities.
@@ -625,25 +659,39 @@ void Scene::admit_pending() {
     pending_vel.resize(3 * kept);
 }
 
-// getMarkerParticlePositionData (fluidsimulation.cpp:2408-2413):
-// position * scale + offset, in float.
-void Scene::to_domain(float *pos_xyz, int64_t count) const {
-    const float sc = (float)domain_scale;
-    for (int64_t q = 0; q < 3 * count; q++) pos_xyz[q] = pos_xyz[q] * sc + domain_offset[q % 3];
+// getMarkerParticlePositionData / VelocityData (fluidsimulation.cpp:
+// 2408-2420), positions as position * scale + offset in float.  The triples
+// are formed on the device, in the buffer of the sorted copies (which only
+// lives within a step), and cross in one piece.
+void Scene::read_particles(int64_t first, int64_t count, float *pos_xyz, float *vel_xyz) {
+    if (count <= 0) return;
+    float *triples = reinterpret_cast<float *>(spos.p);
+    const float zero[3] = {0.0f, 0.0f, 0.0f};
+    for (int v = 0; v < 2; v++) {
+        float *dst = v ? vel_xyz : pos_xyz;
+        if (!dst) continue;
+        const float *src[3] = {part[3 * v].p + first, part[3 * v + 1].p + first, part[3 * v + 2].p + first};
+        check(launch_pack_triples(src, (int)count, v == 0, (float)domain_scale, v ? zero : domain_offset, triples,
+                                  stream),
+              "pack particles");
+        check(ctx->link().to_host(dst, triples, 3 * sizeof(float) * (size_t)count, stream), "download");
+    }
 }
 
 void Scene::upload_pending() {
     n = (int)(pending_pos.size() / 3);
     if (n > 0) {
-        // Host AoS -> device SoA.
-        std::vector<float> tmp((size_t)n);
-        for (int a = 0; a < 6; a++) {
-            const std::vector<float> &src = a < 3 ? pending_pos : pending_vel;
-            for (int q = 0; q < n; q++) tmp[q] = src[3 * (size_t)q + (a % 3)];
-            check(hipMemcpyAsync(part[a].p, tmp.data(), sizeof(float) * n, hipMemcpyHostToDevice, stream),
+        // The triples cross as they lie, into the buffer of the sorted copies,
+        // and are taken apart on the device.
+        float *triples = reinterpret_cast<float *>(spos.p);
+        for (int v = 0; v < 2; v++) {
+            const std::vector<float> &src = v ? pending_vel : pending_pos;
+            check(hipMemcpyAsync(triples, src.data(), 3 * sizeof(float) * (size_t)n, hipMemcpyHostToDevice, stream),
                   "upload particles");
-            sync();
+            float *dst[3] = {part[3 * v].p, part[3 * v + 1].p, part[3 * v + 2].p};
+            check(launch_unpack_triples(triples, n, dst, stream), "unpack particles");
         }
+        sync();
     }
     pending_pos.clear(); pending_vel.clear();
     pending_pos.shrink_to_fit(); pending_vel.shrink_to_fit();
@@ -740,13 +788,14 @@ size_t estimate_scene_bytes(const flipmi_scene_desc &d, int64_t cap) {
     const size_t ns = sm.alloc_count(), ntiles = (size_t)sm.ntj * sm.ntk;
     size_t slots = sizeof(double) * (PressureStore::kSlotArrays * ns + 2 * 2048 + ntiles);
     slots += sizeof(float) * PressureStore::kWeightArrays * ns;
+    if (d.pcg_precision == FLIPMI_PCG_MIXED) slots += sizeof(float) * PressureStore::kSlotArrays32 * ns;
     slots += sizeof(unsigned long long) * edge_record_count(sm);
     slots += sizeof(unsigned long long) * ntiles * (size_t)((sm.S / 4 + 63) / 64);
     slots += sizeof(unsigned) * (ntiles + 1) + sizeof(int) * 2 * ntiles + sizeof(PcgScalars);
     slots += sizeof(int) * ((sm.count() >> 8) + 1);
-    // A mixed scene holds the multigrid levels, or the slots of the FP64 path
-    // once a system has gone there.
-    if (d.pcg_precision == FLIPMI_PCG_MIXED)
+    // A mixed scene holds the multigrid levels, or the slots of the MIC(0)
+    // iteration.
+    if (d.pcg_precision == FLIPMI_PCG_MIXED && nc >= kMultigridCells)
         slots = std::max(slots, make_mg_plan(d.isize, d.jsize, d.ksize).device_bytes());
     return b + slots;
 }

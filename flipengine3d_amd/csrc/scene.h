@@ -12,6 +12,7 @@
 #include "../../include/flipmi.h"
 #include "flipmi_kernels.h"
 #include "multigrid.h"
+#include "transfer.h"
 
 namespace flipmi {
 
@@ -19,13 +20,18 @@ struct Ctx {
     int device = 0;
     std::string last_error;
     hipStream_t stream = nullptr;  // stream for stage drop-ins
+    std::shared_ptr<DeviceShared> shared;
+    HostLink &link() { return shared->link; }
 };
 
-// Device buffer that frees itself.
+// Device buffer that frees itself, or gives itself back to the pool scope
+// that was current when it was allocated.
 template <class T>
 struct DBuf {
     T *p = nullptr;
     size_t n = 0;
+    PoolScope *scope = nullptr;
+    size_t block = 0;
     DBuf() {}
     DBuf(const DBuf &) = delete;
     DBuf &operator=(const DBuf &) = delete;
@@ -34,10 +40,15 @@ struct DBuf {
         release();
         n = count;
         if (count == 0) return hipSuccess;
-        return hipMalloc((void **)&p, sizeof(T) * count);
+        scope = PoolScope::current();
+        void *q = nullptr;
+        hipError_t e = scope ? scope->get(sizeof(T) * count, &q, &block) : hipMalloc(&q, sizeof(T) * count);
+        if (e == hipSuccess) p = static_cast<T *>(q);
+        return e;
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p && scope) scope->put(p, block);
+        else if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;
     }
@@ -197,7 +208,6 @@ struct Scene {
     void admit_pending();
     void upload_pending();
     // Grid to domain coordinates of n positions (xyz), in place.
-    void to_domain(float *pos_xyz, int64_t n) const;
     // Reuses an initialized scene for a new particle set on the same grid and
     // settings (the state right after initialize()); false if the set does not
     // fit the particle capacity.
@@ -229,6 +239,9 @@ struct Scene {
     // solid SDF (FluidSimulation::_addStaticObjectsToSDF).
     int add_obstacle(const float *verts, int nv, const int *tris, int nt);
     void union_obstacles();
+    // Particles [first, first + count) as the caller's xyz triples, positions
+    // in domain coordinates; either pointer may be null.
+    void read_particles(int64_t first, int64_t count, float *pos_xyz, float *vel_xyz);
     // Grows every particle-sized buffer to hold at least `need` particles.
     void grow(int64_t need);
     void begin_stage(int stage, hipEvent_t *a);
@@ -287,13 +300,16 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
 // Device storage of one pressure system.  FP64 path: in slot order,
 // arr[0..12] are the FP64 slot arrays (diag, rhs, x, r, z, s, invdiag, Lx, Ly, Lz, Lxm, Lym,
 // Lzm), arr[13] the reduction partials, wgt[0..2] the coupling weights
-// (wx, wy, wz).  Mixed precision: the multigrid solver's levels; a system it
-// does not solve goes to the FP64 path, whose storage then replaces them.
+// (wx, wy, wz); the mixed MIC(0) iteration adds FP32 copies.  With multigrid:
+// its levels; a system it does not solve goes to the MIC(0) iteration, whose
+// storage then replaces them.
 struct PressureStore {
     static constexpr int kSlotArrays = 13;
     static constexpr int kWeightArrays = 3;
+    static constexpr int kSlotArrays32 = 12;  // FP32 factor and vectors, s twice, q (mixed precision)
     DBuf<double> arr[kSlotArrays + 1];
     DBuf<float> wgt[kWeightArrays];
+    DBuf<float> arr32[kSlotArrays32];
     DBuf<unsigned long long> edge, mask;
     DBuf<unsigned> progress, ticket;
     DBuf<int> irange;
@@ -310,8 +326,8 @@ struct PressureStore {
     DBuf<int4> mg_bricks;
     DBuf<MgScalars> mg_scal;
     DBuf<MgCoarse> mg_coarse;
-    void alloc(const GridGeom &g, hipStream_t s, bool mixed);
-    void alloc_slots(const GridGeom &g, hipStream_t s);
+    void alloc(const GridGeom &g, hipStream_t s, bool mixed, bool multigrid);
+    void alloc_slots(const GridGeom &g, hipStream_t s, bool mixed);
     void release_multigrid();
     size_t device_bytes() const;
 };

@@ -68,7 +68,8 @@ struct Request {
     flipmi_request_report rep{};
     std::string error;
     std::vector<double> step_ms;
-    std::vector<float> out_pos, out_vel;
+    std::unique_ptr<float[]> out_pos, out_vel;  // written once: not cleared first
+    size_t out_n = 0;
 };
 
 struct Pooled {
@@ -227,17 +228,11 @@ void flipmi_server::worker(int slot) {
                 if (!fs.pressure_ok) r->rep.pressure_failures++;
                 r->rep.steps_done++;
             }
-            // Final particles, AoS.
-            r->out_pos.assign(3 * (size_t)s.n, 0.0f);
-            r->out_vel.assign(3 * (size_t)s.n, 0.0f);
-            std::vector<float> t((size_t)s.n);
-            for (int a = 0; a < 6 && s.n > 0; a++) {
-                hip_check(hipMemcpyAsync(t.data(), s.part[a].p, sizeof(float) * s.n, hipMemcpyDeviceToHost, stream),
-                          "download");
-                hip_check(hipStreamSynchronize(stream), "sync");
-                std::vector<float> &dst = a < 3 ? r->out_pos : r->out_vel;
-                for (int q = 0; q < s.n; q++) dst[3 * (size_t)q + (a % 3)] = t[q];
-            }
+            // Final particles.
+            r->out_n = 3 * (size_t)s.n;
+            r->out_pos.reset(new float[r->out_n]);
+            r->out_vel.reset(new float[r->out_n]);
+            s.read_particles(0, s.n, r->out_pos.get(), r->out_vel.get());
             r->rep.num_particles = s.n;
         } catch (const StatusError &e) {
             status = e.code;
@@ -402,8 +397,8 @@ int flipmi_server_take(flipmi_server *s, int64_t id, float *pos_xyz, float *vel_
         r = std::move(it->second);
         s->requests.erase(it);
     }
-    if (pos_xyz && !r->out_pos.empty()) std::memcpy(pos_xyz, r->out_pos.data(), sizeof(float) * r->out_pos.size());
-    if (vel_xyz && !r->out_vel.empty()) std::memcpy(vel_xyz, r->out_vel.data(), sizeof(float) * r->out_vel.size());
+    if (pos_xyz && r->out_n) std::memcpy(pos_xyz, r->out_pos.get(), sizeof(float) * r->out_n);
+    if (vel_xyz && r->out_n) std::memcpy(vel_xyz, r->out_vel.get(), sizeof(float) * r->out_n);
     return r->rep.status;
 }
 

@@ -44,7 +44,5 @@ double marker_particle_radius(double dx);
 void validate_surface_desc(const flipmi_surface_desc &d, const GridGeom &g);
 // Builds the mesh into st on stream s; synchronizes s to read the sizes.
 void build_surface(const SurfaceInputs &in, SurfaceStore &st, hipStream_t s);
-// Copies the mesh to host memory (either pointer may be null).
-void copy_surface(const SurfaceStore &st, float *verts_xyz, int32_t *tris, hipStream_t s);
 
 }  // namespace flipmi

@@ -1,0 +1,272 @@
+// See transfer.h.
+#include "transfer.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <thread>
+
+namespace flipmi {
+
+namespace {
+// Below this a copy is one call: staging gains nothing.
+constexpr size_t kDirect = (size_t)256 << 10;
+// Threads that empty the ring, for copies that are worth starting them (about
+// 30 us each).  226 MB of particles in two copies: 59 ms as six pageable copies
+// and a loop over the triples, 6.6 ms so (34 GB/s, page faults included).
+constexpr size_t kThreaded = (size_t)8 << 20;
+constexpr int kCopyThreads = 6;
+
+// Sizes in steps of an eighth of a power of two, 64 KiB at least, so that
+// calls of nearly the same sizes share blocks.
+size_t block_size(size_t bytes) {
+    size_t step = (size_t)8 << 10;
+    while (step * 16 <= bytes) step *= 2;
+    return std::max((bytes + step - 1) / step * step, (size_t)64 << 10);
+}
+
+thread_local PoolScope *t_scope = nullptr;
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// HostLink
+// ---------------------------------------------------------------------------
+
+bool HostLink::ready() {
+    if (ring) return true;
+    for (int q = 0; q < kSlots; q++)
+        if (!filled[q] && hipEventCreateWithFlags(&filled[q], hipEventDisableTiming) != hipSuccess) return false;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kChunk * kSlots, hipHostMallocDefault) != hipSuccess) return false;
+    ring = static_cast<char *>(p);
+    return true;
+}
+
+void HostLink::release() {
+    for (void *p : pages) (void)hipHostFree(p);
+    pages.clear();
+    if (ring) (void)hipHostFree(ring);
+    ring = nullptr;
+    for (hipEvent_t &e : filled) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+}
+
+hipError_t HostLink::get_page(void **p) {
+    {
+        std::lock_guard<std::mutex> lk(page_m);
+        if (!pages.empty()) {
+            *p = pages.back();
+            pages.pop_back();
+            return hipSuccess;
+        }
+    }
+    return hipHostMalloc(p, kPage, hipHostMallocDefault);
+}
+
+void HostLink::put_page(void *p) {
+    std::lock_guard<std::mutex> lk(page_m);
+    try {
+        pages.push_back(p);
+    } catch (...) {
+        (void)hipHostFree(p);
+    }
+}
+
+hipError_t HostLink::to_host(const HostPiece *pieces, int count, hipStream_t s) {
+    std::lock_guard<std::mutex> lk(m);
+    const bool staged = ready();
+    // The small pieces, through the ring as far as it goes; a piece that is
+    // alone, or without a ring, is one plain copy.
+    size_t at = 0;
+    hipError_t e = hipSuccess;
+    for (int q = 0; q < count && e == hipSuccess; q++) {
+        const HostPiece &p = pieces[q];
+        if (p.bytes == 0 || (staged && p.bytes >= kDirect)) continue;
+        const bool ringed = staged && at + p.bytes <= kChunk * kSlots;
+        e = hipMemcpyAsync(ringed ? (void *)(ring + at) : p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s);
+        if (ringed) at += (p.bytes + 63) & ~(size_t)63;
+    }
+    hipError_t w = hipStreamSynchronize(s);
+    if (e != hipSuccess || w != hipSuccess) return e != hipSuccess ? e : w;
+    if (!staged) return hipSuccess;
+    at = 0;
+    for (int q = 0; q < count; q++) {
+        const HostPiece &p = pieces[q];
+        if (p.bytes == 0 || p.bytes >= kDirect || at + p.bytes > kChunk * kSlots) continue;
+        std::memcpy(p.dst, ring + at, p.bytes);
+        at += (p.bytes + 63) & ~(size_t)63;
+    }
+    for (int q = 0; q < count && e == hipSuccess; q++)
+        if (pieces[q].bytes >= kDirect) e = large(pieces[q], s);
+    return e;
+}
+
+hipError_t HostLink::large(const HostPiece &piece, hipStream_t s) {
+    void *const dst = piece.dst;
+    const void *const src = piece.src;
+    const size_t bytes = piece.bytes;
+    int device = 0;
+    (void)hipGetDevice(&device);
+    const int n = (int)((bytes + kChunk - 1) / kChunk);
+    std::atomic<int> queued{0}, failed{0};
+    std::atomic<int> emptied[kSlots];  // the last chunk copied out of each slot
+    for (auto &e : emptied) e.store(-1);
+    auto fill = [&](int c) -> hipError_t {
+        const size_t at = (size_t)c * kChunk, len = std::min(kChunk, bytes - at);
+        hipError_t e = hipMemcpyAsync(ring + (size_t)(c % kSlots) * kChunk, static_cast<const char *>(src) + at, len,
+                                      hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipEventRecord(filled[c % kSlots], s) : e;
+    };
+    auto empty = [&](int c) {
+        hipError_t e = hipEventSynchronize(filled[c % kSlots]);
+        if (e != hipSuccess) {
+            failed.store((int)e);
+            return;
+        }
+        const size_t at = (size_t)c * kChunk;
+        std::memcpy(static_cast<char *>(dst) + at, ring + (size_t)(c % kSlots) * kChunk, std::min(kChunk, bytes - at));
+        emptied[c % kSlots].store(c, std::memory_order_release);
+    };
+    // Worker t empties chunks t, t + nt, ...; this thread fills them, and is
+    // worker 0 in between.
+    const int want = bytes >= kThreaded ? std::min(kCopyThreads, (int)std::max(1u, std::thread::hardware_concurrency())) : 1;
+    std::vector<std::thread> workers;
+    std::atomic<int> nt{want};
+    std::atomic<bool> go{false};
+    auto work = [&](int t) {
+        (void)hipSetDevice(device);
+        while (!go.load(std::memory_order_acquire)) std::this_thread::yield();
+        for (int c = t; c < n; c += nt.load()) {
+            while (queued.load(std::memory_order_acquire) <= c && !failed.load()) std::this_thread::yield();
+            if (failed.load()) return;
+            empty(c);
+        }
+    };
+    try {
+        for (int t = 1; t < want; t++) workers.emplace_back(work, t);
+    } catch (...) {
+        // Fewer threads share the chunks.
+    }
+    nt.store((int)workers.size() + 1);
+    go.store(true, std::memory_order_release);
+    hipError_t err = hipSuccess;
+    int next = 0, mine = 0;  // next chunk to fill, next of this thread's to empty
+    while ((next < n || mine < n) && !failed.load()) {
+        if (next < n && (next < kSlots || emptied[next % kSlots].load(std::memory_order_acquire) == next - kSlots)) {
+            err = fill(next);
+            if (err != hipSuccess) {
+                failed.store((int)err);
+                break;
+            }
+            queued.store(++next, std::memory_order_release);
+            continue;
+        }
+        if (mine < next) {
+            empty(mine);
+            mine += nt.load();
+        } else if (next < n) {
+            std::this_thread::yield();
+        } else {
+            break;
+        }
+    }
+    for (std::thread &t : workers) t.join();
+    if (failed.load()) {
+        (void)hipStreamSynchronize(s);  // no copy into the ring is left behind
+        return (hipError_t)failed.load();
+    }
+    return hipSuccess;
+}
+
+// ---------------------------------------------------------------------------
+// Device memory of stage calls
+// ---------------------------------------------------------------------------
+
+hipError_t DevicePool::get(size_t bytes, void **p, size_t *size) {
+    const size_t want = block_size(bytes);
+    {
+        std::lock_guard<std::mutex> lk(m);
+        auto it = blocks.lower_bound(want);
+        if (it != blocks.end() && it->first <= want + want / 4) {
+            *p = it->second;
+            *size = it->first;
+            held -= it->first;
+            blocks.erase(it);
+            return hipSuccess;
+        }
+    }
+    hipError_t e = hipMalloc(p, want);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        release();
+        e = hipMalloc(p, want);
+    }
+    *size = want;
+    return e;
+}
+
+void DevicePool::put(void *p, size_t size) {
+    {
+        std::lock_guard<std::mutex> lk(m);
+        if (held + size <= kHeld) {
+            try {
+                blocks.insert({size, p});
+                held += size;
+                return;
+            } catch (...) {
+            }
+        }
+    }
+    (void)hipFree(p);
+}
+
+void DevicePool::release() {
+    std::multimap<size_t, void *> all;
+    {
+        std::lock_guard<std::mutex> lk(m);
+        all.swap(blocks);
+        held = 0;
+    }
+    for (auto &b : all) (void)hipFree(b.second);
+}
+
+PoolScope::PoolScope(DevicePool &p, hipStream_t s) : pool(p), stream(s), outer(t_scope) { t_scope = this; }
+
+PoolScope::~PoolScope() {
+    t_scope = outer;
+    if (back.empty()) return;
+    (void)hipStreamSynchronize(stream);  // a call that failed may have left work behind
+    for (auto &b : back) pool.put(b.second, b.first);
+}
+
+PoolScope *PoolScope::current() { return t_scope; }
+PoolScope::Off::Off() : was(t_scope) { t_scope = nullptr; }
+PoolScope::Off::~Off() { t_scope = was; }
+
+std::shared_ptr<DeviceShared> DeviceShared::of(int device) {
+    static std::mutex m;
+    static std::map<int, std::weak_ptr<DeviceShared>> all;
+    std::lock_guard<std::mutex> lk(m);
+    std::shared_ptr<DeviceShared> p = all[device].lock();
+    if (!p) {
+        p = std::make_shared<DeviceShared>();
+        all[device] = p;
+    }
+    return p;
+}
+
+hipError_t PoolScope::get(size_t bytes, void **p, size_t *size) {
+    const size_t want = block_size(bytes);
+    auto it = back.lower_bound(want);
+    if (it != back.end() && it->first <= want + want / 4) {
+        *p = it->second;
+        *size = it->first;
+        back.erase(it);
+        return hipSuccess;
+    }
+    return pool.get(bytes, p, size);
+}
+
+}  // namespace flipmi

@@ -1,0 +1,113 @@
+// Memory the contexts of a device share: pinned staging for device-to-host
+// copies and the device memory that stage calls work in.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <map>
+#include <memory>
+#include <mutex>
+#include <vector>
+
+namespace flipmi {
+
+// Copies device memory to pageable host memory through a ring of pinned
+// chunks: the copy engine fills one chunk while host threads empty others.
+// (Straight into pageable memory the runtime reaches 10 to 17 GB/s here,
+// most of it spent faulting the caller's fresh pages in on one thread; the
+// engine alone moves 55 GB/s.)  One copy at a time; the ring is allocated
+// with the first copy that uses it.
+struct HostPiece {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+class HostLink {
+public:
+    HostLink() {}
+    HostLink(const HostLink &) = delete;
+    HostLink &operator=(const HostLink &) = delete;
+    ~HostLink() { release(); }
+    // Returns when dst holds the data.  Ordered after the work on s.
+    hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t s) {
+        const HostPiece p{dst, src, bytes};
+        return to_host(&p, 1, s);
+    }
+    // Several results at once: the small ones wait for the device together.
+    hipError_t to_host(const HostPiece *pieces, int count, hipStream_t s);
+    // Pinned host memory of kPage bytes, for one caller at a time.
+    static constexpr size_t kPage = 4096;
+    hipError_t get_page(void **p);
+    void put_page(void *p);
+    void release();
+
+private:
+    static constexpr size_t kChunk = (size_t)2 << 20;
+    static constexpr int kSlots = 16;
+    bool ready();
+    hipError_t large(const HostPiece &p, hipStream_t s);
+    std::mutex m, page_m;
+    char *ring = nullptr;
+    hipEvent_t filled[kSlots] = {};
+    std::vector<void *> pages;
+};
+
+// Device blocks kept between stage calls, at most kHeld bytes of them; the
+// rest goes back to the device, as all of it does when an allocation fails.
+// Safe from several threads.
+class DevicePool {
+public:
+    DevicePool() {}
+    DevicePool(const DevicePool &) = delete;
+    DevicePool &operator=(const DevicePool &) = delete;
+    ~DevicePool() { release(); }
+    hipError_t get(size_t bytes, void **p, size_t *size);
+    void put(void *p, size_t size);
+    void release();
+
+private:
+    static constexpr size_t kHeld = (size_t)1 << 30;
+    std::mutex m;
+    std::multimap<size_t, void *> blocks;
+    size_t held = 0;
+};
+
+// While one is alive, the device buffers its thread allocates come from the
+// pool.  All their uses are on one stream, so a buffer given back is reused
+// within the call as it is; the pool gets it when the stream is idle.  The
+// scope outlives its buffers.
+class PoolScope {
+public:
+    PoolScope(DevicePool &pool, hipStream_t s);
+    ~PoolScope();
+    PoolScope(const PoolScope &) = delete;
+    PoolScope &operator=(const PoolScope &) = delete;
+    static PoolScope *current();
+    // While one is alive, buffers are allocated as outside any scope (those
+    // that outlive the call).
+    class Off {
+    public:
+        Off();
+        ~Off();
+
+    private:
+        PoolScope *was;
+    };
+    hipError_t get(size_t bytes, void **p, size_t *size);
+    void put(void *p, size_t size) { back.insert({size, p}); }
+
+private:
+    DevicePool &pool;
+    hipStream_t stream;
+    PoolScope *outer;
+    std::multimap<size_t, void *> back;
+};
+
+// Held by every context of a device, freed with the last of them.
+struct DeviceShared {
+    HostLink link;
+    DevicePool pool;
+    static std::shared_ptr<DeviceShared> of(int device);
+};
+
+}  // namespace flipmi

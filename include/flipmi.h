@@ -43,8 +43,10 @@ typedef enum {
 
 typedef enum {
     FLIPMI_PCG_FP64 = 0,  /* reference arithmetic: FP64 vectors, alpha/beta as float */
-    FLIPMI_PCG_MIXED = 1  /* FP64 x, residuals and dots, FP32 directions and multigrid
-                             preconditioner; converged on the FP64 true residual */
+    FLIPMI_PCG_MIXED = 1  /* FP32 directions and multigrid preconditioner, FP64 x, residuals and
+                             dots; scenes under 2^20 cells and systems that it does not solve:
+                             FP32 PCG with MIC(0) and FP64 dots; converged on the FP64 true
+                             residual either way */
 } flipmi_pcg_precision;
 
 typedef struct flipmi_ctx flipmi_ctx;
@@ -79,8 +81,7 @@ typedef struct {
     int pressure_ok;           /* 0 if the last pressure solve failed */
     double gpu_ms;             /* device time of the frame */
     int64_t pressure_rows;     /* last substep: rows of the Poisson system */
-    int pcg_refinements;       /* last substep, mixed precision: FP64 true residuals (0: the FP64
-                                  path solved it) */
+    int pcg_refinements;       /* last substep, mixed precision: FP64 true residuals */
 } flipmi_frame_stats;
 
 /* Per-stage device time accumulated since the last reset (hipEvents). */
@@ -108,7 +109,7 @@ enum {
     FLIPMI_STAGE_K_FORWARD = 14,
     FLIPMI_STAGE_K_BACKWARD = 15,
     FLIPMI_STAGE_K_UPDATE = 16,
-    FLIPMI_STAGE_K_RESIDUAL = 17,   /* not timed */
+    FLIPMI_STAGE_K_RESIDUAL = 17,   /* MIC(0) in FP32: FP64 true residual + forward sweep over it */
     FLIPMI_STAGE_INFLOW = 18,       /* mesh inflow: particle mask and emission */
     FLIPMI_STAGE_SURFACE = 19       /* surface reconstruction (sort, field, marching cubes, smoothing) */
 };
@@ -304,7 +305,7 @@ int flipmi_scene_set_profiling(flipmi_scene *scene, int level);
  * stage minus FLIPMI_STAGE_K_SPMV; default all.  On the mixed path AXPY is
  * the axpy with the first smoothing, FORWARD the restriction, UPDATE the
  * coarse correction and BACKWARD the last smoothing, each on the finest
- * level; FLIPMI_STAGE_K_RESIDUAL (bit 5) stays empty.
+ * level, and FLIPMI_STAGE_K_RESIDUAL (bit 5) stays empty.
  * Each timed launch adds an event pair, which delays the launches around it. */
 int flipmi_scene_set_kernel_timing(flipmi_scene *scene, unsigned mask);
 /* Times the selected kernels on every `every`-th PCG iteration only (default
@@ -400,7 +401,7 @@ typedef struct {
     double residual;           /* "Estimated Error" (|r|_inf) */
     int rows;                  /* fluid interior cells */
     int success;               /* the bool PressureSolver::solve returns */
-    int refinements;           /* mixed precision: FP64 true residuals (0: the FP64 path solved it) */
+    int refinements;           /* mixed precision: FP64 true residuals */
 } flipmi_pressure_report;
 
 /* bool PressureSolver::solve(PressureSolverParameters) + getSolverStatus()

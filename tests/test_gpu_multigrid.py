@@ -7,10 +7,10 @@ and, the smallest, a single cell per level.  Both paths stop on the same FP64
 true residual, 1e-9 of |b|_inf, so the pressures agree to the bound the mixed
 path states (1e-6 of the largest) and the velocities to 1e-5 of the fastest.
 
-What the preconditioner does not solve goes to the FP64 path, with that
-path's results bit for bit: an iteration cap below its need, values that are
-not finite, and a pocket that borders no air (its pressure is fixed up to a
-constant only).
+What it does not solve goes to the MIC(0) iteration, which treats the system
+as the FP64 path does: an iteration cap below its need, values that are not
+finite.  So does, in the projection call, a pocket that borders no air (its
+pressure is fixed up to a constant, which follows from the preconditioner).
 """
 
 import numpy as np
@@ -36,8 +36,8 @@ def test_level_sizes(gpu, oracle, dims, box):
     inputs = _projection_inputs(oracle, *dims, seed=5, box=box)
     a, b = _both(gpu, inputs, dims)
     assert a["ok"] == b["ok"] == 1 and a["rows"] == b["rows"] > 0
-    # One true residual confirms the solve; 0: the FP64 path did it, which only
-    # the smallest grid calls for (cells of its single layer touch no air).
+    # One true residual confirms a multigrid solve.  The smallest grid's single
+    # layer touches no air in one of the boxes.
     assert b["refinements"] == 1 or dims == (8, 5, 6)
     assert np.abs(a["soln"] - b["soln"]).max() <= 1e-6 * np.abs(a["soln"]).max()
     vmax = max(float(np.abs(g).max()) for g in a["mac"])
@@ -59,13 +59,14 @@ def test_no_rows(gpu, oracle):
 
 
 @pytest.mark.parametrize("cap", [1, 4])
-def test_capped_solve_is_the_fp64_paths(gpu, oracle, cap):
+def test_capped_solve_is_mic0s(gpu, oracle, cap):
+    # As many iterations of the same method in FP32 and in FP64: the iterates
+    # agree to FP32 rounding.
     dims = (24, 28, 21)
     a, b = _both(gpu, _projection_inputs(oracle, *dims), dims, maxiter=cap)
-    assert a["iters"] == b["iters"] == cap and a["ok"] == b["ok"] and a["err"] == b["err"]
-    assert bits_equal(a["soln"], b["soln"])
-    for x, y in zip(a["mac"], b["mac"]):
-        assert bits_equal(x, y)
+    assert a["iters"] == b["iters"] == cap and a["ok"] == b["ok"]
+    assert abs(a["err"] - b["err"]) <= 1e-5 * a["err"]
+    assert np.abs(a["soln"] - b["soln"]).max() <= 1e-5 * np.abs(a["soln"]).max()
 
 
 def test_not_finite(gpu, oracle):
@@ -85,16 +86,18 @@ def test_pocket_keeps_its_constant(gpu, oracle):
     dims = (20, 18, 17)
     dx, solid, weights, liquid, mac, valid, *_ = pocket_inputs(oracle, *dims)
     a, b = _both(gpu, (dx, solid, weights, liquid, mac, valid), dims)
-    assert a["ok"] == b["ok"] == 1 and bits_equal(a["soln"], b["soln"])
+    assert a["ok"] == b["ok"] == 1
+    assert np.abs(a["soln"] - b["soln"]).max() <= 1e-6 * np.abs(a["soln"]).max()
 
 
-def test_scene_goes_on_after_the_fp64_path_took_over(gpu):
+def test_scene_goes_on_after_mic0_took_over(gpu):
+    # The smallest scenes that solve with multigrid hold 2^20 cells.
     import flipengine3d_amd as fa
-    n = 24
-    s = dam(n, n, n, seed=2)
+    I, J, K = 1024, 32, 32
+    s = dam(I, J, K, seed=2, box=(0.0, 0.0, 0.0, 0.2, 0.5, 1.0))
     sims = []
     for prec in (fa.PCG_FP64, fa.PCG_MIXED):
-        sim = fa.FluidSimulation(n, n, n, s.dx, ctx=gpu, precision=prec)
+        sim = fa.FluidSimulation(I, J, K, s.dx, ctx=gpu, precision=prec)
         sim.addBodyForce(0.0, -9.81, 0.0)
         sim.setPressureSolverTolerance(1e-9, 5)
         sim.loadMarkerParticleData(s.positions, s.velocities)
@@ -102,7 +105,49 @@ def test_scene_goes_on_after_the_fp64_path_took_over(gpu):
         sim.set_launch_graphs(True)
         sims.append(sim)
     for f in range(3):
-        st = [sim.update(1 / 60) for sim in sims]
+        st = [sim.update(1 / 480) for sim in sims]
         assert st[0].pressure_ok == st[1].pressure_ok and st[0].pcg_iterations == st[1].pcg_iterations
+        (p0, v0), (p1, v1) = sims[0].particles(), sims[1].particles()
+        assert np.abs(p0 - p1).max() <= 1e-3 * s.dx and np.abs(v0 - v1).max() <= 1e-3
+
+
+def test_scene_on_either_side_of_the_line(gpu):
+    # 2^20 cells and one plane less: both follow the FP64 path.
+    import flipengine3d_amd as fa
+    for I in (1024, 1023):
+        s = dam(I, 32, 32, seed=3, box=(0.0, 0.0, 0.0, 0.15, 0.6, 1.0))
+        sims = []
+        for prec in (fa.PCG_FP64, fa.PCG_MIXED):
+            sim = fa.FluidSimulation(I, 32, 32, s.dx, ctx=gpu, precision=prec)
+            sim.addBodyForce(0.0, -9.81, 0.0)
+            sim.loadMarkerParticleData(s.positions, s.velocities)
+            sim.initialize()
+            sim.set_launch_graphs(True)
+            sims.append(sim)
+        for _ in range(2):
+            st = [sim.update(1 / 480) for sim in sims]
+            assert st[0].pressure_ok == st[1].pressure_ok == 1
+            # Multigrid confirms with one true residual; MIC(0) in FP32 replaces
+            # its residual several times on the way.
+            assert (st[1].pcg_refinements == 1) == (I == 1024)
+        (p0, v0), (p1, v1) = sims[0].particles(), sims[1].particles()
+        assert p0.shape == p1.shape
+        assert np.abs(p0 - p1).max() <= 1e-3 * s.dx and np.abs(v0 - v1).max() <= 1e-3
+
+
+def test_graph_batches_match_kernel_launches(gpu):
+    import flipengine3d_amd as fa
+    s = dam(1024, 32, 32, seed=7, box=(0.0, 0.0, 0.0, 0.12, 0.5, 1.0))
+    sims = []
+    for graphs in (False, True):
+        sim = fa.FluidSimulation(1024, 32, 32, s.dx, ctx=gpu, precision=fa.PCG_MIXED)
+        sim.addBodyForce(0.0, -9.81, 0.0)
+        sim.loadMarkerParticleData(s.positions, s.velocities)
+        sim.initialize()
+        sim.set_launch_graphs(graphs)
+        sims.append(sim)
+    for _ in range(4):
+        st = [sim.update(1 / 480) for sim in sims]
+        assert st[0].pcg_iterations == st[1].pcg_iterations and st[0].pressure_ok == st[1].pressure_ok == 1
         for x, y in zip(sims[0].particles(), sims[1].particles()):
             assert bits_equal(x, y)
