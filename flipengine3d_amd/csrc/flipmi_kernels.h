@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <utility>
 
 namespace flipmi {
 
@@ -201,18 +202,22 @@ struct PressureBuffers {
     // the FP32 PCG vectors; x and the matrix stay FP64.
     float *invdiag32, *Lx32, *Ly32, *Lz32, *Lxm32, *Lym32, *Lzm32;
     float *r32, *z32, *s32;
-    // Mixed precision: the SpMV forms the new direction s = z + beta s from
-    // the old one, so s lives in two buffers: s32 is read, s32b written, and
-    // the host swaps them after each SpMV launch.  s_plain: the next SpMV
-    // reads s32 as it is (right after initialisation).
+    // The SpMV forms the new direction s = z + beta s from the old one, so s
+    // lives in two buffers: s (s32) is read, sb (s32b) written, and the host
+    // swaps them after each SpMV launch.  FP64: q = A s goes to the buffer
+    // that z, which the SpMV reads, is not in; the forward sweep replaces it
+    // there by its result, so the two are swapped as well.  s_plain: the next
+    // SpMV takes the first direction (s32, or z) as it is.
     float *s32b;
+    double *sb, *q;  // FP64 only (null with the FP32 arrays)
     int s_plain;
-    int s_turn;  // which of the two s32 is
+    int s_turn;  // which of the two buffers s is in
     void swap_directions() {
-        float *t = s32;
-        s32 = s32b;
-        s32b = t;
+        std::swap(s32, s32b);
         s_turn ^= 1;
+        if (!sb) return;
+        std::swap(s, sb);
+        std::swap(z, q);
     }
     float *q32;  // mixed precision: q = A s, read by the axpy
     double *partials;                   // per-block partial sums
@@ -257,9 +262,8 @@ hipError_t launch_mic0_factor(const GridGeom &g, const float *liquid, PressureBu
 // replacement (requires the FP32 arrays of pb).
 hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, bool mixed,
                            PressureBuffers &pb, hipStream_t s);
-// The kernels of one PCG iteration.  The FP64 path runs spmv, axpy,
-// forward, backward, update.  The mixed MIC(0) iteration folds the axpy into
-// the forward sweep and the direction update into the SpMV, and runs
+// The kernels of one PCG iteration.  The MIC(0) iterations run spmv (with the
+// direction update), forward (with the axpy) and backward; the mixed one runs
 // kPcgResidual (a true residual and a forward sweep over it) between the
 // forward and the backward sweep; it exits at once unless the forward sweep's
 // residual norm called for a true residual.  With multigrid
@@ -279,6 +283,8 @@ inline unsigned pcg_sweeps_per_iteration(bool mixed) { return mixed ? 3u : 2u; }
 struct KernelTiming {
     hipEvent_t start = nullptr, stop = nullptr;
 };
+// After the last FP64 iteration: completes x.  first_turn: pb.s_turn after launch_pcg_init.
+hipError_t launch_pcg_finish(PressureBuffers &pb, int first_turn, int iterations, hipStream_t s);
 // One iteration; the pieces with a start event in kt are timed.
 hipError_t launch_pcg_iteration(const GridGeom &g, bool mixed, PressureBuffers &pb, hipStream_t s,
                                 const KernelTiming (&kt)[kPcgPieces]);

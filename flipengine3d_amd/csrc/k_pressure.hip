@@ -32,12 +32,6 @@ namespace flipmi {
 
 constexpr int kTile = 8;
 constexpr int kRedBlocks = 1024;
-// The axpy's grid: fewer, longer-lived blocks stream its four arrays faster
-// (mixed axpy on the 256x128x128 double dam break: 20.6 us per launch with
-// 1024 blocks, 15.7 with 512, 15.0 with 384, 16.1 with 256).  Its reduction
-// is a maximum, so the grid does not change any result; the SpMV's is a sum
-// whose order follows the grid, so it keeps kRedBlocks.  A multiple of kXcds.
-constexpr int kAxpyBlocks = 384;
 constexpr int kRedThreads = 256;
 constexpr unsigned kSpinLimit = 1u << 20;  // ~1 s of polling: a legitimate wait is microseconds
 constexpr int kRecWords = 2;       // 64-bit words per tagged FP64 record
@@ -316,10 +310,11 @@ hipError_t launch_group_mask(PressureBuffers &pb, hipStream_t s) {
 enum { kFactor = 0, kForward = 1, kBackward = 2 };
 // A sweep launch's mode: what it reduces or decides at its end.  Nothing;
 // the z.r dot of the first or a later iteration (backward); the residual
-// norm of the axpy the forward sweep did; or (forward, a launch that runs
-// only when a true residual is due) the norm of the true residual it
-// computes before sweeping.
-enum { kDotNone = 0, kDotInit = 1, kDotIter = 2, kAxpyNorm = 3, kTrueResidual = 4 };
+// norm of the axpy the forward sweep did (FP32: whether a true residual is
+// due; FP64: the convergence test); or (forward, a launch that runs only when
+// a true residual is due) the norm of the true residual it computes before
+// sweeping.
+enum { kDotNone = 0, kDotInit = 1, kDotIter = 2, kAxpyNorm = 3, kTrueResidual = 4, kAxpyTest = 5 };
 
 // Values another workgroup reads within the same kernel are stored and
 // loaded as relaxed device-scope atomics, which are coherent across XCDs by
@@ -511,7 +506,7 @@ __device__ void finish_sweep(PressureBuffers &pb, int mode, double tile_acc, int
     const int lane = threadIdx.x & 63;
     const int ntiles = pb.sm.ntj * pb.sm.ntk;
     const bool dot = mode == kDotInit || mode == kDotIter;
-    const bool norm = mode == kAxpyNorm || mode == kTrueResidual;
+    const bool norm = mode == kAxpyNorm || mode == kTrueResidual || mode == kAxpyTest;
     if (dot || norm) {
         double part = dot ? wave_sum_fixed(tile_acc) : wave_max(tile_acc);
         if (lane == 0) st_dev(&pb.partials[tile], part);
@@ -544,6 +539,16 @@ __device__ void finish_sweep(PressureBuffers &pb, int mode, double tile_acc, int
                 sc->iters += 1;
                 if (m <= sc->tol || m < sc->delta * sc->rmax || sc->iters >= sc->maxiter) sc->refresh = 1;
                 else sc->resid = m;
+            } else if (mode == kAxpyTest) {
+                // |r|_inf after the axpy decides (pcgsolver.h:291).
+                sc->resid = m;
+                sc->iters += 1;
+                if (m <= sc->tol) {
+                    sc->converged = 1;
+                    sc->done = 1;
+                } else if (sc->iters >= sc->maxiter) {
+                    sc->done = 1;
+                }
             } else {
                 // |b - A x|_inf in FP64 decides convergence.
                 sc->resid = m;
@@ -886,6 +891,7 @@ struct SweepOps {
     const T *dotvec;   // backward: vector of the fused dot product, or null
     const T *inv;      // invdiag
     const T *c1, *c2, *c3;  // forward: Lzm, Lym, Lxm; backward: Lx, Ly, Lz
+    const T *q = nullptr;   // forward with the axpy: A s
 };
 
 template <class T>
@@ -1065,21 +1071,36 @@ __device__ void sweep_poller(PressureBuffers &pb, SweepMailbox<T> &mb, int tile,
     }
 }
 
+// The new direction s = z + beta s of the previous iteration
+// (pcgsolver.h:300-302), formed where the SpMV reads it.
+template <class T>
+struct NextDirection {
+    const T *__restrict__ z, *__restrict__ s;
+    float beta;
+    __device__ __forceinline__ T operator[](size_t q) const { return z[q] + beta * s[q]; }
+};
+template <class T>
+struct SameDirection {
+    const T *__restrict__ s;
+    __device__ __forceinline__ T operator[](size_t q) const { return s[q]; }
+};
+
 // y = A x at slot p of cell (i, j, k) (sparsematrix.h:187-216: row entries
 // in increasing column order).
-__device__ __forceinline__ double spmv_slot(const PressureBuffers &pb, double mf, const double *__restrict__ x,
-                                            size_t p, int i, int j, int k) {
+template <class Dir>
+__device__ __forceinline__ double spmv_slot_dir(const PressureBuffers &pb, double mf, const Dir &x, size_t p,
+                                                int i, int j, int k) {
     const SlotMap &sm = pb.sm;
     const unsigned pzm = sm.slot32(i, j, k - 1), pym = sm.slot32(i, j - 1, k), pxm = sm.slot32(i - 1, j, k);
     const unsigned pxp = sm.slot32(i + 1, j, k), pyp = sm.slot32(i, j + 1, k), pzp = sm.slot32(i, j, k + 1);
-    double s = 0;
-    s += coupling(pb.wz[pzm], mf) * x[pzm];
-    s += coupling(pb.wy[pym], mf) * x[pym];
-    s += coupling(pb.wx[pxm], mf) * x[pxm];
-    s += pb.diag[p] * x[p];
-    s += coupling(pb.wx[p], mf) * x[pxp];
-    s += coupling(pb.wy[p], mf) * x[pyp];
-    s += coupling(pb.wz[p], mf) * x[pzp];
+    double s = 0.0;
+    s += coupling(pb.wz[pzm], mf) * (double)x[pzm];
+    s += coupling(pb.wy[pym], mf) * (double)x[pym];
+    s += coupling(pb.wx[pxm], mf) * (double)x[pxm];
+    s += pb.diag[p] * (double)x[p];
+    s += coupling(pb.wx[p], mf) * (double)x[pxp];
+    s += coupling(pb.wy[p], mf) * (double)x[pyp];
+    s += coupling(pb.wz[p], mf) * (double)x[pzp];
     return s;
 }
 
@@ -1108,7 +1129,7 @@ __device__ double tile_true_residual(const GridGeom &g, const PressureBuffers &p
             p[u] = ok[u] ? tile0 + (size_t)gi * 256 + (size_t)(e & 255) : tile0;
             int i, j, k;
             in[u] = stencil_cell(g, pb.sm, p[u], i, j, k);
-            ax[u] = spmv_slot(pb, mf, pb.x, p[u], i, j, k);
+            ax[u] = spmv_slot_dir(pb, mf, SameDirection<double>{pb.x}, p[u], i, j, k);
             bs[u] = pb.rhs[p[u]];
         }
 #pragma unroll
@@ -1226,20 +1247,27 @@ __device__ void sweep_dot_wave(PressureBuffers &pb, SweepMailbox<float> &mb, con
     finish_sweep(pb, mode, acc, tile, false, mb.epoch + 1);
 }
 
-// AX (FP32 forward sweep of the mixed path only): the sweep also does the
-// iteration's axpy (pcgsolver.h:289-290).  The compute wave reads
-// r32 + (-alpha) q32 in place of r32 (off the step's dependency chain),
-// stores it back to r32 and takes its max norm; the third wave updates x
-// (sweep_x_wave).  Each value is rounded as a separate axpy pass would
-// round it, and the max is order-independent.
-// AUX (FP32 sweeps of the mixed path): a third wave helps, the axpy's x
-// update on the forward sweep (AX), the z.r dot on the backward one (DW).
+// AX (a forward sweep): the sweep also does the iteration's axpy
+// (pcgsolver.h:289-290).  The compute wave reads r + (-alpha) q in place of r
+// (off the step's dependency chain), stores it back to r and takes its max
+// norm; x follows in a third wave (FP32: sweep_x_wave) or in the next SpMV
+// (FP64).  Each value is rounded as a separate axpy pass would round it, and
+// the max is order-independent.
+// DW (the FP32 backward sweep of an iteration): a third wave takes the z.r dot.
+// AUX is AX on a forward sweep and DW on a backward one.
+//
+// What bounds the FP64 sweep: one tile alone takes 100 ns a march step (116
+// with the axpy), a hand-over to the next tile 16 steps and 1.3 us.  The
+// step's dependent chain is 52 ns of that; its 2.6 to 3 KB of operands come in
+// at the 25 to 30 bytes a nanosecond that one compute unit takes from beyond
+// its L2, and that is the bound: moving the record stores or the loads to
+// other waves of the workgroup, or two to four tiles into one, made it slower.
 template <class T, int DIR, int D, bool AUX = false>
 __global__ __launch_bounds__(256) void k_sweep(GridGeom g, PressureBuffers pb, SweepOps<T> op,
                                                           int mode) {
     constexpr int C = kChunk;
     constexpr bool FWD = DIR == kForward;
-    static_assert(!AUX || sizeof(T) == 4, "helper waves serve the FP32 sweeps only");
+    static_assert(!AUX || FWD || sizeof(T) == 4, "a dot wave serves the FP32 sweep only");
     constexpr bool AX = AUX && FWD, DW = AUX && !FWD;
     constexpr int NV = FWD ? (AX ? 6 : 5) : (DW ? 5 : 6);
     constexpr int RW = Record<T>::W;
@@ -1279,12 +1307,11 @@ __global__ __launch_bounds__(256) void k_sweep(GridGeom g, PressureBuffers pb, S
     }
     if (wave == 1)
         return sweep_poller<T, FWD>(pb, mb, tile, up_j, up_k, tb, nchunks, ubj, uej, ubk, uek, lane, gb);
-    if constexpr (AX)
+    if constexpr (AX && sizeof(T) == 4)
         if (wave == 2) return sweep_x_wave(pb, mb, tile, tb, te, lane, gb);
     if constexpr (DW)
         if (wave == 2) return sweep_dot_wave(pb, mb, op, tile, tb, nchunks, lane, gb, mode);
 
-    const int src_j = (FWD ? lane - 1 : lane + 1) & 63;  // neighbour lane along j
     const int src_k = (FWD ? lane - 8 : lane + 8) & 63;  // neighbour lane along k
     // Lane position in its 16-lane DPP row and the row that takes the
     // permlane32 result (lane_k).
@@ -1321,9 +1348,9 @@ __global__ __launch_bounds__(256) void k_sweep(GridGeom g, PressureBuffers pb, S
     const auto r_inv = buffer_view(op.inv + tile0, tile_bytes);
     const auto r_dot = buffer_view(dotsrc + tile0, tile_bytes);
     const auto r_out = buffer_view(op.out + tile0, tile_bytes);
-    // AX: the SpMV result q32 read beside r32, and r32 written back.
-    const auto r_q = buffer_view((AX ? (const T *)pb.q32 : op.c1) + tile0, tile_bytes);
-    const auto r_rw = buffer_view((AX ? (const T *)pb.r32 : op.out) + tile0, tile_bytes);
+    // AX: the SpMV's result q read beside r, and r written back.
+    const auto r_q = buffer_view((AX ? op.q : op.c1) + tile0, tile_bytes);
+    const auto r_rw = buffer_view((AX ? op.in : op.out) + tile0, tile_bytes);
     const T naf = AX ? T(-pb.sc->alpha_f) : T(0);
     T rmax = T(0);  // AX: max |r| over the tile's updated residual
     const unsigned vlane = (unsigned)lane * 4u * (unsigned)sizeof(T);
@@ -1437,32 +1464,36 @@ __global__ __launch_bounds__(256) void k_sweep(GridGeom g, PressureBuffers pb, S
     #pragma unroll
                     for (int s = 0; s < C; s++) {
                         // Values produced one step earlier by the neighbouring lanes.
-                        // FP32: DPP / permlane exchange; FP64: the LDS crossbar
-                        // (two dwords per value make the permlane route longer).
-                        T nj_cur, nk_cur;
-                        if constexpr (sizeof(T) == 4) {
-                            nj_cur = lane_j<FWD>(cur);
-                            nk_cur = lane_k<FWD>(cur, low_half, row_sel);
-                        } else {
-                            nj_cur = shfl_t(cur, src_j);
-                            nk_cur = shfl_t(cur, src_k);
-                        }
+                        // Along j a DPP row shift.  Along k the permlane route
+                        // for FP32; the LDS crossbar for FP64, where two
+                        // dwords make the permlane route longer (one tile of
+                        // 250 cells: 31 against 41 us).
+                        const T nj_cur = lane_j<FWD>(cur);
+                        T nk_cur;
+                        if constexpr (sizeof(T) == 4) nk_cur = lane_k<FWD>(cur, low_half, row_sel);
+                        else nk_cur = shfl_t(cur, src_k);
                         const T qy = edge_j ? evj[s] : nj_cur;
                         const T qz = edge_k ? evk[s] : nk_cur;
                         // AX: the updated residual r + (-alpha) q, off the
                         // step's dependency chain; fmaxf(m, |r|) is the
-                        // compare-and-keep maximum here (m is never NaN).
+                        // compare-and-keep maximum of the FP64 branch (m is
+                        // never NaN).
                         T bs = v[0][s];
                         if constexpr (AX) {
                             bs = v[0][s] + naf * v[NV - 1][s];
                             bv[s] = bs;
-                            rmax = fmaxf(rmax, fabsf(bs));
+                            if constexpr (sizeof(T) == 4) {
+                                rmax = fmaxf(rmax, fabsf(bs));
+                            } else {
+                                const T ab = fabs(bs);
+                                rmax = ab > rmax ? ab : rmax;
+                            }
                         }
                         // c1..c3 multiply the -z, -y, -x neighbours (forward) or
                         // the +x, +y, +z ones (backward).
                         T q;
                         if constexpr (sizeof(T) == 8) {
-                            q = FWD ? ref_step(v[0][s], v[1][s], qz, v[2][s], qy, v[3][s], cur, v[4][s])
+                            q = FWD ? ref_step(bs, v[1][s], qz, v[2][s], qy, v[3][s], cur, v[4][s])
                                     : ref_step(v[0][s], v[1][s], cur, v[2][s], qy, v[3][s], qz, v[4][s]);
                         } else {
                             q = FWD ? fused_step(bs, v[3][s], cur, v[2][s], qy, v[1][s], qz, v[4][s])
@@ -1491,7 +1522,7 @@ __global__ __launch_bounds__(256) void k_sweep(GridGeom g, PressureBuffers pb, S
         }
     }
     if constexpr (DW) return;  // the dot wave finishes the launch
-    const int fin = FWD ? (AX ? kAxpyNorm : (mode == kTrueResidual ? kTrueResidual : kDotNone))
+    const int fin = FWD ? (AX ? (sizeof(T) == 8 ? kAxpyTest : kAxpyNorm) : (mode == kTrueResidual ? kTrueResidual : kDotNone))
                         : (dot ? mode : kDotNone);
     finish_sweep(pb, fin, AX ? (double)rmax : (FWD ? tres_max : dot_acc), tile, false, epoch + 1);
 }
@@ -1536,12 +1567,9 @@ static hipError_t launch_sweep(int dir, const GridGeom &g, PressureBuffers &pb, 
     }
     int ntiles = pb.sm.ntj * pb.sm.ntk;
     constexpr int D = SweepDepth<T>::D;
-    if (mode == kAxpyNorm) {
-        if constexpr (sizeof(T) == 4) {
-            if (dir == kForward) return launch_on(k_sweep<T, kForward, D, true>, ntiles, 192, s, kt, g, pb, op, mode);
-        }
-        return hipErrorInvalidValue;
-    }
+    // With the axpy: FP32 has a third wave for x.
+    if (mode == kAxpyNorm || mode == kAxpyTest)
+        return launch_on(k_sweep<T, kForward, D, true>, ntiles, sizeof(T) == 4 ? 192 : 128, s, kt, g, pb, op, mode);
     // The forward sweep over a fresh true residual has four waves for the
     // residual; two of them then leave.
     if (dir == kForward)
@@ -1555,13 +1583,14 @@ static hipError_t launch_sweep(int dir, const GridGeom &g, PressureBuffers &pb, 
 }
 
 static SweepOps<double> fwd_ops64(PressureBuffers &pb, const double *r, double *z) {
-    return SweepOps<double>{r, z, nullptr, pb.invdiag, pb.Lzm, pb.Lym, pb.Lxm};
+    return SweepOps<double>{r, z, nullptr, pb.invdiag, pb.Lzm, pb.Lym, pb.Lxm, pb.z};
 }
 static SweepOps<double> bwd_ops64(PressureBuffers &pb, double *z, const double *dotvec) {
     return SweepOps<double>{nullptr, z, dotvec, pb.invdiag, pb.Lx, pb.Ly, pb.Lz};
 }
 static SweepOps<float> fwd_ops32(PressureBuffers &pb) {
-    return SweepOps<float>{pb.r32, pb.z32, nullptr, pb.invdiag32, pb.Lzm32, pb.Lym32, pb.Lxm32};
+    return SweepOps<float>{pb.r32, pb.z32, nullptr, pb.invdiag32, pb.Lzm32, pb.Lym32, pb.Lxm32,
+                           pb.q32};
 }
 static SweepOps<float> bwd_ops32(PressureBuffers &pb) {
     return SweepOps<float>{nullptr, pb.z32, pb.r32, pb.invdiag32, pb.Lx32, pb.Ly32, pb.Lz32};
@@ -1638,35 +1667,58 @@ __device__ bool last_block(unsigned *counter, unsigned (*groups)[32]) {
     return is_last;
 }
 
-// z = A s and alpha = rho / (s . z), alpha rounded to float as the
-// reference's BLAS::addScaled takes it (blaswrapper.h:135-158).
-__global__ __launch_bounds__(kRedThreads) void k_spmv_dot(GridGeom g, PressureBuffers pb) {
-    __shared__ double sh[kRedThreads / 64];
-    if (pb.sc->done) return;
+// FP64 iteration, first launch.  sb = s = z + beta s (pcgsolver.h:300-302; z
+// itself on a solve's first iteration), q = A s and alpha = rho / (s . q),
+// alpha rounded to float as the reference's BLAS::addScaled takes it
+// (blaswrapper.h:135-158); and the previous iteration's x += alpha s
+// (pcgsolver.h:290), whose s this launch reads anyway.  z and s are only
+// read, so the stencil reads race with no write.  Every value is rounded as
+// passes of their own over s and x would round it, and the dot keeps its
+// order.  Passes of their own (direction update 3.7 us, axpy 4.6 us per
+// iteration at 64^3, where launches and not bytes count) read z, s and x
+// once more each.
+template <class Dir>
+__device__ __forceinline__ double spmv_dot_body(const GridGeom &g, const PressureBuffers &pb, const Dir &dir,
+                                                bool update_x) {
     double acc = 0.0;
     const ListRange lr = xcd_list(*pb.active_count);
     const double mf = pb.sc->mf;  // coupling scale of the assembled system
+    const float af = pb.sc->alpha_f;  // the previous iteration's
     constexpr int U = 2;
     for (int e0 = lr.begin; e0 < lr.end; e0 += U * lr.step) {
         size_t p[U];
         bool ok[U], in[U];
-        double zc[U], sp[U];
+        double zc[U], sp[U], xs[U], so[U];
         list_slots<U>(pb, lr, e0, p, ok);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             int i, j, k;
             in[u] = stencil_cell(g, pb.sm, p[u], i, j, k);
-            zc[u] = spmv_slot(pb, mf, pb.s, p[u], i, j, k);
-            sp[u] = pb.s[p[u]];
+            zc[u] = spmv_slot_dir(pb, mf, dir, p[u], i, j, k);
+            sp[u] = dir[p[u]];
+            if (update_x) {  // uniform
+                xs[u] = pb.x[p[u]];
+                so[u] = pb.s[p[u]];
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (!ok[u]) continue;  // uniform
-            const double z = in[u] ? zc[u] : 0.0;
-            pb.z[p[u]] = z;
-            acc += sp[u] * z;
+            const double q = in[u] ? zc[u] : 0.0;
+            pb.q[p[u]] = q;
+            pb.sb[p[u]] = sp[u];
+            if (update_x) pb.x[p[u]] = xs[u] + af * so[u];
+            acc += sp[u] * q;
         }
     }
+    return acc;
+}
+
+__global__ __launch_bounds__(kRedThreads) void k_spmv_dot(GridGeom g, PressureBuffers pb) {
+    __shared__ double sh[kRedThreads / 64];
+    if (pb.sc->done) return;
+    double acc = pb.s_plain ? spmv_dot_body(g, pb, SameDirection<double>{pb.z}, false)
+                            : spmv_dot_body(g, pb, NextDirection<double>{pb.z, pb.s, pb.sc->beta_f}, true);
     double bs = block_reduce<0>(acc, sh);
     if (threadIdx.x == 0) st_dev(&pb.partials[blockIdx.x], bs);
     if (!last_block(&pb.sc->counter[1], pb.sc->group_counter[0])) return;
@@ -1683,81 +1735,22 @@ __global__ __launch_bounds__(kRedThreads) void k_spmv_dot(GridGeom g, PressureBu
     }
 }
 
-// x += alpha s, r -= alpha z, resid = |r|_inf; convergence test
-// (pcgsolver.h:280-291).
-__global__ __launch_bounds__(kRedThreads) void k_axpy_norm(GridGeom g, PressureBuffers pb) {
-    __shared__ double sh[kRedThreads / 64];
-    if (pb.sc->done) return;
-    float af = pb.sc->alpha_f;
-    float naf = (float)(-pb.sc->alpha);
-    double mx = 0.0;
+// The last iteration's x += alpha s, which no SpMV follows.
+__global__ __launch_bounds__(kRedThreads) void k_last_x(PressureBuffers pb, const double *__restrict__ s) {
+    if (pb.sc->iters == 0) return;
+    const float af = pb.sc->alpha_f;
     const ListRange lr = xcd_list(*pb.active_count);
-    constexpr int U = 4;
-    for (int e0 = lr.begin; e0 < lr.end; e0 += U * lr.step) {
-        size_t p[U];
-        bool ok[U];
-        double xs[U], ss[U], rs[U], zs[U];
-        list_slots<U>(pb, lr, e0, p, ok);
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            xs[u] = pb.x[p[u]]; ss[u] = pb.s[p[u]];
-            rs[u] = pb.r[p[u]]; zs[u] = pb.z[p[u]];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (!ok[u]) continue;  // uniform
-            pb.x[p[u]] = xs[u] + af * ss[u];
-            const double r = rs[u] + naf * zs[u];
-            pb.r[p[u]] = r;
-            const double a = fabs(r);
-            mx = a > mx ? a : mx;
-        }
-    }
-    double bm = block_reduce<1>(mx, sh);
-    if (threadIdx.x == 0) st_dev(&pb.partials[kRedBlocks + blockIdx.x], bm);
-    if (!last_block(&pb.sc->counter[2], pb.sc->group_counter[1])) return;
-    double m = 0.0;
-    for (int q = threadIdx.x; q < (int)gridDim.x; q += kRedThreads) {
-        double v = ld_dev(&pb.partials[kRedBlocks + q]);
-        m = v > m ? v : m;
-    }
-    m = block_reduce<1>(m, sh);
-    if (threadIdx.x == 0) {
-        PcgScalars *sc = pb.sc;
-        sc->resid = m;
-        sc->iters += 1;
-        if (m <= sc->tol) {
-            sc->converged = 1;
-            sc->done = 1;
-        } else if (sc->iters >= sc->maxiter) {
-            sc->done = 1;
-        }
-        sc->counter[2] = 0;
+    for (int e = lr.begin; e < lr.end; e += lr.step) {
+        const size_t p = ((size_t)pb.active_list[e] << 8) + threadIdx.x;
+        pb.x[p] = pb.x[p] + af * s[p];
     }
 }
 
-// s = z + beta s (pcgsolver.h:295-296), or s = z on the first application.
-__global__ __launch_bounds__(kRedThreads) void k_update_s(GridGeom g, PressureBuffers pb, int first) {
-    if (pb.sc->done) return;
-    float bf = first ? 0.0f : pb.sc->beta_f;
-    const ListRange lr = xcd_list(*pb.active_count);
-    constexpr int U = 4;
-    for (int e0 = lr.begin; e0 < lr.end; e0 += U * lr.step) {
-        size_t p[U];
-        bool ok[U];
-        double zs[U], ss[U];
-        list_slots<U>(pb, lr, e0, p, ok);
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            zs[u] = pb.z[p[u]];
-            ss[u] = pb.s[p[u]];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (!ok[u]) continue;  // uniform
-            pb.s[p[u]] = first ? zs[u] : zs[u] + bf * ss[u];
-        }
-    }
+hipError_t launch_pcg_finish(PressureBuffers &pb, int first_turn, int iterations, hipStream_t s) {
+    // Iteration n wrote its direction to the buffer of turn first_turn ^ (n & 1).
+    const bool current = pb.s_turn == (first_turn ^ (iterations & 1));
+    k_last_x<<<kRedBlocks, kRedThreads, 0, s>>>(pb, current ? pb.s : pb.sb);
+    return hipGetLastError();
 }
 
 // x = 0, r = b; scalars for a new solve.
@@ -1768,7 +1761,9 @@ __global__ void k_pcg_init_vectors(GridGeom g, PressureBuffers pb) {
         pb.x[p] = 0.0;
         pb.r[p] = pb.rhs[p];
         pb.z[p] = 0.0;
+        pb.q[p] = 0.0;
         pb.s[p] = 0.0;
+        pb.sb[p] = 0.0;
     }
 }
 
@@ -1986,35 +1981,6 @@ __global__ void k_pcg_init_vectors32(PressureBuffers pb) {
 // rounding costs about 9 % more iterations on the workloads here: 126
 // against 115), rebuilt from the FP32 face weights, FP32 s, FP64 sums,
 // rounded once.
-// The new direction s = z + beta s of the previous iteration
-// (pcgsolver.h:300-302), formed where the SpMV reads it.
-struct NextDirection {
-    const float *__restrict__ z, *__restrict__ s;
-    float beta;
-    __device__ __forceinline__ float operator[](size_t q) const { return z[q] + beta * s[q]; }
-};
-struct SameDirection {
-    const float *__restrict__ s;
-    __device__ __forceinline__ float operator[](size_t q) const { return s[q]; }
-};
-
-template <class Dir>
-__device__ __forceinline__ double spmv_slot_dir(const PressureBuffers &pb, double mf, const Dir &x, size_t p,
-                                                int i, int j, int k) {
-    const SlotMap &sm = pb.sm;
-    const unsigned pzm = sm.slot32(i, j, k - 1), pym = sm.slot32(i, j - 1, k), pxm = sm.slot32(i - 1, j, k);
-    const unsigned pxp = sm.slot32(i + 1, j, k), pyp = sm.slot32(i, j + 1, k), pzp = sm.slot32(i, j, k + 1);
-    double s = 0.0;
-    s += coupling(pb.wz[pzm], mf) * (double)x[pzm];
-    s += coupling(pb.wy[pym], mf) * (double)x[pym];
-    s += coupling(pb.wx[pxm], mf) * (double)x[pxm];
-    s += pb.diag[p] * (double)x[p];
-    s += coupling(pb.wx[p], mf) * (double)x[pxp];
-    s += coupling(pb.wy[p], mf) * (double)x[pyp];
-    s += coupling(pb.wz[p], mf) * (double)x[pzp];
-    return s;
-}
-
 // s32b = z32 + beta s32 (or s32 as it is), q32 = A s32b and alpha = rho /
 // (s . q) with an FP64 dot.  z32 and s32 are only read, so the stencil
 // reads race with no write.
@@ -2052,8 +2018,8 @@ __device__ __forceinline__ double spmv_dot32_body(const GridGeom &g, const Press
 __global__ __launch_bounds__(kRedThreads) void k_spmv_dot32(GridGeom g, PressureBuffers pb) {
     __shared__ double sh[kRedThreads / 64];
     if (pb.sc->done) return;
-    double acc = pb.s_plain ? spmv_dot32_body(g, pb, SameDirection{pb.s32})
-                            : spmv_dot32_body(g, pb, NextDirection{pb.z32, pb.s32, pb.sc->beta_f});
+    double acc = pb.s_plain ? spmv_dot32_body(g, pb, SameDirection<float>{pb.s32})
+                            : spmv_dot32_body(g, pb, NextDirection<float>{pb.z32, pb.s32, pb.sc->beta_f});
     double bs = block_reduce<0>(acc, sh);
     if (threadIdx.x == 0) st_dev(&pb.partials[blockIdx.x], bs);
     if (!last_block(&pb.sc->counter[1], pb.sc->group_counter[0])) return;
@@ -2116,20 +2082,20 @@ hipError_t launch_pcg_init(const GridGeom &g, double tolf, int maxiter, bool mix
     }
     k_pcg_init_vectors<<<kRedBlocks, kRedThreads, 0, s>>>(g, pb);
     k_pcg_init_scalars<<<1, 1, 0, s>>>(pb, tolf, maxiter);
-    // z = M^-1 r, rho = z . r, s = z (pcgsolver.h:270-279).
+    // z = M^-1 r, rho = z . r; the first SpMV takes s = z (pcgsolver.h:270-279).
     hipError_t e = launch_sweep(kForward, g, pb, fwd_ops64(pb, pb.r, pb.z), kDotNone, s);
     if (e != hipSuccess) return e;
     e = launch_sweep(kBackward, g, pb, bwd_ops64(pb, pb.z, pb.r), kDotInit, s);
     if (e != hipSuccess) return e;
-    k_update_s<<<kRedBlocks, kRedThreads, 0, s>>>(g, pb, 1);
+    pb.s_plain = 1;
     return hipGetLastError();
 }
 
-// Mixed precision folds the axpy into the forward sweep and the direction
-// update into the next SpMV; the FP64 path has no true-residual step.
+// The axpy is folded into the forward sweep and the direction update into the
+// next SpMV; the FP64 path has no true-residual step.
 bool pcg_piece_used(int piece, bool mixed) {
-    if (mixed) return piece != kPcgUpdate && piece != kPcgAxpy;
-    return piece != kPcgResidual;
+    if (piece == kPcgUpdate || piece == kPcgAxpy) return false;
+    return mixed || piece != kPcgResidual;
 }
 
 static hipError_t launch_pcg_piece(int piece, const GridGeom &g, bool mixed, PressureBuffers &pb,
@@ -2155,12 +2121,16 @@ static hipError_t launch_pcg_piece(int piece, const GridGeom &g, bool mixed, Pre
         }
     }
     switch (piece) {
-        case kPcgSpmv: return launch_on(k_spmv_dot, rg, rb, s, kt, g, pb);
-        case kPcgAxpy: return launch_on(k_axpy_norm, dim3(kAxpyBlocks), rb, s, kt, g, pb);
-        case kPcgForward: return launch_sweep(kForward, g, pb, fwd_ops64(pb, pb.r, pb.z), kDotNone, s, kt);
+        case kPcgSpmv: {
+            hipError_t e = launch_on(k_spmv_dot, rg, rb, s, kt, g, pb);
+            // From here on s is the new direction and z holds q, which the
+            // forward sweep reads and overwrites with its result.
+            pb.swap_directions();
+            pb.s_plain = 0;
+            return e;
+        }
+        case kPcgForward: return launch_sweep(kForward, g, pb, fwd_ops64(pb, pb.r, pb.z), kAxpyTest, s, kt);
         case kPcgBackward: return launch_sweep(kBackward, g, pb, bwd_ops64(pb, pb.z, pb.r), kDotIter, s, kt);
-        case kPcgUpdate: return launch_on(k_update_s, rg, rb, s, kt, g, pb, 0);
-        case kPcgResidual: return hipSuccess;
         default: return hipErrorInvalidValue;
     }
 }
@@ -2188,7 +2158,7 @@ __global__ void k_spmv_plain(GridGeom g, PressureBuffers pb, const double *__res
          p += (size_t)gridDim.x * blockDim.x) {
         int i, j, k;
         decode_slot(pb.sm, p, i, j, k);
-        y[p] = interior(g, i, j, k) ? spmv_slot(pb, mf, x, p, i, j, k) : 0.0;
+        y[p] = interior(g, i, j, k) ? spmv_slot_dir(pb, mf, SameDirection<double>{x}, p, i, j, k) : 0.0;
     }
 }
 

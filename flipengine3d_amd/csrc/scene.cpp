@@ -113,6 +113,7 @@ size_t PressureStore::device_bytes() const {
     size_t b = edge.bytes() + mask.bytes() + progress.bytes() + ticket.bytes() + irange.bytes() + scal.bytes() +
                alist.bytes();
     for (int q = 0; q <= kSlotArrays; q++) b += arr[q].bytes();
+    for (int q = 0; q < 2; q++) b += arr64[q].bytes();
     for (int q = 0; q < kWeightArrays; q++) b += wgt[q].bytes();
     for (int q = 0; q < kSlotArrays32; q++) b += arr32[q].bytes();
     for (int q = 0; q < 6; q++) b += mg_f64[q].bytes();
@@ -203,6 +204,17 @@ void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s, bool mixed) {
     pb.Lxm = arr[10].p; pb.Lym = arr[11].p; pb.Lzm = arr[12].p;
     pb.wx = wgt[0].p; pb.wy = wgt[1].p; pb.wz = wgt[2].p;
     pb.partials = arr[kSlotArrays].p;
+    pb.sb = pb.q = nullptr;
+    pb.s_turn = 0;
+    if (!mixed) {
+        for (int q = 0; q < 2; q++) {
+            if (arr64[q].alloc(ns) != hipSuccess)
+                throw StatusError{FLIPMI_ERR_OOM, "pressure arrays: out of device memory"};
+            (void)launch_fill_f64(arr64[q].p, ns, 0.0, s);
+        }
+        pb.sb = arr64[0].p;
+        pb.q = arr64[1].p;
+    }
     if (mixed) {
         for (int q = 0; q < kSlotArrays32; q++) {
             if (arr32[q].alloc(ns) != hipSuccess)
@@ -278,6 +290,22 @@ static int iterations_needed(double before, double now, int iterations, double t
     const double rate = std::log(now / before) / iterations;  // < 0
     const double need = std::log(target / now) / rate;
     return need > 0 && need < 1e6 ? (int)std::ceil(need) : -1;
+}
+
+// Iterations to enqueue when the observed rate needs `need` more.  The rate
+// varies along a solve, and a look at the scalars between two batches costs
+// about three iterations launched for nothing: most of a long way at once,
+// and the last few with one to spare.  (The whole of it plus two launched 219
+// iterations for 135 in three solves of a 64^3 dam break.)  Few sizes, as each
+// is a captured graph.
+static int next_batch(int need) {
+    static const int kSizes[] = {2, 3, 4, 6, 8, 12, 16, 24, 32, 48};
+    const int want = need > 8 ? need * 3 / 4 : need + 1;
+    int size = kSizes[0];
+    for (int c : kSizes) {
+        if (need > 8 ? c <= want : size < want) size = c;
+    }
+    return size;
 }
 
 // Events for the selected kernels of an iteration at profiling level 2.
@@ -426,16 +454,16 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
     }
     if (prof) prof->begin_stage(FLIPMI_STAGE_MIC0, &ev);
     const bool mixed = w.precision == FLIPMI_PCG_MIXED;
-    if (mixed && !pb.r32) throw StatusError{FLIPMI_ERR_INVALID_ARG, "mixed precision arrays not allocated"};
+    if (mixed ? !pb.r32 : !pb.sb)
+        throw StatusError{FLIPMI_ERR_INVALID_ARG, "arrays of this precision not allocated"};
     hip_check(launch_group_mask(pb, s), "group mask");
     hip_check(launch_mic0_factor(w.g, w.liquid, pb, s), "mic0 factor");
     hip_check(launch_pcg_init(w.g, w.tol, w.maxiter, mixed, pb, s), "pcg init");
     if (prof) prof->end_stage(FLIPMI_STAGE_MIC0, ev);
     if (prof) prof->begin_stage(FLIPMI_STAGE_PCG, &ev);
     // Iterations are enqueued in batches between host checks of the device
-    // scalars.  After the first batch, the batch size is the number of
-    // iterations the observed convergence rate still needs (plus a margin),
-    // so few launches are wasted past convergence.
+    // scalars; next_batch sizes them.
+    const int first_turn = pb.s_turn;
     int batch = 8;
     int launched = 0;
     int prev_iters = 0;
@@ -463,7 +491,7 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
         };
         if (use_graph)
             launch_pcg_batch_graph(*w.graphs, batch, pb.s_turn, s, all, [&] {
-                if (mixed && (batch & 1)) pb.swap_directions();
+                if (batch & 1) pb.swap_directions();
                 pb.epoch += sweeps;
             });
         else
@@ -476,11 +504,11 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
         if (launched > w.maxiter + 16)
             throw StatusError{FLIPMI_ERR_HIP, "pcg did not terminate within its iteration cap"};
         const int need = iterations_needed(prev_resid, hs->resid, hs->iters - prev_iters, target);
-        const int next = need > 0 ? need + 2 : std::min(batch * 2, 32);
         prev_iters = hs->iters;
         prev_resid = hs->resid;
-        batch = std::max(2, std::min(next, 64));
+        batch = next_batch(need > 0 ? need : batch * 2);
     }
+    if (!mixed) hip_check(launch_pcg_finish(pb, first_turn, hs->iters, s), "pcg finish");
     if (prof) prof->end_stage(FLIPMI_STAGE_PCG, ev);
     if (prof) prof->stage_calls[FLIPMI_STAGE_PCG_ITERS] += hs->iters;
     out.iterations = hs->failed ? 0 : hs->iters;
@@ -789,6 +817,7 @@ size_t estimate_scene_bytes(const flipmi_scene_desc &d, int64_t cap) {
     size_t slots = sizeof(double) * (PressureStore::kSlotArrays * ns + 2 * 2048 + ntiles);
     slots += sizeof(float) * PressureStore::kWeightArrays * ns;
     if (d.pcg_precision == FLIPMI_PCG_MIXED) slots += sizeof(float) * PressureStore::kSlotArrays32 * ns;
+    else slots += sizeof(double) * 2 * ns;
     slots += sizeof(unsigned long long) * edge_record_count(sm);
     slots += sizeof(unsigned long long) * ntiles * (size_t)((sm.S / 4 + 63) / 64);
     slots += sizeof(unsigned) * (ntiles + 1) + sizeof(int) * 2 * ntiles + sizeof(PcgScalars);

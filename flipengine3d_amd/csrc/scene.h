@@ -308,6 +308,7 @@ struct PressureStore {
     static constexpr int kWeightArrays = 3;
     static constexpr int kSlotArrays32 = 12;  // FP32 factor and vectors, s twice, q (mixed precision)
     DBuf<double> arr[kSlotArrays + 1];
+    DBuf<double> arr64[2];        // FP64 iteration only: the second direction buffer, q
     DBuf<float> wgt[kWeightArrays];
     DBuf<float> arr32[kSlotArrays32];
     DBuf<unsigned long long> edge, mask;
