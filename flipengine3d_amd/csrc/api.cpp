@@ -668,8 +668,9 @@ int flipmi_extrapolate(flipmi_ctx *ctx, int ni, int nj, int nk, float *grid, con
         DBuf<uint8_t> dv, st;
         upload(dg, grid, n, s);
         upload(dv, valid, n, s);
-        alloc_dev(st, n);
-        hipck(launch_extrapolate(ni, nj, nk, dg.p, dv.p, st.p, layers, s), "extrapolate");
+        alloc_dev(st, extrapolate_status_bytes(n));
+        const ExtrapolateField field{ni, nj, nk, dg.p, dv.p, st.p + kExtrapolatePad};
+        hipck(launch_extrapolate(&field, 1, layers, s), "extrapolate");
         download(ctx->c, grid, dg, n, s);
     });
 }

@@ -107,8 +107,17 @@ inline size_t p2g_face_count(const GridGeom &g) {
 }
 
 // ---- grid passes (k_grid.hip) ----
-hipError_t launch_extrapolate(int ni, int nj, int nk, float *grid, const uint8_t *valid,
-                              uint8_t *status, int layers, hipStream_t s);
+// Up to three fields, each with a status buffer of extrapolate_status_bytes of
+// its faces: status points kExtrapolatePad bytes into it, at a multiple of 4.
+constexpr size_t kExtrapolatePad = 16;
+inline size_t extrapolate_status_bytes(size_t faces) { return (faces + 2 * kExtrapolatePad + 255) / 256 * 256; }
+struct ExtrapolateField {
+    int ni, nj, nk;
+    float *grid;
+    const uint8_t *valid;
+    uint8_t *status;
+};
+hipError_t launch_extrapolate(const ExtrapolateField *fields, int count, int layers, hipStream_t s);
 // Looks up the device address of the no-allocation scratch array on
 // `device` (current) once; noalloc.hip.
 hipError_t noalloc_scratch_init(int device);

@@ -25,7 +25,7 @@ namespace flipmi {
 constexpr size_t kNoallocScratchBytes = FLIPMI_NOALLOC_SCRATCH_BYTES;
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) uint8_t scratch[kNoallocScratchBytes];
+static __device__ __align__(256) uint8_t scratch[kNoallocScratchBytes + 2 * kExtrapolatePad];
 
 namespace {
 std::mutex g_scratch_mutex;
@@ -79,7 +79,8 @@ extern "C" int flipmi_extrapolate_noalloc(flipmi_ctx *ctx, int ni, int nj, int n
     hipError_t e = hipSetDevice(c.device);
     if (e == hipSuccess) {
         hipStream_t s = stream ? (hipStream_t)stream : c.stream;
-        e = launch_extrapolate(ni, nj, nk, grid_dev, valid_dev, status, layers, s);
+        const ExtrapolateField field{ni, nj, nk, grid_dev, valid_dev, status + kExtrapolatePad};
+        e = launch_extrapolate(&field, 1, layers, s);
     }
     if (e != hipSuccess) {
         c.last_error = std::string("flipmi_extrapolate_noalloc: ") + hipGetErrorString(e);

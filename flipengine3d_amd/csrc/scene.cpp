@@ -640,7 +640,7 @@ void Scene::alloc_all() {
     need(u.alloc(nU)); need(v.alloc(nV)); need(w.alloc(nW));
     need(su.alloc(nU)); need(sv.alloc(nV)); need(sw.alloc(nW));
     need(vu.alloc(nU)); need(vv.alloc(nV)); need(vw.alloc(nW));
-    need(status.alloc(nf));
+    need(status.alloc(3 * extrapolate_status_bytes(nf)));
     press = new PressureStore();
     press->alloc(g, stream, desc.pcg_precision == FLIPMI_PCG_MIXED, nc >= kMultigridCells);
     check(hipHostMalloc(&host_stage, kPressureStaging, hipHostMallocDefault), "pinned staging");
@@ -811,7 +811,7 @@ size_t estimate_scene_bytes(const flipmi_scene_desc &d, int64_t cap) {
     const size_t nci = (size_t)std::ceil((double)I * dx / (3 * dx)), ncj = (size_t)std::ceil((double)J * dx / (3 * dx)),
                  nck = (size_t)std::ceil((double)K * dx / (3 * dx));
     b += 2 * nci * ncj * nck;
-    b += sizeof(float) * nc + sizeof(float) * 2 * (nU + nV + nW) + (nU + nV + nW) + nf;
+    b += sizeof(float) * nc + sizeof(float) * 2 * (nU + nV + nW) + (nU + nV + nW) + 3 * extrapolate_status_bytes(nf);
     SlotMap sm = make_slot_map(d.isize, d.jsize, d.ksize);
     const size_t ns = sm.alloc_count(), ntiles = (size_t)sm.ntj * sm.ntk;
     size_t slots = sizeof(double) * (PressureStore::kSlotArrays * ns + 2 * 2048 + ntiles);
@@ -906,9 +906,12 @@ void Scene::build_mesh() {
 void Scene::extrapolate_all(int layers) {
     hipEvent_t ev = nullptr;
     begin_stage(FLIPMI_STAGE_EXTRAPOLATE, &ev);
-    check(launch_extrapolate(g.I + 1, g.J, g.K, u.p, vu.p, status.p, layers, stream), "extrapolate");
-    check(launch_extrapolate(g.I, g.J + 1, g.K, v.p, vv.p, status.p, layers, stream), "extrapolate");
-    check(launch_extrapolate(g.I, g.J, g.K + 1, w.p, vw.p, status.p, layers, stream), "extrapolate");
+    const size_t stride = status.n / 3;
+    uint8_t *const st = status.p + kExtrapolatePad;
+    const ExtrapolateField fields[3] = {{g.I + 1, g.J, g.K, u.p, vu.p, st},
+                                        {g.I, g.J + 1, g.K, v.p, vv.p, st + stride},
+                                        {g.I, g.J, g.K + 1, w.p, vw.p, st + 2 * stride}};
+    check(launch_extrapolate(fields, 3, layers, stream), "extrapolate");
     end_stage(FLIPMI_STAGE_EXTRAPOLATE, ev);
 }
 
