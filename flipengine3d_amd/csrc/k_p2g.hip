@@ -323,8 +323,11 @@ inline TileMap make_tile_map(const GridGeom &g) {
     return m;
 }
 
-// This block's face, or false when its lane has none.
-__device__ __forceinline__ bool tile_face(const GridGeom &g, const TileMap &m, int &comp, size_t &f) {
+// This block's face, or false when its lane has none; its tile's first face in
+// i0, j0, k (comp < 0: no tile).
+__device__ __forceinline__ bool tile_face(const GridGeom &g, const TileMap &m, int &comp, size_t &f, int &i0, int &j0,
+                                          int &k) {
+    comp = -1;
     const unsigned b = blockIdx.x;
     const unsigned tile = (b & 7u) * (m.nblocks >> 3) + (b >> 3);
     if (tile >= m.ntiles) return false;
@@ -332,13 +335,31 @@ __device__ __forceinline__ bool tile_face(const GridGeom &g, const TileMap &m, i
     int local = (int)(tile % (unsigned)m.per_group);
     comp = local < m.ntc[0] ? 0 : (local < m.ntc[0] + m.ntc[1] ? 1 : 2);
     local -= comp == 0 ? 0 : (comp == 1 ? m.ntc[0] : m.ntc[0] + m.ntc[1]);
-    const int jp = group % m.njp, k = group / m.njp;
-    const int i = local * 32 + (int)(threadIdx.x & 31), j = 2 * jp + (int)(threadIdx.x >> 5);
+    k = group / m.njp;
+    i0 = local * 32;
+    j0 = 2 * (group % m.njp);
+    const int i = i0 + (int)(threadIdx.x & 31), j = j0 + (int)(threadIdx.x >> 5);
     int ni, nj, nk;
     face_dims(g, comp, ni, nj, nk);
     if (i >= ni || j >= nj || k >= nk) return false;
     f = (size_t)i + (size_t)ni * ((size_t)j + (size_t)nj * (size_t)k);
     return true;
+}
+
+// Whether any face of the tile has candidates: one of the tile's 6 x 4 rows of
+// half-cells, a lane each, holds a particle.  Tiles of air are most of many
+// scenes, and end here with zeros instead of walking 16 empty rows a face.
+__device__ __forceinline__ bool tile_has_particles(const P2GArgs &a, int comp, int i0, int j0, int k) {
+    const int lane = threadIdx.x;
+    const int NI = 2 * a.g.I, NJ = 2 * a.g.J, NK = 2 * a.g.K;
+    const int sy = 2 * j0 + (comp != 1) - 2 + lane % 6, sz = 2 * k + (comp != 2) - 2 + lane / 6;
+    bool any = false;
+    if (lane < 24 && sy >= 0 && sz >= 0 && sy < NJ && sz < NK) {
+        const size_t row = (size_t)NI * ((size_t)sy + (size_t)NJ * (size_t)sz);
+        const int b = max(2 * i0 + (comp != 0) - 2, 0), e = min(2 * (i0 + 31) + (comp != 0) + 2, NI);
+        any = b < e && a.sub_offset[row + (size_t)b] < a.sub_offset[row + (size_t)e];
+    }
+    return __ballot(any) != 0ull;
 }
 
 template <class Key>
@@ -349,7 +370,16 @@ __global__ __launch_bounds__(kThreads) void k_p2g(P2GArgs a, TileMap tm) {
     __shared__ float s_w[kCap + 1][kThreads];
     int comp = 0;
     size_t f = 0;
-    const bool active = tile_face(a.g, tm, comp, f);
+    int i0 = 0, j0 = 0, k0 = 0;
+    const bool active = tile_face(a.g, tm, comp, f, i0, j0, k0);
+    if (comp < 0) return;  // uniform
+    if (!tile_has_particles(a, comp, i0, j0, k0)) {
+        if (active) {
+            a.out[comp][f] = 0.0f;
+            a.valid[comp][f] = 0;
+        }
+        return;
+    }
     const int t = threadIdx.x;
     FaceCtx c;
     int nh = 0, dropped = 0;
