@@ -78,8 +78,11 @@ TRUE_RESIDUAL_BYTES = 40 + 24
 # The coarser levels repeat restriction, correction and the smoothings (24
 # before, 28 after) on an eighth of the rows each time.  The true residual
 # reads x, b and the matrix and writes r: 8 + 8 + 20 + 8.
+# The FP64 iteration forms the direction in the SpMV, which also brings x up to
+# date (z, old s, new s, q, matrix, x r/w), and does the rest of the axpy in the
+# forward sweep (r r/w, q, factor, z).
 KERNEL_BYTES = {
-    "fp64": PCG_BYTES["fp64"],
+    "fp64": {"k_spmv_dot": 68, "k_axpy_norm": 0, "k_forward": 64, "k_backward": 56, "k_update_s": 0},
     "mixed_mic0": PCG_BYTES["mixed"],
     "mixed": {"k_spmv_dot": 40, "k_axpy_norm": 68, "k_forward": 24.5, "k_backward": 36, "k_update_s": 28.5},
 }
