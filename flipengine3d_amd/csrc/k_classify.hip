@@ -13,6 +13,7 @@
 // The result is bit-identical to the reference.
 #include "device_math.h"
 #include "flipmi_kernels.h"
+#include "half_cell_rows.h"
 
 namespace flipmi {
 
@@ -194,34 +195,9 @@ __global__ __launch_bounds__(kSdfThreads) void k_liquid_sdf(
 // 37x22x30 (8 k cells): 841 -> 62 us.  Bound by the latency of the dependent
 // loads (half-cell offsets, then particles), so no LDS limits the wavefronts
 // in flight.
-constexpr int kCellRows = 100;                 // 10 x 10 rows of half-cells around a cell
 constexpr int kTileI = 16, kTileJ = 4, kTileK = 4;  // cells of a workgroup
 static_assert(kTileI * kTileJ * kTileK == kSdfThreads, "one thread per cell");
-static_assert(kCellRows % 4 == 0, "rows are walked four at a time");
 static_assert(4 * (kTileJ + 4) * (kTileK + 4) == kSdfThreads, "one half-cell row per thread");
-
-// Rows (oy, oz), half-cells relative to the cell's first, by their distance
-// from the cell's centre: half-cells 0 and 1 touch it, -1 and 2 lie half a
-// cell away, and so on to two cells (ring 4).
-struct CellRow {
-    signed char oy, oz, ry, rz;  // offsets and rings
-};
-struct CellRows {
-    CellRow r[kCellRows];
-};
-constexpr CellRows make_cell_rows() {
-    CellRows t{};
-    int n = 0;
-    for (int d = 0; d <= 32; d++)
-        for (int oz = -4; oz <= 5; oz++)
-            for (int oy = -4; oy <= 5; oy++) {
-                const int ry = oy < 1 ? -oy : oy - 1, rz = oz < 1 ? -oz : oz - 1;
-                if (ry * ry + rz * rz == d)
-                    t.r[n++] = CellRow{(signed char)oy, (signed char)oz, (signed char)ry, (signed char)rz};
-            }
-    return t;
-}
-__constant__ CellRows c_cell_rows = make_cell_rows();
 
 struct CellSdfArgs {
     GridGeom g;

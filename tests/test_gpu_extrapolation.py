@@ -5,7 +5,7 @@ all, and more layers than the grid has."""
 import numpy as np
 import pytest
 
-from helpers import bits_equal
+from tests.helpers import bits_equal
 
 pytestmark = pytest.mark.gpu
 

@@ -6,7 +6,7 @@ import itertools
 import numpy as np
 import pytest
 
-from helpers import bits_equal
+from tests.helpers import bits_equal
 
 pytestmark = pytest.mark.gpu
 
