@@ -99,9 +99,11 @@ KERNEL_NAMES = {
 # HBM bytes moved per launch, measured with rocprofv3 FETCH_SIZE and WRITE_SIZE
 # passes scaled by a plain 256 MiB copy (x2.0 and x1.0), on the default
 # workload; the commands and counter readings are in
-# profiles/traffic_pcg_kernels_double_dam_256x128x128_mixed.md.  Keyed by
+# profiles/traffic_kernels_double_dam_256x128x128_mixed.md.  Keyed by
 # (precision, grid); other workloads report null.
-MEASURED_TRAFFIC = {}
+MEASURED_TRAFFIC = {
+    ("mixed", (256, 128, 128)): {"k_spmv_dot": 85.3e6, "k_axpy_norm": 150.6e6, "k_forward": 42.5e6, "k_update_s": 50.6e6, "k_backward": 73.8e6},
+}
 
 def parse_args(argv=None):
     p = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
