@@ -100,6 +100,20 @@ __device__ __forceinline__ double partials_total(const double *__restrict__ part
     return block_total<MAX>(v);
 }
 
+// Whether the solve has ended, the same for every wave of the workgroup: in
+// the kernels that may end it, another workgroup of the same launch can do so
+// between two waves' reads, and a wave that went on alone would take the sums
+// of those that left from LDS nobody wrote.
+__device__ __forceinline__ bool ended(const MgScalars *sc) {
+    __shared__ int done;
+    if (threadIdx.x == 0) done = __hip_atomic_load(&sc->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    return done != 0;
+}
+__device__ __forceinline__ void end_solve(MgScalars *sc) {
+    __hip_atomic_store(&sc->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Calls f(q, x, y, z, in) for this block's share of the level's active
 // bricks: cell (x, y, z) at flat index q, or (in = false) a lane outside the
 // level, whose q is the brick's first cell.  The call is uniform over the
@@ -290,14 +304,14 @@ template <bool FIRST>
 __global__ __launch_bounds__(kMgThreads) void k_mg_spmv(MgFine f, MgLevel L, MgLists ls, const float *__restrict__ s,
                                                         float *s_out, const double *__restrict__ part_zr, int nzr,
                                                         double *part_sq, MgScalars *sc, int turn) {
-    if (sc->done) return;
+    if (ended(sc)) return;
     const double rho = partials_total<false>(part_zr, nzr);
     const float beta = FIRST ? 0.0f : (float)(rho / sc->rho[turn ^ 1]);
     const bool bad = !(rho > 0.0) || !(rho <= 1.7976931348623157e308) || !(beta == beta);
     if (bad) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             sc->failed = 1;
-            sc->done = 1;
+            end_solve(sc);
         }
         return;
     }
@@ -339,7 +353,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_axpy_smooth(MgFine f, MgLevel
                                                                const float *__restrict__ s,
                                                                const double *__restrict__ part_sq, int nsq,
                                                                double *part_norm, MgScalars *sc, int turn) {
-    if (sc->done) return;
+    if (ended(sc)) return;
     double alpha = 0.0;
     if (MODE == kIterate) {
         const double sq = partials_total<false>(part_sq, nsq);
@@ -347,7 +361,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_axpy_smooth(MgFine f, MgLevel
         if (!(sq > 0.0) || !(alpha == alpha) || !(alpha <= 1.7976931348623157e308)) {
             if (blockIdx.x == 0 && threadIdx.x == 0) {
                 sc->failed = 1;
-                sc->done = 1;
+                end_solve(sc);
             }
             return;
         }
@@ -440,7 +454,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_smooth_down(MgLevel L, MgList
 __global__ __launch_bounds__(kMgThreads) void k_mg_restrict(MgLevel L, MgLists ls, MgLevel C, const double *norm,
                                                             int nnorm, MgScalars *sc) {
     __shared__ float sh[4][64];
-    if (sc->done) return;
+    if (ended(sc)) return;
     if (norm) {
         const double m = partials_total<true>(norm, nnorm);
         const bool stop = m <= sc->tol;
@@ -448,7 +462,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_restrict(MgLevel L, MgLists l
             const int it = sc->iters + 1;
             sc->iters = it;
             sc->resid = m;
-            if (stop || it >= sc->maxiter) sc->done = 1;
+            if (stop || it >= sc->maxiter) end_solve(sc);
         }
         if (stop) return;
     }
