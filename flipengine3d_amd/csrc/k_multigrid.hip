@@ -74,6 +74,9 @@ __device__ __forceinline__ double wave_max(double v) {
     }
     return v;
 }
+// The maximum m with a further magnitude.  A NaN counts as infinite, so it can
+// pass neither for a right-hand side below the tolerance nor for convergence.
+__device__ __forceinline__ double larger(double m, double a) { return a <= m ? m : (a == a ? a : INFINITY); }
 // Sum (MAX: maximum) over the workgroup in a fixed order, to every thread.
 template <bool MAX>
 __device__ __forceinline__ double block_total(double v) {
@@ -191,8 +194,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_assemble(GridGeom g, double d
             float inv = 0.0f, excess = 0.0f;
             if (is_row_cell(g, in.liquid, x + 1, y + 1, z + 1)) {
                 row = assemble_row(g, mf, in, x + 1, y + 1, z + 1);
-                const double a = fabs(row.rhs);
-                bmax = a > bmax ? a : bmax;
+                bmax = larger(bmax, fabs(row.rhs));
                 rows += 1.0;
                 row_here = 1;
                 if (row.diag > 0.0) {
@@ -381,9 +383,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_axpy_smooth(MgFine f, MgLevel
             L.z[p] = jacobi(kDampB, ip, rf, kDampA * (ip * rf), c);
             if (MODE == kIterate) f.x[p] += alpha * (double)s[p];
             if (MODE == kInit) f.x[p] = 0.0;
-            // A NaN counts as infinite, so it cannot pass for convergence.
-            const double a = fabs(rp);
-            mx = a <= mx ? mx : (a == a ? a : INFINITY);
+            mx = larger(mx, fabs(rp));
         }
     });
     const double t = block_total<true>(mx);
@@ -408,10 +408,10 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_true_residual(MgFine f, MgLev
         v += coupling(wx[p], mf) * x[p + 1];
         v += coupling(wy[p], mf) * x[p + px];
         v += coupling(wz[p], mf) * x[p + pz];
-        const double rp = f.rhs[p] - v, a = fabs(rp);
+        const double rp = f.rhs[p] - v;
         if (in) {
             r_out[p] = rp;
-            mx = a <= mx ? mx : (a == a ? a : INFINITY);
+            mx = larger(mx, fabs(rp));
         }
     });
     const double t = block_total<true>(mx);

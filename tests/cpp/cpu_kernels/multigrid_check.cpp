@@ -168,9 +168,28 @@ static void late_end() {
     }
 }
 
+// A right-hand side that is not a number anywhere is no solved system, though
+// the rest of it is below the tolerance.
+static void not_a_number() {
+    for (float bad : {NAN, -NAN, INFINITY}) {
+        System s(20, 20, 20);
+        s.pool(14);
+        s.u[s.fu(9, 6, 11)] = bad;
+        Solver a(s);
+        a.solve(s);
+        CHECK(a.sc.done && !a.sc.converged && a.sc.failed);
+    }
+    System still(20, 20, 20);
+    still.pool(14);
+    Solver a(still);
+    a.solve(still);
+    CHECK(a.sc.done && a.sc.converged && a.sc.iters == 0);
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "late_end") late_end();
+    else if (name == "not_a_number") not_a_number();
     else return 2;
     std::printf("ok\n");
     return 0;

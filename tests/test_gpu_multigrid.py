@@ -82,6 +82,20 @@ def test_not_finite(gpu, oracle):
     assert a["ok"] == b["ok"] == 1
 
 
+def test_not_finite_in_a_field_at_rest(gpu, oracle):
+    # Every other row of the right-hand side is zero.
+    dims = (24, 28, 21)
+    dx, solid, weights, liquid, mac, valid = _projection_inputs(oracle, *dims)
+    still = [np.zeros_like(g) for g in mac]
+    rows = (liquid < 0) & (weights[1][:, 1:] > 0)
+    k, j, i = np.argwhere(rows[1:-1, 1:-1, 1:-1])[5] + 1
+    still[1][k, j + 1, i] = np.nan
+    a, b = _both(gpu, (dx, solid, weights, liquid, still, valid), dims)
+    assert a["ok"] == b["ok"] == 0
+    for x, y in zip(a["mac"], b["mac"]):
+        assert bits_equal(x, y)
+
+
 def test_pocket_keeps_its_constant(gpu, oracle):
     dims = (20, 18, 17)
     dx, solid, weights, liquid, mac, valid, *_ = pocket_inputs(oracle, *dims)

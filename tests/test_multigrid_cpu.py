@@ -20,3 +20,7 @@ def check(tmp_path_factory):
 
 def test_a_solve_that_ends_during_a_launch_leaves_no_partial_sums(check):
     check("late_end")
+
+
+def test_a_right_hand_side_that_is_not_a_number_is_not_solved(check):
+    check("not_a_number")
