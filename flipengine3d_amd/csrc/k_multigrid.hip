@@ -56,6 +56,11 @@ constexpr int kBrickX = 64, kBrickY = 2, kBrickZ = 2;
 constexpr int kMgBlocks = 1024;
 static_assert(5 * kMgBlocks <= (int)kMgPartials, "five partial arrays");
 constexpr float kDampA = 1.5f, kDampB = 0.6f;
+// Least excess of a row's diagonal over its couplings, relative to their sum,
+// that is more than rounding (six products and sums in FP64, under 1e-14).  A
+// cell of some level that holds a whole region without air has no coupling, and
+// an inverse of 1e15 made of such rounding broke the iteration down.
+constexpr double kLeastExcess = 1e-12;
 
 // ---------------------------------------------------------------------------
 // Shared pieces
@@ -199,7 +204,8 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_assemble(GridGeom g, double d
                 row_here = 1;
                 if (row.diag > 0.0) {
                     inv = (float)(mf / row.diag);
-                    excess = (float)fmax(row.diag / mf - row.coupled, 0.0);
+                    const double e = row.diag / mf - row.coupled;
+                    excess = e > kLeastExcess * row.coupled ? (float)e : 0.0f;
                 }
             }
             f.rhs[q] = row.rhs;

@@ -24,3 +24,7 @@ def test_a_solve_that_ends_during_a_launch_leaves_no_partial_sums(check):
 
 def test_a_right_hand_side_that_is_not_a_number_is_not_solved(check):
     check("not_a_number")
+
+
+def test_regions_without_air_converge(check):
+    check("pockets")
