@@ -242,7 +242,9 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_assemble_total(const double *
 
 // Level l + 1 from level l, brick by brick.  e and the couplings are halves
 // of sums over children, so the coarse diagonal e + sum of couplings has no
-// cancellation.
+// cancellation.  A cell above a row counts as active even where that diagonal
+// is zero (it holds a whole region without air): the correction reads its z,
+// which must be this solve's zero and not what an earlier one left there.
 __global__ __launch_bounds__(kMgThreads) void k_mg_coarsen(MgLevel F, MgLevel C, int *flags) {
     const ListRange lr = xcd_list(C.nbx * C.nby * C.nbz);
     const int lx = (int)(threadIdx.x & 63u), ly = (int)((threadIdx.x >> 6) & 1u), lz = (int)(threadIdx.x >> 7);
@@ -261,6 +263,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarsen(MgLevel F, MgLevel C,
                     for (int a = 0; a < nx2; a++) {
                         const int q = f0 + a + F.px * b2 + F.pxy * c;
                         e += F.e[q];
+                        row_here |= F.inv[q] > 0.0f;
                         if (a == 0) xm += F.wx[q - 1]; else xp += F.wx[q];
                         if (b2 == 0) ym += F.wy[q - F.px]; else yp += F.wy[q];
                         if (c == 0) zm += F.wz[q - F.pxy]; else zp += F.wz[q];
@@ -273,7 +276,7 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_coarsen(MgLevel F, MgLevel C,
             C.wz[q] = zp;
             C.e[q] = e;
             C.inv[q] = d > 0.0f ? 1.0f / d : 0.0f;
-            row_here = d > 0.0f;
+            row_here |= d > 0.0f;
         }
         const int any = __syncthreads_or(row_here);
         if (flags && threadIdx.x == 0) flags[b] = any ? 1 : 0;

@@ -214,11 +214,34 @@ static void pockets() {
     }
 }
 
+// A solve's result does not depend on what the same store solved before.  The
+// pocket's cell of level 1 has no couplings and lies in a brick that holds
+// nothing else in the second system, and rows in the first.
+static void history() {
+    System first(36, 36, 20), second(36, 36, 20);
+    first.pool(33);
+    first.stir(2);
+    second.pool(6);
+    second.pocket(9, 29, 9, 2);
+    second.stir(11);
+    Solver used(first), fresh(second);
+    CHECK(used.plan.nglobal >= 2);
+    used.solve(first, 1e-2, 4);
+    used.solve(second, 1e-3, 8);
+    fresh.solve(second, 1e-3, 8);
+    CHECK(used.sc.iters == fresh.sc.iters && used.sc.converged && fresh.sc.converged);
+    for (int k = 1; k < 19; k++)
+        for (int j = 1; j < 35; j++)
+            for (int i = 1; i < 35; i++)
+                if (second.liquid[second.cell(i, j, k)] < 0) CHECK(used.x(i, j, k) == fresh.x(i, j, k));
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "late_end") late_end();
     else if (name == "not_a_number") not_a_number();
     else if (name == "pockets") pockets();
+    else if (name == "history") history();
     else return 2;
     std::printf("ok\n");
     return 0;

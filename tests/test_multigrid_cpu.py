@@ -28,3 +28,7 @@ def test_a_right_hand_side_that_is_not_a_number_is_not_solved(check):
 
 def test_regions_without_air_converge(check):
     check("pockets")
+
+
+def test_a_solve_does_not_depend_on_the_one_before(check):
+    check("history")
