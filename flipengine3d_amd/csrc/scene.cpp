@@ -124,13 +124,50 @@ size_t PressureStore::device_bytes() const {
 
 void PressureStore::alloc(const GridGeom &g, hipStream_t s, bool mixed, bool multigrid) {
     const MgPlan plan = mixed && multigrid ? make_mg_plan(g.I, g.J, g.K) : MgPlan{};
+    mg_wanted = plan.usable();
     // Grids without interior cells (no rows) and past 32-bit indices have no
     // levels; the MIC(0) iteration takes them, or refuses them, by itself.
-    if (!plan.usable()) {
+    if (!mg_wanted) {
         alloc_slots(g, s, mixed);
         return;
     }
-    graphs.clear();
+    release();
+    try {
+        bind_multigrid(plan, s);
+    } catch (...) {
+        release();
+        throw;
+    }
+    ready = kMultigrid;
+}
+
+void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s, bool mixed) {
+    release();
+    try {
+        bind_slots(g, s, mixed);
+    } catch (...) {
+        release();
+        throw;
+    }
+    ready = kMic0;
+}
+
+void PressureStore::release() {
+    ready = kNone;
+    graphs.clear();  // captured launches point into the buffers
+    for (int q = 0; q <= kSlotArrays; q++) arr[q].release();
+    for (int q = 0; q < 2; q++) arr64[q].release();
+    for (int q = 0; q < kWeightArrays; q++) wgt[q].release();
+    for (int q = 0; q < kSlotArrays32; q++) arr32[q].release();
+    edge.release(); mask.release(); progress.release(); ticket.release(); irange.release(); alist.release();
+    scal.release();
+    pb = PressureBuffers{};
+    for (int q = 0; q < 6; q++) mg_f64[q].release();
+    mg_part.release(); mg_f32.release(); mg_ints.release(); mg_bricks.release(); mg_scal.release();
+    mg_coarse.release();
+}
+
+void PressureStore::bind_multigrid(const MgPlan &plan, hipStream_t s) {
     auto need = [&](hipError_t e) {
         if (e != hipSuccess) throw StatusError{FLIPMI_ERR_OOM, "mixed-precision arrays: out of device memory"};
     };
@@ -155,20 +192,10 @@ void PressureStore::alloc(const GridGeom &g, hipStream_t s, bool mixed, bool mul
     // Padding and guards are read and never written: they stay zero.
     if (mg.clear(s) != hipSuccess)
         throw StatusError{FLIPMI_ERR_HIP, "pressure arrays: clearing failed"};
-    mg_on = true;
     mg_dirty = false;
 }
 
-void PressureStore::release_multigrid() {
-    graphs.clear();
-    for (int q = 0; q < 6; q++) mg_f64[q].release();
-    mg_part.release(); mg_f32.release(); mg_ints.release(); mg_bricks.release(); mg_scal.release();
-    mg_coarse.release();
-    mg_on = false;
-}
-
-void PressureStore::alloc_slots(const GridGeom &g, hipStream_t s, bool mixed) {
-    graphs.clear();  // captured launches point into the buffers replaced here
+void PressureStore::bind_slots(const GridGeom &g, hipStream_t s, bool mixed) {
     SlotMap sm = make_slot_map(g.I, g.J, g.K);
     // Slot arrays carry the zero and sink groups after the last tile.
     size_t ns = sm.alloc_count();
@@ -422,15 +449,19 @@ static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *h
 
 PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *host_sc, hipStream_t s, Scene *prof) {
     PressureOutcome out;
-    if (ps.mg_on) {
+    const bool mixed = w.precision == FLIPMI_PCG_MIXED;
+    // An earlier solve found no room for its buffers: there may be some now.
+    if (ps.ready == PressureStore::kNone) ps.alloc(w.g, s, mixed, ps.mg_wanted);
+    if (ps.ready == PressureStore::kMultigrid) {
         if (run_multigrid(w, ps, static_cast<MgScalars *>(host_sc), s, prof, out)) return out;
         // Not positive definite, not finite, or capped: the reference's
         // preconditioner decides, here and for the rest of this store's life.
         hip_check(hipStreamSynchronize(s), "pcg sync");
-        ps.release_multigrid();
         ps.alloc_slots(w.g, s, true);
     }
     PressureBuffers &pb = ps.pb;
+    if (ps.ready != PressureStore::kMic0 || (mixed ? !pb.r32 : !pb.sb))
+        throw StatusError{FLIPMI_ERR_INVALID_ARG, "arrays of this precision not allocated"};
     PcgScalars *hs = static_cast<PcgScalars *>(host_sc);
     hipEvent_t ev = nullptr;
     if (prof) prof->begin_stage(FLIPMI_STAGE_ASSEMBLE, &ev);
@@ -453,9 +484,6 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
         return out;
     }
     if (prof) prof->begin_stage(FLIPMI_STAGE_MIC0, &ev);
-    const bool mixed = w.precision == FLIPMI_PCG_MIXED;
-    if (mixed ? !pb.r32 : !pb.sb)
-        throw StatusError{FLIPMI_ERR_INVALID_ARG, "arrays of this precision not allocated"};
     hip_check(launch_group_mask(pb, s), "group mask");
     hip_check(launch_mic0_factor(w.g, w.liquid, pb, s), "mic0 factor");
     hip_check(launch_pcg_init(w.g, w.tol, w.maxiter, mixed, pb, s), "pcg init");

@@ -43,7 +43,12 @@ struct DBuf {
         scope = PoolScope::current();
         void *q = nullptr;
         hipError_t e = scope ? scope->get(sizeof(T) * count, &q, &block) : hipMalloc(&q, sizeof(T) * count);
-        if (e == hipSuccess) p = static_cast<T *>(q);
+        if (e == hipSuccess) {
+            p = static_cast<T *>(q);
+        } else {
+            n = 0;
+            (void)hipGetLastError();  // reported here, not by the next launch
+        }
         return e;
     }
     void release() {
@@ -318,8 +323,12 @@ struct PressureStore {
     DBuf<PcgScalars> scal;
     PressureBuffers pb{};
     PcgGraphs graphs;             // captured iteration batches (pointers into these buffers)
-    MgSolver mg;                  // bound while its buffers are allocated
-    bool mg_on = false;
+    MgSolver mg;
+    // The solver whose buffers are all there and bound; none after an
+    // allocation that failed.
+    enum Solver { kNone, kMultigrid, kMic0 };
+    Solver ready = kNone;
+    bool mg_wanted = false;       // alloc() takes multigrid
     bool mg_dirty = false;        // the last solve may have left values that are not finite
     DBuf<double> mg_f64[6], mg_part;
     DBuf<float> mg_f32;
@@ -327,10 +336,16 @@ struct PressureStore {
     DBuf<int4> mg_bricks;
     DBuf<MgScalars> mg_scal;
     DBuf<MgCoarse> mg_coarse;
+    // Both replace what is there.  alloc: multigrid where it is asked for,
+    // serves the precision and has levels, else MIC(0)'s slots.
     void alloc(const GridGeom &g, hipStream_t s, bool mixed, bool multigrid);
     void alloc_slots(const GridGeom &g, hipStream_t s, bool mixed);
-    void release_multigrid();
     size_t device_bytes() const;
+
+private:
+    void release();
+    void bind_slots(const GridGeom &g, hipStream_t s, bool mixed);
+    void bind_multigrid(const MgPlan &plan, hipStream_t s);
 };
 
 // Device bytes a scene with these settings and particle capacity allocates.

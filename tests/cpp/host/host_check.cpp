@@ -1,0 +1,118 @@
+// Checks of the library's host side over a runtime without a device
+// (fake_hip.h), one per command-line name; see tests/test_host_side.py.
+#include <cstdio>
+#include <cstring>
+#include <memory>
+
+#include "../../../flipengine3d_amd/csrc/scene.h"
+#include "fake_hip.h"
+
+using namespace flipmi;
+using fake::rt;
+
+#define CHECK(c)                                            \
+    do {                                                    \
+        if (!(c)) {                                         \
+            std::printf("line %d: %s\n", __LINE__, #c);     \
+            std::exit(1);                                   \
+        }                                                   \
+    } while (0)
+// With the two values where they differ.
+#define CHECK_EQ(a, b)                                                                           \
+    do {                                                                                         \
+        const long long x = (long long)(a), y = (long long)(b);                                  \
+        if (x != y) {                                                                            \
+            std::printf("line %d: %s == %s: %lld against %lld\n", __LINE__, #a, #b, x, y);       \
+            std::exit(1);                                                                        \
+        }                                                                                        \
+    } while (0)
+
+// A mixed-precision projection on a store of its own.  How its two solvers end
+// is set by `multigrid` and `mic0`, written over the scalars they read back.
+struct Projection {
+    PressureStore ps;
+    PressureWork w;
+    std::vector<float> grid;
+    std::vector<uint8_t> flags;
+    char host[kPressureStaging];
+    bool multigrid = true, mic0 = true;
+    hipStream_t stream = nullptr;
+    Projection() {
+        CHECK(hipStreamCreateWithFlags(&stream, 0) == hipSuccess);
+        grid.assign(34 * 35 * 35, 0.0f);
+        flags.assign(grid.size(), 0);
+        w.g.I = 33; w.g.J = w.g.K = 34;
+        w.g.dx = 1.0 / 32;
+        w.g.invdx = 32;
+        w.dt = 1.0 / 60;
+        w.tol = 1e-9;
+        w.acceptable = 1.0;
+        w.maxiter = 100;
+        w.precision = FLIPMI_PCG_MIXED;
+        w.liquid = w.wU = w.wV = w.wW = w.wC = w.sU = w.sV = w.sW = grid.data();
+        w.u = w.v = w.w = grid.data();
+        w.vu = w.vv = w.vw = flags.data();
+        rt().on_download = [this](void *dst, size_t bytes) {
+            if (bytes == sizeof(MgScalars)) {
+                MgScalars *sc = static_cast<MgScalars *>(dst);
+                sc->bnorm = 1.0;
+                sc->done = 1;
+                sc->converged = multigrid;
+                sc->failed = !multigrid;
+            } else if (bytes == sizeof(PcgScalars)) {
+                PcgScalars *sc = static_cast<PcgScalars *>(dst);
+                const double one = 1.0;
+                std::memcpy(&sc->absmax_bits, &one, sizeof one);
+                sc->done = sc->converged = mic0;
+                sc->failed = !mic0;
+                sc->done = 1;
+            }
+        };
+    }
+    ~Projection() { rt().on_download = nullptr; }
+    // The status a solve ends with; `first` is set to its first launch.
+    int solve(size_t *first = nullptr) {
+        if (first) *first = rt().launched.size();
+        try {
+            return run_pressure(w, ps, host, stream, nullptr).success ? FLIPMI_OK : FLIPMI_ERR_HIP;
+        } catch (const StatusError &e) {
+            return e.code;
+        }
+    }
+};
+
+// The MIC(0) iteration that takes over from multigrid does not fit: that solve
+// and the next ones report it, and none runs on arrays that are not there.
+static void no_room_to_fall_back() {
+    Projection p;
+    p.ps.alloc(p.w.g, p.stream, true, true);
+    CHECK_EQ(p.solve(), FLIPMI_OK);
+    {
+        PressureStore slots;
+        const size_t before = rt().in_use;
+        slots.alloc_slots(p.w.g, p.stream, true);
+        CHECK(rt().in_use - before > before);  // MIC(0)'s arrays are the larger
+    }
+    rt().limit = rt().in_use;
+    p.multigrid = false;
+    size_t first = 0;
+    for (int q = 0; q < 3; q++) {
+        CHECK_EQ(p.solve(&first), FLIPMI_ERR_OOM);
+        CHECK(!rt().was_launched("k_reset_scalars", first) && !rt().was_launched("k_assemble", first));
+        CHECK(rt().in_use <= rt().limit);
+    }
+    // With room again, it is solved again.
+    rt().limit = ~(size_t)0;
+    CHECK_EQ(p.solve(), FLIPMI_OK);
+    p.multigrid = true;
+    CHECK_EQ(p.solve(), FLIPMI_OK);
+}
+
+int main(int argc, char **argv) {
+    const std::string name = argc > 1 ? argv[1] : "";
+    if (name == "no_room_to_fall_back") no_room_to_fall_back();
+    else return 2;
+    std::printf("ok\n");
+    std::fflush(stdout);
+    return 0;
+}

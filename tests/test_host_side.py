@@ -1,0 +1,32 @@
+"""What the library does on the host when something fails or several callers meet, without a device: a check program
+defines the HIP runtime's functions itself (tests/cpp/host)."""
+
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HOST = os.path.join(ROOT, "tests", "cpp", "host")
+LIB = os.path.join(ROOT, "flipengine3d_amd")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("host") / "host_check")
+    if not os.path.exists(os.path.join(LIB, "libflipmi.so")):
+        import flipengine3d_amd.build
+        flipengine3d_amd.build.build()
+    # The HIP runtime itself is the library's to load, and hidden by these definitions.
+    subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-w", "-rdynamic", "-pthread", "-I",
+                    "/opt/rocm/include", os.path.join(HOST, "host_check.cpp"), os.path.join(HOST, "fake_hip.cpp"), "-o",
+                    exe, "-L", LIB, "-lflipmi", "-Wl,-rpath," + LIB, "-Wl,--allow-shlib-undefined"], check=True)
+
+    def run(name):
+        r = subprocess.run([exe, name], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_a_fallback_without_room_is_an_error_each_time(check):
+    check("no_room_to_fall_back")
