@@ -167,6 +167,22 @@ void PressureStore::release() {
     mg_coarse.release();
 }
 
+// One system that is not finite, or capped, says little about the next, so
+// multigrid is tried again in the next solve.  A scene that it keeps failing on
+// (an iteration cap below its need) pays for the failed solve and for changing
+// the buffers less and less often: after 0, 1, 3, 7, ... 63 solves.
+bool PressureStore::multigrid_due() {
+    if (ready != kMic0 || !mg_wanted) return false;
+    if (mg_wait == 0) return true;
+    mg_wait--;
+    return false;
+}
+
+void PressureStore::multigrid_ended(bool converged) {
+    mg_wait = converged ? 0 : mg_backoff;
+    mg_backoff = converged ? 0 : std::min(2 * mg_backoff + 1, 63);
+}
+
 void PressureStore::bind_multigrid(const MgPlan &plan, hipStream_t s) {
     auto need = [&](hipError_t e) {
         if (e != hipSuccess) throw StatusError{FLIPMI_ERR_OOM, "mixed-precision arrays: out of device memory"};
@@ -450,12 +466,18 @@ static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *h
 PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *host_sc, hipStream_t s, Scene *prof) {
     PressureOutcome out;
     const bool mixed = w.precision == FLIPMI_PCG_MIXED;
-    // An earlier solve found no room for its buffers: there may be some now.
-    if (ps.ready == PressureStore::kNone) ps.alloc(w.g, s, mixed, ps.mg_wanted);
+    // An earlier solve found no room for its buffers (there may be some now), or
+    // went to MIC(0) and multigrid's turn has come again.
+    if (ps.ready == PressureStore::kNone || ps.multigrid_due()) {
+        hip_check(hipStreamSynchronize(s), "pcg sync");
+        ps.alloc(w.g, s, mixed, ps.mg_wanted);
+    }
     if (ps.ready == PressureStore::kMultigrid) {
-        if (run_multigrid(w, ps, static_cast<MgScalars *>(host_sc), s, prof, out)) return out;
+        const bool solved = run_multigrid(w, ps, static_cast<MgScalars *>(host_sc), s, prof, out);
+        ps.multigrid_ended(solved);
+        if (solved) return out;
         // Not positive definite, not finite, or capped: the reference's
-        // preconditioner decides, here and for the rest of this store's life.
+        // preconditioner decides.
         hip_check(hipStreamSynchronize(s), "pcg sync");
         ps.alloc_slots(w.g, s, true);
     }
@@ -794,6 +816,7 @@ bool Scene::rearm(const float *pos, const float *vel, int64_t count_in) {
     last_resid = 0.0;
     last_rows = 0;
     last_refinements = 0;
+    press->start_over();
     for (int q = 0; q < FLIPMI_NUM_STAGES; q++) {
         stage_ms[q] = 0.0;
         stage_calls[q] = 0;

@@ -307,7 +307,7 @@ PressureOutcome run_pressure(const PressureWork &w, PressureStore &ps, void *hos
 // Lzm), arr[13] the reduction partials, wgt[0..2] the coupling weights
 // (wx, wy, wz); the mixed MIC(0) iteration adds FP32 copies.  With multigrid:
 // its levels; a system it does not solve goes to the MIC(0) iteration, whose
-// storage then replaces them.
+// storage then replaces them until multigrid's turn comes again.
 struct PressureStore {
     static constexpr int kSlotArrays = 13;
     static constexpr int kWeightArrays = 3;
@@ -329,6 +329,9 @@ struct PressureStore {
     enum Solver { kNone, kMultigrid, kMic0 };
     Solver ready = kNone;
     bool mg_wanted = false;       // alloc() takes multigrid
+    // After a solve that multigrid did not converge: solves left to MIC(0)
+    // before the next try, and how many it will be after the next failure.
+    int mg_wait = 0, mg_backoff = 0;
     bool mg_dirty = false;        // the last solve may have left values that are not finite
     DBuf<double> mg_f64[6], mg_part;
     DBuf<float> mg_f32;
@@ -341,6 +344,11 @@ struct PressureStore {
     void alloc(const GridGeom &g, hipStream_t s, bool mixed, bool multigrid);
     void alloc_slots(const GridGeom &g, hipStream_t s, bool mixed);
     size_t device_bytes() const;
+    // Forgets how earlier solves ended: the next one chooses as the first did.
+    void start_over() { mg_wait = mg_backoff = 0; }
+    // Whether the coming solve, MIC(0)'s as things are, is multigrid's again.
+    bool multigrid_due();
+    void multigrid_ended(bool converged);
 
 private:
     void release();

@@ -108,9 +108,46 @@ static void no_room_to_fall_back() {
     CHECK_EQ(p.solve(), FLIPMI_OK);
 }
 
+// A solve that multigrid does not converge is redone by MIC(0), and the next one
+// is multigrid's again; while it keeps failing it is tried more and more rarely,
+// at least once in 64 solves.
+static void multigrid_again() {
+    Projection p;
+    p.ps.alloc(p.w.g, p.stream, true, true);
+    size_t first = 0;
+    auto tried = [&]() {
+        CHECK_EQ(p.solve(&first), FLIPMI_OK);
+        return rt().was_launched("k_mg_assemble", first);
+    };
+    auto redone = [&]() { return rt().was_launched("k_assemble", first); };
+    CHECK(tried() && !redone());
+    p.multigrid = false;
+    CHECK(tried() && redone());
+    p.multigrid = true;
+    for (int q = 0; q < 3; q++) CHECK(tried() && !redone());
+    p.multigrid = false;
+    int since = 0, longest = 0, tries = 0;
+    for (int q = 0; q < 400; q++) {
+        if (tried()) {
+            tries++;
+            longest = std::max(longest, since);
+            since = 0;
+        } else {
+            since++;
+        }
+        CHECK(redone());
+    }
+    CHECK(tries >= 7 && tries <= 12 && longest <= 64);
+    // Where the count stands does not outlive the request.
+    p.ps.start_over();
+    p.multigrid = true;
+    CHECK(tried() && !redone());
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
+    else if (name == "multigrid_again") multigrid_again();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

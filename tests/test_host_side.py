@@ -30,3 +30,7 @@ def check(tmp_path_factory):
 
 def test_a_fallback_without_room_is_an_error_each_time(check):
     check("no_room_to_fall_back")
+
+
+def test_multigrid_is_tried_again_after_a_fallback(check):
+    check("multigrid_again")
