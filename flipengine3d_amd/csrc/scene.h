@@ -42,13 +42,9 @@ struct DBuf {
         if (count == 0) return hipSuccess;
         scope = PoolScope::current();
         void *q = nullptr;
-        hipError_t e = scope ? scope->get(sizeof(T) * count, &q, &block) : hipMalloc(&q, sizeof(T) * count);
-        if (e == hipSuccess) {
-            p = static_cast<T *>(q);
-        } else {
-            n = 0;
-            (void)hipGetLastError();  // reported here, not by the next launch
-        }
+        hipError_t e = scope ? scope->get(sizeof(T) * count, &q, &block) : device_alloc(&q, sizeof(T) * count);
+        if (e == hipSuccess) p = static_cast<T *>(q);
+        else n = 0;
         return e;
     }
     void release() {

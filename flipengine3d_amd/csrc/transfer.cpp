@@ -197,13 +197,16 @@ hipError_t DevicePool::get(size_t bytes, void **p, size_t *size) {
             return hipSuccess;
         }
     }
-    hipError_t e = hipMalloc(p, want);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        release();
-        e = hipMalloc(p, want);
-    }
     *size = want;
+    hipError_t e = hipMalloc(p, want);
+    if (e == hipSuccess) return e;
+    release();
+    e = hipMalloc(p, want);
+    if (e != hipSuccess) {
+        *size = bytes;  // the step may be what does not fit
+        e = hipMalloc(p, bytes);
+    }
+    (void)hipGetLastError();  // reported here, not by the next launch
     return e;
 }
 
@@ -245,16 +248,42 @@ PoolScope *PoolScope::current() { return t_scope; }
 PoolScope::Off::Off() : was(t_scope) { t_scope = nullptr; }
 PoolScope::Off::~Off() { t_scope = was; }
 
-std::shared_ptr<DeviceShared> DeviceShared::of(int device) {
-    static std::mutex m;
+namespace {
+std::mutex g_shared_mutex;
+std::map<int, std::weak_ptr<DeviceShared>> &all_shared() {
     static std::map<int, std::weak_ptr<DeviceShared>> all;
-    std::lock_guard<std::mutex> lk(m);
-    std::shared_ptr<DeviceShared> p = all[device].lock();
+    return all;
+}
+}  // namespace
+
+std::shared_ptr<DeviceShared> DeviceShared::of(int device) {
+    std::lock_guard<std::mutex> lk(g_shared_mutex);
+    std::weak_ptr<DeviceShared> &held = all_shared()[device];
+    std::shared_ptr<DeviceShared> p = held.lock();
     if (!p) {
         p = std::make_shared<DeviceShared>();
-        all[device] = p;
+        held = p;
     }
     return p;
+}
+
+std::shared_ptr<DeviceShared> DeviceShared::find(int device) {
+    std::lock_guard<std::mutex> lk(g_shared_mutex);
+    auto it = all_shared().find(device);
+    return it == all_shared().end() ? nullptr : it->second.lock();
+}
+
+hipError_t device_alloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    int device = 0;
+    if (e == hipSuccess || hipGetDevice(&device) != hipSuccess) return e;
+    const std::shared_ptr<DeviceShared> shared = DeviceShared::find(device);
+    if (shared) {
+        shared->pool.release();
+        e = hipMalloc(p, bytes);
+    }
+    (void)hipGetLastError();  // reported here, not by the next launch
+    return e;
 }
 
 hipError_t PoolScope::get(size_t bytes, void **p, size_t *size) {
@@ -266,7 +295,14 @@ hipError_t PoolScope::get(size_t bytes, void **p, size_t *size) {
         back.erase(it);
         return hipSuccess;
     }
-    return pool.get(bytes, p, size);
+    hipError_t e = pool.get(bytes, p, size);
+    if (e != hipSuccess && !back.empty()) {
+        (void)hipStreamSynchronize(stream);
+        for (auto &b : back) (void)hipFree(b.second);
+        back.clear();
+        e = pool.get(bytes, p, size);
+    }
+    return e;
 }
 
 }  // namespace flipmi

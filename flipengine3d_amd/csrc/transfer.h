@@ -53,8 +53,8 @@ private:
 };
 
 // Device blocks kept between stage calls, at most kHeld bytes of them; the
-// rest goes back to the device, as all of it does when an allocation fails.
-// Safe from several threads.
+// rest goes back to the device, as all of it does when an allocation fails
+// here or in device_alloc.  Safe from several threads.
 class DevicePool {
 public:
     DevicePool() {}
@@ -74,8 +74,8 @@ private:
 
 // While one is alive, the device buffers its thread allocates come from the
 // pool.  All their uses are on one stream, so a buffer given back is reused
-// within the call as it is; the pool gets it when the stream is idle.  The
-// scope outlives its buffers.
+// within the call as it is; the pool gets it when the stream is idle, and the
+// device when an allocation fails.  The scope outlives its buffers.
 class PoolScope {
 public:
     PoolScope(DevicePool &pool, hipStream_t s);
@@ -108,6 +108,12 @@ struct DeviceShared {
     HostLink link;
     DevicePool pool;
     static std::shared_ptr<DeviceShared> of(int device);
+    // Null where no context holds one.
+    static std::shared_ptr<DeviceShared> find(int device);
 };
+
+// hipMalloc on the current device, which has what the device's pool holds idle
+// before it reports that the memory is out.
+hipError_t device_alloc(void **p, size_t bytes);
 
 }  // namespace flipmi

@@ -144,10 +144,59 @@ static void multigrid_again() {
     CHECK(tried() && !redone());
 }
 
+// Memory that a stage call left in the pool is there for every other allocation,
+// and so are the blocks that a call has given back itself.
+static void pool_gives_way() {
+    flipmi_ctx *ctx = nullptr;
+    CHECK_EQ(flipmi_ctx_create(0, &ctx), FLIPMI_OK);
+    const int n = 256;
+    std::vector<float> field((size_t)n * n * n, 0.0f);
+    std::vector<uint8_t> valid(field.size(), 0);
+    CHECK_EQ(flipmi_extrapolate(ctx, n, n, n, field.data(), valid.data(), 1), FLIPMI_OK);
+    const size_t idle = rt().in_use;
+    CHECK(idle > ((size_t)64 << 20));
+    // Outside any stage call: all but a little of the memory is the pool's.
+    rt().limit = idle + ((size_t)1 << 20);
+    {
+        DBuf<float> buffer;
+        CHECK_EQ(buffer.alloc(field.size()), hipSuccess);
+        CHECK(!buffer.scope);
+        CHECK_EQ(buffer.alloc(64 * field.size()), hipErrorOutOfMemory);
+        CHECK(!buffer.p && buffer.n == 0);
+        CHECK_EQ(hipGetLastError(), hipSuccess);
+    }
+    CHECK_EQ(rt().in_use, 0);
+    // Inside one: a buffer given back makes room for a larger one.
+    DevicePool pool;
+    rt().limit = 100 << 20;
+    {
+        hipStream_t s = nullptr;
+        CHECK(hipStreamCreateWithFlags(&s, 0) == hipSuccess);
+        PoolScope scope(pool, s);
+        DBuf<float> a, b;
+        CHECK_EQ(a.alloc(15 << 20), hipSuccess);  // 60 MiB
+        a.release();
+        CHECK_EQ(b.alloc(22 << 20), hipSuccess);  // 88 MiB
+        CHECK_EQ(hipGetLastError(), hipSuccess);
+    }
+    // A block that fits exactly is had, though blocks come in steps.
+    {
+        pool.release();
+        PoolScope scope(pool, nullptr);
+        DBuf<char> c;
+        CHECK_EQ(c.alloc((100 << 20) - 3), hipSuccess);
+        CHECK_EQ(hipGetLastError(), hipSuccess);
+    }
+    pool.release();
+    rt().limit = ~(size_t)0;
+    CHECK_EQ(flipmi_ctx_destroy(ctx), FLIPMI_OK);
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
     else if (name == "multigrid_again") multigrid_again();
+    else if (name == "pool_gives_way") pool_gives_way();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

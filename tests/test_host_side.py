@@ -34,3 +34,7 @@ def test_a_fallback_without_room_is_an_error_each_time(check):
 
 def test_multigrid_is_tried_again_after_a_fallback(check):
     check("multigrid_again")
+
+
+def test_idle_pool_memory_is_there_for_others(check):
+    check("pool_gives_way")
