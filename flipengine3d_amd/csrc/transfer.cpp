@@ -34,12 +34,14 @@ thread_local PoolScope *t_scope = nullptr;
 
 bool HostLink::ready() {
     if (ring) return true;
-    for (int q = 0; q < kSlots; q++)
-        if (!filled[q] && hipEventCreateWithFlags(&filled[q], hipEventDisableTiming) != hipSuccess) return false;
+    hipError_t e = hipSuccess;
+    for (int q = 0; q < kSlots && e == hipSuccess; q++)
+        if (!filled[q]) e = hipEventCreateWithFlags(&filled[q], hipEventDisableTiming);
     void *p = nullptr;
-    if (hipHostMalloc(&p, kChunk * kSlots, hipHostMallocDefault) != hipSuccess) return false;
-    ring = static_cast<char *>(p);
-    return true;
+    if (e == hipSuccess) e = hipHostMalloc(&p, kChunk * kSlots, hipHostMallocDefault);
+    if (e == hipSuccess) ring = static_cast<char *>(p);
+    else (void)hipGetLastError();  // plain copies do: no launch is to report it
+    return ring != nullptr;
 }
 
 void HostLink::release() {
@@ -62,7 +64,9 @@ hipError_t HostLink::get_page(void **p) {
             return hipSuccess;
         }
     }
-    return hipHostMalloc(p, kPage, hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc(p, kPage, hipHostMallocDefault);
+    if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
+    return e;
 }
 
 void HostLink::put_page(void *p) {

@@ -192,11 +192,35 @@ static void pool_gives_way() {
     CHECK_EQ(flipmi_ctx_destroy(ctx), FLIPMI_OK);
 }
 
+// Without pinned memory results come by plain copies, and the failure to get any
+// is not taken for that of a later launch.
+static void no_pinned_memory() {
+    flipmi_ctx *ctx = nullptr;
+    CHECK_EQ(flipmi_ctx_create(0, &ctx), FLIPMI_OK);
+    const int n = 64;
+    std::vector<float> field((size_t)n * n * n, 0.0f);
+    std::vector<uint8_t> valid(field.size(), 0);
+    rt().pinned_fails = true;
+    for (int q = 0; q < 3; q++) {
+        for (size_t c = 0; c < field.size(); c++) field[c] = (float)c;
+        CHECK_EQ(flipmi_extrapolate(ctx, n, n, n, field.data(), valid.data(), 1), FLIPMI_OK);
+        for (size_t c = 0; c < field.size(); c++) CHECK(field[c] == (float)c);
+        CHECK_EQ(hipGetLastError(), hipSuccess);
+    }
+    void *page = nullptr;
+    HostLink link;
+    CHECK_EQ(link.get_page(&page), hipErrorOutOfMemory);
+    CHECK_EQ(hipGetLastError(), hipSuccess);
+    rt().pinned_fails = false;
+    CHECK_EQ(flipmi_ctx_destroy(ctx), FLIPMI_OK);
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
     else if (name == "multigrid_again") multigrid_again();
     else if (name == "pool_gives_way") pool_gives_way();
+    else if (name == "no_pinned_memory") no_pinned_memory();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

@@ -38,3 +38,7 @@ def test_multigrid_is_tried_again_after_a_fallback(check):
 
 def test_idle_pool_memory_is_there_for_others(check):
     check("pool_gives_way")
+
+
+def test_results_come_without_pinned_memory(check):
+    check("no_pinned_memory")
