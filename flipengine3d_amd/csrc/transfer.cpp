@@ -248,6 +248,15 @@ PoolScope::~PoolScope() {
     for (auto &b : back) pool.put(b.second, b.first);
 }
 
+void PoolScope::put(void *p, size_t size) noexcept {
+    try {
+        back.insert({size, p});
+    } catch (...) {
+        (void)hipStreamSynchronize(stream);  // its last use may still run
+        (void)hipFree(p);
+    }
+}
+
 PoolScope *PoolScope::current() { return t_scope; }
 PoolScope::Off::Off() : was(t_scope) { t_scope = nullptr; }
 PoolScope::Off::~Off() { t_scope = was; }

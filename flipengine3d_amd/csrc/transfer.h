@@ -94,7 +94,7 @@ public:
         PoolScope *was;
     };
     hipError_t get(size_t bytes, void **p, size_t *size);
-    void put(void *p, size_t size) { back.insert({size, p}); }
+    void put(void *p, size_t size) noexcept;  // from destructors
 
 private:
     DevicePool &pool;

@@ -1,14 +1,26 @@
 // Checks of the library's host side over a runtime without a device
 // (fake_hip.h), one per command-line name; see tests/test_host_side.py.
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <new>
 
 #include "../../../flipengine3d_amd/csrc/scene.h"
 #include "fake_hip.h"
 
 using namespace flipmi;
 using fake::rt;
+
+// Host allocations of this thread fail while set.
+static thread_local bool t_no_host_memory = false;
+void *operator new(size_t n) {
+    void *p = t_no_host_memory ? nullptr : std::malloc(n);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 #define CHECK(c)                                            \
     do {                                                    \
@@ -215,12 +227,35 @@ static void no_pinned_memory() {
     CHECK_EQ(flipmi_ctx_destroy(ctx), FLIPMI_OK);
 }
 
+// A buffer is given back without host memory to note it in: no exception leaves
+// its destructor, and the device gets it.
+static void give_back_without_host_memory() {
+    DevicePool pool;
+    hipStream_t s = nullptr;
+    CHECK(hipStreamCreateWithFlags(&s, 0) == hipSuccess);
+    bool waited = false;
+    rt().on_stream_wait = [&](hipStream_t) { waited = true; };
+    {
+        PoolScope scope(pool, s);
+        std::unique_ptr<DBuf<float>> buffer(new DBuf<float>());
+        CHECK_EQ(buffer->alloc(1000), hipSuccess);
+        CHECK(rt().in_use > 0);
+        t_no_host_memory = true;
+        buffer.reset();
+        t_no_host_memory = false;
+        CHECK_EQ(rt().in_use, 0);
+        CHECK(waited);  // its last use may still run
+    }
+    rt().on_stream_wait = nullptr;
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
     else if (name == "multigrid_again") multigrid_again();
     else if (name == "pool_gives_way") pool_gives_way();
     else if (name == "no_pinned_memory") no_pinned_memory();
+    else if (name == "give_back_without_host_memory") give_back_without_host_memory();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

@@ -42,3 +42,7 @@ def test_idle_pool_memory_is_there_for_others(check):
 
 def test_results_come_without_pinned_memory(check):
     check("no_pinned_memory")
+
+
+def test_a_buffer_is_given_back_without_host_memory(check):
+    check("give_back_without_host_memory")
