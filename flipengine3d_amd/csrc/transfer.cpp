@@ -9,7 +9,7 @@
 namespace flipmi {
 
 namespace {
-// Below this a copy is one call: staging gains nothing.
+// Below this a result is small: one copy into a slab; the ring gains nothing.
 constexpr size_t kDirect = (size_t)256 << 10;
 // Threads that empty the ring, for copies that are worth starting them (about
 // 30 us each).  226 MB of particles in two copies: 59 ms as six pageable copies
@@ -45,8 +45,10 @@ bool HostLink::ready() {
 }
 
 void HostLink::release() {
-    for (void *p : pages) (void)hipHostFree(p);
-    pages.clear();
+    for (auto *idle : {&pages, &slabs}) {
+        for (void *p : *idle) (void)hipHostFree(p);
+        idle->clear();
+    }
     if (ring) (void)hipHostFree(ring);
     ring = nullptr;
     for (hipEvent_t &e : filled) {
@@ -55,55 +57,75 @@ void HostLink::release() {
     }
 }
 
-hipError_t HostLink::get_page(void **p) {
+hipError_t HostLink::take(std::vector<void *> &idle, size_t bytes, void **p) {
     {
-        std::lock_guard<std::mutex> lk(page_m);
-        if (!pages.empty()) {
-            *p = pages.back();
-            pages.pop_back();
+        std::lock_guard<std::mutex> lk(idle_m);
+        if (!idle.empty()) {
+            *p = idle.back();
+            idle.pop_back();
             return hipSuccess;
         }
     }
-    const hipError_t e = hipHostMalloc(p, kPage, hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
     if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
     return e;
 }
 
-void HostLink::put_page(void *p) {
-    std::lock_guard<std::mutex> lk(page_m);
-    try {
-        pages.push_back(p);
-    } catch (...) {
-        (void)hipHostFree(p);
+void HostLink::give(std::vector<void *> &idle, size_t most, void *p) {
+    {
+        std::lock_guard<std::mutex> lk(idle_m);
+        if (idle.size() < most) {
+            try {
+                idle.push_back(p);
+                return;
+            } catch (...) {
+            }
+        }
     }
+    (void)hipHostFree(p);
 }
 
 hipError_t HostLink::to_host(const HostPiece *pieces, int count, hipStream_t s) {
-    std::lock_guard<std::mutex> lk(m);
-    const bool staged = ready();
-    // The small pieces, through the ring as far as it goes; a piece that is
-    // alone, or without a ring, is one plain copy.
+    // The small pieces go through a slab as far as it reaches; the rest of them,
+    // and all without one, are plain copies.
+    auto small = [](const HostPiece &p) { return p.bytes > 0 && p.bytes < kDirect; };
+    auto room = [](size_t bytes) { return (bytes + 63) & ~(size_t)63; };
+    void *block = nullptr;
+    bool any = false;
+    for (int q = 0; q < count; q++) any |= small(pieces[q]);
+    if (any && take(slabs, kSlab, &block) != hipSuccess) block = nullptr;
+    char *const slab = static_cast<char *>(block);
     size_t at = 0;
     hipError_t e = hipSuccess;
     for (int q = 0; q < count && e == hipSuccess; q++) {
         const HostPiece &p = pieces[q];
-        if (p.bytes == 0 || (staged && p.bytes >= kDirect)) continue;
-        const bool ringed = staged && at + p.bytes <= kChunk * kSlots;
-        e = hipMemcpyAsync(ringed ? (void *)(ring + at) : p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s);
-        if (ringed) at += (p.bytes + 63) & ~(size_t)63;
+        if (!small(p)) continue;
+        const bool staged = slab && at + p.bytes <= kSlab;
+        e = hipMemcpyAsync(staged ? (void *)(slab + at) : p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s);
+        if (staged) at += room(p.bytes);
     }
-    hipError_t w = hipStreamSynchronize(s);
-    if (e != hipSuccess || w != hipSuccess) return e != hipSuccess ? e : w;
-    if (!staged) return hipSuccess;
+    const hipError_t w = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = w;
     at = 0;
-    for (int q = 0; q < count; q++) {
+    for (int q = 0; q < count && slab && e == hipSuccess; q++) {
         const HostPiece &p = pieces[q];
-        if (p.bytes == 0 || p.bytes >= kDirect || at + p.bytes > kChunk * kSlots) continue;
-        std::memcpy(p.dst, ring + at, p.bytes);
-        at += (p.bytes + 63) & ~(size_t)63;
+        if (!small(p) || at + p.bytes > kSlab) continue;
+        std::memcpy(p.dst, slab + at, p.bytes);
+        at += room(p.bytes);
     }
-    for (int q = 0; q < count && e == hipSuccess; q++)
-        if (pieces[q].bytes >= kDirect) e = large(pieces[q], s);
+    if (slab) give(slabs, kSlabs, slab);
+    for (int q = 0; q < count && e == hipSuccess; q++) {
+        const HostPiece &p = pieces[q];
+        if (p.bytes < kDirect) continue;
+        std::lock_guard<std::mutex> lk(m);
+        if (ready()) {
+            e = large(p, s);
+        } else {
+            e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s);
+            const hipError_t done = hipStreamSynchronize(s);
+            if (e == hipSuccess) e = done;
+        }
+    }
     return e;
 }
 

@@ -15,8 +15,10 @@ namespace flipmi {
 // chunks: the copy engine fills one chunk while host threads empty others.
 // (Straight into pageable memory the runtime reaches 10 to 17 GB/s here,
 // most of it spent faulting the caller's fresh pages in on one thread; the
-// engine alone moves 55 GB/s.)  One copy at a time; the ring is allocated
-// with the first copy that uses it.
+// engine alone moves 55 GB/s.)  Small results are staged in a slab of the
+// caller's own.  A caller waits for its stream holding nothing, and for the
+// ring only while another's data crosses.  Both are allocated with the first
+// copy that uses them.
 struct HostPiece {
     void *dst;
     const void *src;
@@ -37,19 +39,27 @@ public:
     hipError_t to_host(const HostPiece *pieces, int count, hipStream_t s);
     // Pinned host memory of kPage bytes, for one caller at a time.
     static constexpr size_t kPage = 4096;
-    hipError_t get_page(void **p);
-    void put_page(void *p);
+    hipError_t get_page(void **p) { return take(pages, kPage, p); }
+    void put_page(void *p) { give(pages, kPages, p); }
     void release();
 
 private:
     static constexpr size_t kChunk = (size_t)2 << 20;
     static constexpr int kSlots = 16;
+    // A stage call has ten results at most, each under the size that takes the
+    // ring when it is small: they all fit one slab.
+    static constexpr size_t kSlab = (size_t)5 << 19;
+    static constexpr size_t kSlabs = 8, kPages = 64;  // kept idle
     bool ready();
     hipError_t large(const HostPiece &p, hipStream_t s);
-    std::mutex m, page_m;
+    // A block of pinned memory from those kept in `idle`, or a new one.
+    hipError_t take(std::vector<void *> &idle, size_t bytes, void **p);
+    void give(std::vector<void *> &idle, size_t most, void *p);
+    std::mutex m;       // the ring
+    std::mutex idle_m;  // the lists below
     char *ring = nullptr;
     hipEvent_t filled[kSlots] = {};
-    std::vector<void *> pages;
+    std::vector<void *> slabs, pages;
 };
 
 // Device blocks kept between stage calls, at most kHeld bytes of them; the

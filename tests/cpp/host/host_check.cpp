@@ -1,10 +1,13 @@
 // Checks of the library's host side over a runtime without a device
 // (fake_hip.h), one per command-line name; see tests/test_host_side.py.
+#include <chrono>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <new>
+#include <thread>
 
 #include "../../../flipengine3d_amd/csrc/scene.h"
 #include "fake_hip.h"
@@ -249,6 +252,49 @@ static void give_back_without_host_memory() {
     rt().on_stream_wait = nullptr;
 }
 
+// While one context's kernels run, another's call begins and ends: the first
+// waits for its stream until the second call has returned.
+static void calls_do_not_wait_for_each_other() {
+    for (int na : {16, 64, 160})
+        for (int nb : {16, 64, 160}) {  // results under 256 KiB, over it, over 8 MiB
+            flipmi_ctx *a = nullptr, *b = nullptr;
+            CHECK_EQ(flipmi_ctx_create(0, &a), FLIPMI_OK);
+            CHECK_EQ(flipmi_ctx_create(0, &b), FLIPMI_OK);
+            std::mutex m;
+            std::condition_variable cv;
+            bool a_waits = false, b_done = false;
+            rt().on_stream_wait = [&](hipStream_t s) {
+                if (s != a->c.stream) return;
+                std::unique_lock<std::mutex> lk(m);
+                a_waits = true;
+                cv.notify_all();
+                CHECK(cv.wait_for(lk, std::chrono::seconds(20), [&] { return b_done; }));
+            };
+            auto call = [](flipmi_ctx *c, int n) {
+                std::vector<float> field((size_t)n * n * n);
+                std::vector<uint8_t> valid(field.size(), 0);
+                for (size_t q = 0; q < field.size(); q++) field[q] = (float)(q % 4099 + n);
+                CHECK_EQ(flipmi_extrapolate(c, n, n, n, field.data(), valid.data(), 1), FLIPMI_OK);
+                for (size_t q = 0; q < field.size(); q++) CHECK(field[q] == (float)(q % 4099 + n));
+            };
+            std::thread first([&] { call(a, na); });
+            {
+                std::unique_lock<std::mutex> lk(m);
+                CHECK(cv.wait_for(lk, std::chrono::seconds(20), [&] { return a_waits; }));
+            }
+            call(b, nb);
+            {
+                std::lock_guard<std::mutex> lk(m);
+                b_done = true;
+            }
+            cv.notify_all();
+            first.join();
+            rt().on_stream_wait = nullptr;
+            CHECK_EQ(flipmi_ctx_destroy(a), FLIPMI_OK);
+            CHECK_EQ(flipmi_ctx_destroy(b), FLIPMI_OK);
+        }
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
@@ -256,6 +302,7 @@ int main(int argc, char **argv) {
     else if (name == "pool_gives_way") pool_gives_way();
     else if (name == "no_pinned_memory") no_pinned_memory();
     else if (name == "give_back_without_host_memory") give_back_without_host_memory();
+    else if (name == "calls_do_not_wait_for_each_other") calls_do_not_wait_for_each_other();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

@@ -46,3 +46,7 @@ def test_results_come_without_pinned_memory(check):
 
 def test_a_buffer_is_given_back_without_host_memory(check):
     check("give_back_without_host_memory")
+
+
+def test_calls_of_two_contexts_do_not_wait_for_each_other(check):
+    check("calls_do_not_wait_for_each_other")
