@@ -743,6 +743,7 @@ void Scene::admit_pending() {
 // lives within a step), and cross in one piece.
 void Scene::read_particles(int64_t first, int64_t count, float *pos_xyz, float *vel_xyz) {
     if (count <= 0) return;
+    const DeviceScope on(ctx->device);  // the caller's thread may have another
     float *triples = reinterpret_cast<float *>(spos.p);
     const float zero[3] = {0.0f, 0.0f, 0.0f};
     for (int v = 0; v < 2; v++) {

@@ -66,6 +66,7 @@ hipError_t HostLink::take(std::vector<void *> &idle, size_t bytes, void **p) {
             return hipSuccess;
         }
     }
+    const DeviceScope on(device);
     const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
     if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
     return e;
@@ -86,6 +87,7 @@ void HostLink::give(std::vector<void *> &idle, size_t most, void *p) {
 }
 
 hipError_t HostLink::to_host(const HostPiece *pieces, int count, hipStream_t s) {
+    const DeviceScope on(device);
     // The small pieces go through a slab as far as it reaches; the rest of them,
     // and all without one, are plain copies.
     auto small = [](const HostPiece &p) { return p.bytes > 0 && p.bytes < kDirect; };
@@ -133,8 +135,6 @@ hipError_t HostLink::large(const HostPiece &piece, hipStream_t s) {
     void *const dst = piece.dst;
     const void *const src = piece.src;
     const size_t bytes = piece.bytes;
-    int device = 0;
-    (void)hipGetDevice(&device);
     const int n = (int)((bytes + kChunk - 1) / kChunk);
     std::atomic<int> queued{0}, failed{0};
     std::atomic<int> emptied[kSlots];  // the last chunk copied out of each slot
@@ -212,6 +212,7 @@ hipError_t HostLink::large(const HostPiece &piece, hipStream_t s) {
 
 hipError_t DevicePool::get(size_t bytes, void **p, size_t *size) {
     const size_t want = block_size(bytes);
+    const DeviceScope on(device);
     {
         std::lock_guard<std::mutex> lk(m);
         auto it = blocks.lower_bound(want);
@@ -296,7 +297,7 @@ std::shared_ptr<DeviceShared> DeviceShared::of(int device) {
     std::weak_ptr<DeviceShared> &held = all_shared()[device];
     std::shared_ptr<DeviceShared> p = held.lock();
     if (!p) {
-        p = std::make_shared<DeviceShared>();
+        p = std::make_shared<DeviceShared>(device);
         held = p;
     }
     return p;

@@ -11,6 +11,23 @@
 
 namespace flipmi {
 
+// Makes a device current while it is alive.
+class DeviceScope {
+public:
+    explicit DeviceScope(int device) {
+        changed = hipGetDevice(&was) == hipSuccess && was != device && hipSetDevice(device) == hipSuccess;
+    }
+    ~DeviceScope() {
+        if (changed) (void)hipSetDevice(was);
+    }
+    DeviceScope(const DeviceScope &) = delete;
+    DeviceScope &operator=(const DeviceScope &) = delete;
+
+private:
+    int was = 0;
+    bool changed = false;
+};
+
 // Copies device memory to pageable host memory through a ring of pinned
 // chunks: the copy engine fills one chunk while host threads empty others.
 // (Straight into pageable memory the runtime reaches 10 to 17 GB/s here,
@@ -18,7 +35,7 @@ namespace flipmi {
 // engine alone moves 55 GB/s.)  Small results are staged in a slab of the
 // caller's own.  A caller waits for its stream holding nothing, and for the
 // ring only while another's data crosses.  Both are allocated with the first
-// copy that uses them.
+// copy that uses them.  The caller's current device may be another.
 struct HostPiece {
     void *dst;
     const void *src;
@@ -26,7 +43,7 @@ struct HostPiece {
 };
 class HostLink {
 public:
-    HostLink() {}
+    explicit HostLink(int on) : device(on) {}
     HostLink(const HostLink &) = delete;
     HostLink &operator=(const HostLink &) = delete;
     ~HostLink() { release(); }
@@ -50,6 +67,7 @@ private:
     // ring when it is small: they all fit one slab.
     static constexpr size_t kSlab = (size_t)5 << 19;
     static constexpr size_t kSlabs = 8, kPages = 64;  // kept idle
+    const int device;
     bool ready();
     hipError_t large(const HostPiece &p, hipStream_t s);
     // A block of pinned memory from those kept in `idle`, or a new one.
@@ -67,7 +85,7 @@ private:
 // here or in device_alloc.  Safe from several threads.
 class DevicePool {
 public:
-    DevicePool() {}
+    explicit DevicePool(int on) : device(on) {}
     DevicePool(const DevicePool &) = delete;
     DevicePool &operator=(const DevicePool &) = delete;
     ~DevicePool() { release(); }
@@ -77,6 +95,7 @@ public:
 
 private:
     static constexpr size_t kHeld = (size_t)1 << 30;
+    const int device;
     std::mutex m;
     std::multimap<size_t, void *> blocks;
     size_t held = 0;
@@ -115,6 +134,7 @@ private:
 
 // Held by every context of a device, freed with the last of them.
 struct DeviceShared {
+    explicit DeviceShared(int device) : link(device), pool(device) {}
     HostLink link;
     DevicePool pool;
     static std::shared_ptr<DeviceShared> of(int device);

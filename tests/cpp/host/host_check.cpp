@@ -182,7 +182,7 @@ static void pool_gives_way() {
     }
     CHECK_EQ(rt().in_use, 0);
     // Inside one: a buffer given back makes room for a larger one.
-    DevicePool pool;
+    DevicePool pool(0);
     rt().limit = 100 << 20;
     {
         hipStream_t s = nullptr;
@@ -223,7 +223,7 @@ static void no_pinned_memory() {
         CHECK_EQ(hipGetLastError(), hipSuccess);
     }
     void *page = nullptr;
-    HostLink link;
+    HostLink link(0);
     CHECK_EQ(link.get_page(&page), hipErrorOutOfMemory);
     CHECK_EQ(hipGetLastError(), hipSuccess);
     rt().pinned_fails = false;
@@ -233,7 +233,7 @@ static void no_pinned_memory() {
 // A buffer is given back without host memory to note it in: no exception leaves
 // its destructor, and the device gets it.
 static void give_back_without_host_memory() {
-    DevicePool pool;
+    DevicePool pool(0);
     hipStream_t s = nullptr;
     CHECK(hipStreamCreateWithFlags(&s, 0) == hipSuccess);
     bool waited = false;
@@ -295,6 +295,52 @@ static void calls_do_not_wait_for_each_other() {
         }
 }
 
+// Results are read from a thread whose current device is another, and nothing of
+// that device gets among the context's memory.
+static void another_device_is_current() {
+    flipmi_ctx *ctx = nullptr;
+    CHECK_EQ(flipmi_ctx_create(1, &ctx), FLIPMI_OK);
+    flipmi_scene_desc d;
+    flipmi_scene_desc_default(&d);
+    d.isize = 24; d.jsize = d.ksize = 16;
+    d.dx = 1.0 / 16;
+    flipmi_scene *scene = nullptr;
+    CHECK_EQ(flipmi_scene_create(ctx, &d, &scene), FLIPMI_OK);
+    std::vector<float> pos(3 * 400000, 0.5f), vel(pos.size(), 0.0f), u((size_t)25 * 16 * 16);
+    CHECK_EQ(flipmi_scene_load_particles(scene, pos.data(), vel.data(), (int64_t)pos.size() / 3), FLIPMI_OK);
+    CHECK_EQ(flipmi_scene_initialize(scene), FLIPMI_OK);
+    CHECK(hipSetDevice(0) == hipSuccess);
+    const auto current = [] {
+        int dev = -1;
+        (void)hipGetDevice(&dev);
+        return dev;
+    };
+    CHECK_EQ(flipmi_scene_get_particles(scene, pos.data(), vel.data()), FLIPMI_OK);
+    CHECK_EQ(flipmi_scene_get_particles_range(scene, 3, 17, pos.data(), nullptr), FLIPMI_OK);
+    CHECK_EQ(flipmi_scene_get_grid(scene, FLIPMI_GRID_U, u.data()), FLIPMI_OK);
+    int64_t nv = 0, nt = 0;
+    CHECK_EQ(flipmi_scene_get_isomesh(scene, &nv, &nt, nullptr, nullptr), FLIPMI_OK);
+    CHECK_EQ(current(), 0);
+    // The pool's blocks are the context's device's, whatever the call came to.
+    const int n = 32;
+    std::vector<float> field((size_t)n * n * n, 0.0f);
+    std::vector<uint8_t> valid(field.size(), 0);
+    (void)flipmi_extrapolate(ctx, n, n, n, field.data(), valid.data(), 1);
+    {
+        std::shared_ptr<DeviceShared> shared = DeviceShared::of(1);
+        void *p = nullptr;
+        size_t size = 0;
+        for (size_t bytes : {sizeof(float) * field.size(), valid.size(), (size_t)1000}) {
+            CHECK_EQ(shared->pool.get(bytes, &p, &size), hipSuccess);
+            CHECK_EQ(fake::device_of(p), 1);
+            shared->pool.put(p, size);
+        }
+    }
+    CHECK_EQ(current(), 0);
+    CHECK_EQ(flipmi_scene_destroy(scene), FLIPMI_OK);
+    CHECK_EQ(flipmi_ctx_destroy(ctx), FLIPMI_OK);
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
@@ -303,6 +349,7 @@ int main(int argc, char **argv) {
     else if (name == "no_pinned_memory") no_pinned_memory();
     else if (name == "give_back_without_host_memory") give_back_without_host_memory();
     else if (name == "calls_do_not_wait_for_each_other") calls_do_not_wait_for_each_other();
+    else if (name == "another_device_is_current") another_device_is_current();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

@@ -50,3 +50,7 @@ def test_a_buffer_is_given_back_without_host_memory(check):
 
 def test_calls_of_two_contexts_do_not_wait_for_each_other(check):
     check("calls_do_not_wait_for_each_other")
+
+
+def test_results_are_read_while_another_device_is_current(check):
+    check("another_device_is_current")
