@@ -724,7 +724,10 @@ int flipmi_pressure_solve(flipmi_ctx *ctx, const flipmi_pressure_args *a, flipmi
             // The pressure of a pocket that borders no air is fixed up to a
             // constant only, which follows from the preconditioner.  Callers
             // of this entry point see the pressures, so such a system keeps
-            // MIC(0) (a scene uses their differences alone).
+            // MIC(0).  (In a scene any constant does that is not much larger
+            // than the pressures, which are rounded to float before their
+            // differences are taken; multigrid's leaves a pocket's mean within
+            // a few hundredths of their range.)
             if (pocket) multigrid = false;
         }
         PressureStore ps;

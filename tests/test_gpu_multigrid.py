@@ -165,3 +165,68 @@ def test_graph_batches_match_kernel_launches(gpu):
         assert st[0].pcg_iterations == st[1].pcg_iterations and st[0].pressure_ok == st[1].pressure_ok == 1
         for x, y in zip(sims[0].particles(), sims[1].particles()):
             assert bits_equal(x, y)
+
+
+def _closed_region(liquid, weights, start):
+    """Cells of the liquid region of `start` over open faces, and whether one of those faces leads to air."""
+    wu, wv, ww = weights
+    cells, todo, air = {start}, [start], False
+    while todo:
+        k, j, i = todo.pop()
+        for w, n in ((wu[k, j, i + 1], (k, j, i + 1)), (wu[k, j, i], (k, j, i - 1)), (wv[k, j + 1, i], (k, j + 1, i)),
+                     (wv[k, j, i], (k, j - 1, i)), (ww[k + 1, j, i], (k + 1, j, i)), (ww[k, j, i], (k - 1, j, i))):
+            if w <= 0:
+                continue
+            if liquid[n] >= 0:
+                air = True
+            elif n not in cells:
+                cells.add(n)
+                todo.append(n)
+    return cells, air
+
+
+def test_closed_cavity_in_a_scene(gpu):
+    # A cavity full of liquid between six slabs borders no air: multigrid solves
+    # it with the rest, and the velocities follow the FP64 path's.
+    import flipengine3d_amd as fa
+    from flipengine3d_amd import scenes
+    I, J, K, dx = 1024, 32, 32, 1 / 32
+    lo, hi = np.array([600.4, 8.4, 9.4]), np.array([608.7, 16.7, 17.7])  # cavity, in cells
+    rng = np.random.default_rng(5)
+    cells = np.stack(np.meshgrid(np.arange(2, 120), np.arange(2, 16), np.arange(2, 30), indexing="ij"), -1).reshape(-1, 3)
+    inner = np.stack(np.meshgrid(*[np.arange(int(a), int(b) + 1) for a, b in zip(lo, hi)], indexing="ij"), -1)
+    cells = np.concatenate([cells, inner.reshape(-1, 3)])
+    off = np.array([[a, b, c] for a in (0.25, 0.75) for b in (0.25, 0.75) for c in (0.25, 0.75)])
+    p = (cells[:, None] + off[None]).reshape(-1, 3)
+    p += (rng.random(p.shape) - 0.5) * 0.2
+    in_cavity = ((p > lo + 0.05) & (p < hi - 0.05)).all(1)
+    p = p[(p[:, 0] < 200) | in_cavity]
+    pos = (p * dx).astype(np.float32)
+    vel = (0.3 * rng.standard_normal(pos.shape)).astype(np.float32)
+    sims = []
+    for prec in (fa.PCG_FP64, fa.PCG_MIXED):
+        sim = fa.FluidSimulation(I, J, K, dx, ctx=gpu, precision=prec)
+        sim.addBodyForce(0.0, -9.81, 0.0)
+        sim.setMinTimeStepsPerFrame(1)
+        sim.setMaxTimeStepsPerFrame(1)
+        for a in range(3):
+            for side in (0, 1):
+                b0, b1 = lo - 3, hi + 3
+                if side:
+                    b0[a] = hi[a]
+                else:
+                    b1[a] = lo[a]
+                sim.addMeshObstacle(*scenes.box_mesh(b0 * dx, b1 * dx))
+        sim.loadMarkerParticleData(pos, vel)
+        sim.initialize()
+        sims.append(sim)
+    for step in range(2):
+        st = [sim.update(1 / 480) for sim in sims]
+        if step == 0:
+            region, air = _closed_region(sims[1].grid(0), [sims[1].grid(w) for w in (5, 6, 7)], (13, 12, 604))
+            assert len(region) >= 7 ** 3 and not air
+        assert st[0].pressure_ok == st[1].pressure_ok == 1
+        assert st[1].pcg_refinements == 1 and st[1].pcg_iterations <= 40  # multigrid's
+        (p0, v0), (p1, v1) = sims[0].particles(), sims[1].particles()
+        assert p0.shape == p1.shape
+        assert np.abs(p0 - p1).max() <= 1e-3 * dx and np.abs(v0 - v1).max() <= 1e-3
