@@ -351,6 +351,15 @@ static int next_batch(int need) {
     return size;
 }
 
+// The multigrid batch of at least n iterations (n <= 16) that is captured:
+// few sizes here too, in up to four states each.
+static int graph_batch(int n) {
+    static const int kSizes[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    for (int c : kSizes)
+        if (c >= n) return c;
+    return 16;
+}
+
 // Events for the selected kernels of an iteration at profiling level 2.
 static bool take_kernel_timings(Scene *prof, KernelTiming (&kt)[kPcgPieces], bool (*used)(int piece)) {
     if (!prof || prof->profiling < 2 || prof->kernel_mask == 0 ||
@@ -404,8 +413,8 @@ static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *h
     // first batch stops short of that and the rate gives the rest.
     int batch = 8, launched = 0, prev_iters = 0;
     double prev_resid = 0.0;
+    const bool use_graph = w.graphs && !(prof && prof->profiling >= 2);
     for (;;) {
-        const bool use_graph = w.graphs && !(prof && prof->profiling >= 2);
         const int state = mg.turn + 2 * (mg.first ? 1 : 0);
         auto all = [&]() -> hipError_t {
             hipError_t e = hipSuccess;
@@ -436,6 +445,7 @@ static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *h
         prev_iters = hs->iters;
         prev_resid = hs->resid;
         batch = std::max(1, std::min(need > 0 ? need : 8, 16));
+        if (use_graph) batch = graph_batch(batch);
     }
     if (prof) prof->end_stage(FLIPMI_STAGE_PCG, ev);
     out.rows = hs->rows;

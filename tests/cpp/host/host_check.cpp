@@ -1,6 +1,7 @@
 // Checks of the library's host side over a runtime without a device
 // (fake_hip.h), one per command-line name; see tests/test_host_side.py.
 #include <chrono>
+#include <cmath>
 #include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
@@ -341,6 +342,32 @@ static void another_device_is_current() {
     CHECK_EQ(flipmi_ctx_destroy(ctx), FLIPMI_OK);
 }
 
+// However many iterations the rate asks for, few batch sizes are captured.
+static void few_graphs() {
+    Projection p;
+    p.w.graphs = &p.ps.graphs;
+    p.ps.alloc(p.w.g, p.stream, true, true);
+    int need = 0, looks = 0;
+    rt().on_download = [&](void *dst, size_t bytes) {
+        if (bytes != sizeof(MgScalars)) return;
+        MgScalars *sc = static_cast<MgScalars *>(dst);
+        sc->bnorm = 1.0;
+        sc->tol = 1e-9;
+        sc->iters = 8;
+        // At the observed rate, `need` iterations more reach the tolerance.
+        sc->resid = std::exp(std::log(1e-9) / (1.0 + (need - 0.5) / 8));
+        sc->done = sc->converged = ++looks > 1;
+    };
+    for (int round = 0; round < 2; round++)
+        for (need = 1; need <= 16; need++) {
+            looks = 0;
+            CHECK_EQ(p.solve(), FLIPMI_OK);
+        }
+    std::map<int, int> sizes;
+    for (auto &g : p.ps.graphs.exec) sizes[g.first.first]++;
+    CHECK(sizes.size() <= 8 && sizes.count(8) && sizes.count(16));
+}
+
 int main(int argc, char **argv) {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "no_room_to_fall_back") no_room_to_fall_back();
@@ -350,6 +377,7 @@ int main(int argc, char **argv) {
     else if (name == "give_back_without_host_memory") give_back_without_host_memory();
     else if (name == "calls_do_not_wait_for_each_other") calls_do_not_wait_for_each_other();
     else if (name == "another_device_is_current") another_device_is_current();
+    else if (name == "few_graphs") few_graphs();
     else return 2;
     std::printf("ok\n");
     std::fflush(stdout);

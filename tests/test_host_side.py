@@ -54,3 +54,7 @@ def test_calls_of_two_contexts_do_not_wait_for_each_other(check):
 
 def test_results_are_read_while_another_device_is_current(check):
     check("another_device_is_current")
+
+
+def test_few_batch_sizes_are_captured(check):
+    check("few_graphs")
