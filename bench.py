@@ -41,53 +41,42 @@ KERNEL_SAMPLE = 8
 # array the kernel must read or write, once.  The matrix is the FP64 diagonal
 # and the three upper couplings (the lower three are the neighbours' upper
 # ones), stored as the FP32 face weights the FP64 entries are rebuilt from
-# exactly: 8 + 3 x 4 = 20 bytes on both paths.  FP64 path, 8-byte vectors:
-#   spmv_dot:   s, matrix, z (= A s)                       -> 8 + 20 + 8
-#   axpy_norm:  x r/w, s, r r/w, z                          -> 6 x 8
-#   forward:    r, invdiag, 3 lower factor entries, z       -> 6 x 8
+# exactly: 8 + 3 x 4 = 20 bytes on every path.
+# "fp64": 8-byte vectors, the direction update and x += alpha s in the SpMV,
+# the rest of the axpy in the forward sweep:
+#   spmv_dot:   z, old s, matrix, new s, q, x r/w           -> 8 + 8 + 20 + 8 + 8 + 16
+#   forward:    r r/w, q, invdiag, 3 lower factor entries, z -> 16 + 8 + 8 + 24 + 8
 #   backward:   z r/w, invdiag, 3 upper factor entries, and
-#               r for the fused z.r                         -> 7 x 8
-#   update_s:   z, s r/w                                    -> 3 x 8
-# A mixed MIC(0) iteration, FP32 vectors and factor, FP64 x and matrix entries
-# (scenes under 2^20 cells):
+#               r for the fused z.r                         -> 16 + 8 + 24 + 8
+# "mixed_mic0" (mixed scenes under 2^20 cells): FP32 vectors and factor, FP64
+# x and matrix entries:
 #   spmv_dot:   z, old s, matrix, new s, q (= A s)          -> 4 + 4 + 20 + 4 + 4
-#   forward with the axpy folded in: r r/w, q, invdiag, 3 lower factor
-#               entries, z, and x r/w (FP64), s             -> 8 + 4 + 4 + 12 + 4 + 16 + 4
+#   forward:    with the axpy: r r/w, q, invdiag, 3 lower
+#               factor entries, z, x r/w (FP64), s          -> 8 + 4 + 4 + 12 + 4 + 16 + 4
 #   backward:   7 x 4
-#   the direction update is folded into spmv_dot.
-# A true residual in that iteration reads x and b (FP64) and the matrix and
-# writes r (FP32): 8 + 8 + 20 + 4 = 40 bytes; the forward sweep over it
-# adds r, invdiag, 3 lower factor entries, z: 6 x 4.
-PCG_BYTES = {
-    "fp64": {"k_spmv_dot": 36, "k_axpy_norm": 48, "k_forward": 48, "k_backward": 56, "k_update_s": 24},
-    "mixed": {"k_spmv_dot": 36, "k_axpy_norm": 0, "k_forward": 52, "k_backward": 28, "k_update_s": 0},
-}
-TRUE_RESIDUAL_BYTES = 40 + 24
-
-# The same for a mixed iteration with the multigrid V-cycle (larger scenes): FP64 x, r, q and diagonal,
-# FP32 couplings (12), inverse diagonal and cycle vectors:
-#   spmv_dot:   z, old s, matrix, new s, q                   -> 4 + 4 + 20 + 4 + 8
+# "mixed" (larger scenes): the multigrid V-cycle, FP64 x, r, q and diagonal,
+# FP32 couplings (12), inverse diagonal and cycle vectors; on the finest level
+#   spmv_dot:   z, old s, matrix, new s, q                  -> 4 + 4 + 20 + 4 + 8
 #   axpy_norm:  r, q, x r/w, s, r', inverse diagonal,
-#               couplings, FP32 r, z (first smoothing)       -> 8 + 8 + 16 + 4 + 8 + 4 + 12 + 4 + 4
+#               couplings, FP32 r, z (first smoothing)      -> 8 + 8 + 16 + 4 + 8 + 4 + 12 + 4 + 4
 #   forward:    restriction: r, z, inverse diagonal,
-#               couplings, an eighth of a coarse r           -> 4 + 4 + 4 + 12 + 0.5
+#               couplings, an eighth of a coarse r          -> 4 + 4 + 4 + 12 + 0.5
 #   update_s:   correction: r, z, coarse z, inverse
-#               diagonal, couplings, y                       -> 4 + 4 + 0.5 + 4 + 12 + 4
+#               diagonal, couplings, y                      -> 4 + 4 + 0.5 + 4 + 12 + 4
 #   backward:   last smoothing: r, y, inverse diagonal,
-#               couplings, z, FP64 r for z.r                 -> 4 + 4 + 4 + 12 + 4 + 8
-# The coarser levels repeat restriction, correction and the smoothings (24
-# before, 28 after) on an eighth of the rows each time.  The true residual
-# reads x, b and the matrix and writes r: 8 + 8 + 20 + 8.
-# The FP64 iteration forms the direction in the SpMV, which also brings x up to
-# date (z, old s, new s, q, matrix, x r/w), and does the rest of the axpy in the
-# forward sweep (r r/w, q, factor, z).
+#               couplings, z, FP64 r for z.r                -> 4 + 4 + 4 + 12 + 4 + 8
 KERNEL_BYTES = {
     "fp64": {"k_spmv_dot": 68, "k_axpy_norm": 0, "k_forward": 64, "k_backward": 56, "k_update_s": 0},
-    "mixed_mic0": PCG_BYTES["mixed"],
+    "mixed_mic0": {"k_spmv_dot": 36, "k_axpy_norm": 0, "k_forward": 52, "k_backward": 28, "k_update_s": 0},
     "mixed": {"k_spmv_dot": 40, "k_axpy_norm": 68, "k_forward": 24.5, "k_backward": 36, "k_update_s": 28.5},
 }
+# The coarser multigrid levels repeat restriction, correction and the
+# smoothings (24 before, 28 after) on an eighth of the rows each time.
 COARSE_LEVEL_BYTES = {"fp64": 0.0, "mixed_mic0": 0.0, "mixed": (24 + 24.5 + 28.5 + 28) / 7}
-RESIDUAL_BYTES = {"fp64": 0, "mixed_mic0": TRUE_RESIDUAL_BYTES, "mixed": 44}
+# A true residual reads x, b and the matrix and writes r: FP32 with MIC(0),
+# where a forward sweep over it follows (r, invdiag, 3 lower factor entries, z);
+# FP64 with multigrid.
+RESIDUAL_BYTES = {"fp64": 0, "mixed_mic0": 8 + 8 + 20 + 4 + 6 * 4, "mixed": 8 + 8 + 20 + 8}
 MULTIGRID_CELLS = 1 << 20  # mixed scenes below this keep MIC(0)
 KERNEL_NAMES = {
     "fp64": {"k_forward": "k_sweep<forward>", "k_backward": "k_sweep<backward>"},
