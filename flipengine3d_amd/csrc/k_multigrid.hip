@@ -21,7 +21,8 @@
 // Why not the reference's MIC(0) here: its triangular solves are a chain of
 // I + J + K dependent steps (about 75 us each way on a 256x128x128 grid, 30
 // tile hand-offs deep), and it takes about 115 iterations to 1e-9 there; the
-// V-cycle has no such chain and takes 13 to 16 iterations at every size.
+// V-cycle has no such chain and takes 10 to 22 iterations to 1e-9 at
+// 16^3 to 320x160x160 (20 there).
 // 256x128x128 double dam break, 1.23 M rows: 21.8 -> 3.2 ms per solve (factor
 // included).
 // The FP64 path keeps MIC(0), bit for bit, and so do mixed scenes of request
@@ -54,7 +55,7 @@ constexpr int kBrickX = 64, kBrickY = 2, kBrickZ = 2;
 // the order of the dot products' partial sums does not depend on anything
 // but the system.
 constexpr int kMgBlocks = 1024;
-static_assert(5 * kMgBlocks <= (int)kMgPartials, "five partial arrays");
+static_assert(4 * kMgBlocks <= (int)kMgPartials, "z.r, s.q, the recursive norm and the true one");
 constexpr float kDampA = 1.5f, kDampB = 0.6f;
 // Least excess of a row's diagonal over its couplings, relative to their sum,
 // that is more than rounding (six products and sums in FP64, under 1e-14).  A

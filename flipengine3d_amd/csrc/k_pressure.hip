@@ -1721,7 +1721,7 @@ __global__ __launch_bounds__(kRedThreads) void k_spmv_dot(GridGeom g, PressureBu
                             : spmv_dot_body(g, pb, NextDirection<double>{pb.z, pb.s, pb.sc->beta_f}, true);
     double bs = block_reduce<0>(acc, sh);
     if (threadIdx.x == 0) st_dev(&pb.partials[blockIdx.x], bs);
-    if (!last_block(&pb.sc->counter[1], pb.sc->group_counter[0])) return;
+    if (!last_block(&pb.sc->counter[1], pb.sc->group_counter)) return;
     double tot = 0.0;
     for (int q = threadIdx.x; q < (int)gridDim.x; q += kRedThreads) tot += ld_dev(&pb.partials[q]);
     tot = block_reduce<0>(tot, sh);
@@ -2022,7 +2022,7 @@ __global__ __launch_bounds__(kRedThreads) void k_spmv_dot32(GridGeom g, Pressure
                             : spmv_dot32_body(g, pb, NextDirection<float>{pb.z32, pb.s32, pb.sc->beta_f});
     double bs = block_reduce<0>(acc, sh);
     if (threadIdx.x == 0) st_dev(&pb.partials[blockIdx.x], bs);
-    if (!last_block(&pb.sc->counter[1], pb.sc->group_counter[0])) return;
+    if (!last_block(&pb.sc->counter[1], pb.sc->group_counter)) return;
     double tot = 0.0;
     for (int q = threadIdx.x; q < (int)gridDim.x; q += kRedThreads) tot += ld_dev(&pb.partials[q]);
     tot = block_reduce<0>(tot, sh);

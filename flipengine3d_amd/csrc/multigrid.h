@@ -104,7 +104,7 @@ private:
     double *r_next() const { return turn ? ra : rb; }
     hipError_t cycle(bool count, hipStream_t s, const KernelTiming *kt);
 };
-constexpr size_t kMgPartials = 5 * 1024;  // doubles
+constexpr size_t kMgPartials = 4 * 1024;  // doubles
 // Lets the multigrid kernel use its LDS on `device` (current), once.
 hipError_t mg_allow_lds(int device);
 

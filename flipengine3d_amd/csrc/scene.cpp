@@ -408,8 +408,8 @@ static bool run_multigrid(const PressureWork &w, PressureStore &ps, MgScalars *h
     if (prof) prof->begin_stage(FLIPMI_STAGE_PCG, &ev);
     hip_check(mg.start(false, s), "pcg start");
     // Iterations are enqueued in batches between host checks of the device
-    // scalars; kernels past convergence return at once.  The count hardly
-    // depends on the system (13 to 16 for 1e-9, 8 to 10 for 1e-6), so the
+    // scalars; kernels past convergence return at once.  The count
+    // depends little on the system (10 to 22 for 1e-9, 7 to 16 for 1e-6), so the
     // first batch stops short of that and the rate gives the rest.
     int batch = 8, launched = 0, prev_iters = 0;
     double prev_resid = 0.0;
@@ -653,14 +653,14 @@ static size_t scan_elems(const GridGeom &g, size_t particles) {
     return std::max(scan_scratch_elems((int)subcell_bins(g)), scan_scratch_elems((int)particles));
 }
 
-// Mixed scenes of this many cells and more solve with multigrid.  It is the
-// faster solver at every size (97x75x83: 1.4 ms a solve against 8.2; 256x128x128:
-// 3.2 against 21.8), so the line is not drawn by speed: scenes of request size
-// run for tens of steps and their results are compared with earlier ones to
-// 1e-6, and two solvers that both converge to 1e-9 do not agree that well there
-// (a last bit in a particle moves some cell's phi across zero, and the runs
-// part: up to 7e-5 after ten steps at 32^3 to 96^3).  Below the line a scene
-// keeps the MIC(0) iteration, bit for bit, served or not.
+// Mixed scenes of this many cells and more solve with multigrid.  The line is
+// not drawn by speed: multigrid is the faster solver on either side (97x75x83:
+// 1.4 ms a solve against 8.2; 256x128x128: 3.2 against 21.8), and a projection
+// call takes it at every size.  Below the line, where the served requests'
+// grids lie, a scene keeps the MIC(0) iteration so that a run of many steps
+// gives the results it gave before there was another solver.  Two solvers that
+// both converge to 1e-9 do not: a last bit in a particle moves some cell's phi
+// across zero, and the runs part (up to 7e-5 after ten steps at 32^3 to 96^3).
 constexpr size_t kMultigridCells = (size_t)1 << 20;
 
 void Scene::alloc_all() {

@@ -109,7 +109,7 @@ enum {
     FLIPMI_STAGE_K_FORWARD = 14,
     FLIPMI_STAGE_K_BACKWARD = 15,
     FLIPMI_STAGE_K_UPDATE = 16,
-    FLIPMI_STAGE_K_RESIDUAL = 17,   /* MIC(0) in FP32: FP64 true residual + forward sweep over it */
+    FLIPMI_STAGE_K_RESIDUAL = 17,   /* mixed MIC(0): FP64 true residual + forward sweep over it */
     FLIPMI_STAGE_INFLOW = 18,       /* mesh inflow: particle mask and emission */
     FLIPMI_STAGE_SURFACE = 19       /* surface reconstruction (sort, field, marching cubes, smoothing) */
 };
@@ -302,10 +302,13 @@ int flipmi_scene_stage_times(flipmi_scene *scene, flipmi_stage_times *out, int r
  * stage, 2 additionally one pair around every PCG kernel launch. */
 int flipmi_scene_set_profiling(flipmi_scene *scene, int level);
 /* PCG kernels timed at profiling level 2, one bit per FLIPMI_STAGE_K_*
- * stage minus FLIPMI_STAGE_K_SPMV; default all.  On the mixed path AXPY is
- * the axpy with the first smoothing, FORWARD the restriction, UPDATE the
- * coarse correction and BACKWARD the last smoothing, each on the finest
- * level, and FLIPMI_STAGE_K_RESIDUAL (bit 5) stays empty.
+ * stage minus FLIPMI_STAGE_K_SPMV; default all.  With MIC(0) (FP64, mixed
+ * scenes under 2^20 cells, and larger ones while it has taken over) SPMV
+ * includes the direction update and FORWARD the axpy, so AXPY and UPDATE stay
+ * empty, as does RESIDUAL in FP64.  With multigrid SPMV includes the direction
+ * update, AXPY is the axpy with the first smoothing, FORWARD the restriction,
+ * UPDATE the coarse correction and BACKWARD the last smoothing, each on the
+ * finest level, and RESIDUAL stays empty.
  * Each timed launch adds an event pair, which delays the launches around it. */
 int flipmi_scene_set_kernel_timing(flipmi_scene *scene, unsigned mask);
 /* Times the selected kernels on every `every`-th PCG iteration only (default
