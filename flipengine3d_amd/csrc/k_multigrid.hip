@@ -545,8 +545,10 @@ __global__ __launch_bounds__(kMgThreads) void k_mg_smooth_up(MgLevel L, MgLists 
 // one workgroup.  Everything it needs is brought to LDS at once: couplings,
 // inverse diagonals and, per cell, where its aggregate lies, so that each of
 // the forty or so dependent passes is a few LDS reads and a barrier.  Bound by
-// that chain: 1024 cells of a 256x128x128 grid 16 us.  (8192 cells with the couplings read from
-// the L2 in every pass took 62 us, more than four launches per level cost.)
+// that chain: 1024 cells of a 256x128x128 grid 19.5 us, 16 on the mean over all
+// launches with those past convergence.  (8192 cells with the couplings read
+// from the L2 in every pass took 62 us on that mean, more than four launches per
+// level cost.)
 // Cells lie unpadded: a neighbour beyond the grid is some other cell, and its
 // coupling is zero (zero guards stand before and after the arrays).
 constexpr int kCoarseThreads = 512;
